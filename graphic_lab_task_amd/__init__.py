@@ -128,7 +128,7 @@ ARRAY_DTYPES = {
     "frame_tex_nodes": FRAME_TEX_NODE_DTYPE, "frame_tex_roots": np.uint32,
     "sbs_nodes": SBS_NODE_DTYPE, "sbs_data": np.uint32, "sbs_data_f": np.float32, "sbs_roots": np.uint32,
     "sbs_headers": SBS_HEADER_DTYPE, "multi_nodes": MULTI_NODE_DTYPE, "multi_values": np.float32,
-    "preset": PRESET_DTYPE, "sbs_mask": np.uint32, "orig_indices": np.uint32, "svs_nodes": SVS_NODE_DTYPE,
+    "preset": PRESET_DTYPE, "sbs_mask": np.uint32, "wide_blocks": np.uint32, "wide_root": np.uint32, "orig_indices": np.uint32, "svs_nodes": SVS_NODE_DTYPE,
     "svs_roots": np.uint32, "tlas_parent": np.uint32, "grid_data": np.float32, "grid_offsets": np.uint32,
     "grid_sizes": np.uint32, "gprim_headers": GPRIM_HEADER_DTYPE, "gprim_points": np.float32,
     "coct_data": np.uint32, "coct_geoms": COCT_GEOM_DTYPE, "coct_mods": np.int32,

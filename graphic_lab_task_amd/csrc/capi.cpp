@@ -90,6 +90,8 @@ lrt::TraceArgs trace_args(lrt_scene* s, const float* pos, const float* dir, lrt_
   // extra leaf visits would change the counts of that mode too
   a.postpone_tri = s->s.preset.render_mode != lrt::MULTI_RENDER_MODE_INTERSECTION_COUNT && s->s.postpone_triangles();
   a.persistent = s->s.persistent ? 1u : 0u;
+  // (the wide walk visits other leaves, too)
+  a.wide = s->s.wide && s->s.preset.render_mode != lrt::MULTI_RENDER_MODE_INTERSECTION_COUNT;
   return a;
 }
 
@@ -116,7 +118,7 @@ lrt_status trace_common(lrt_scene* s, const float* pos, const float* dir, lrt_hi
   // between ours (they share the stream's tail queue) or grow the buffer under us
   lrt::Scene::StreamWork& w = s->s.stream_work(stream);
   std::lock_guard<std::mutex> lock(w.mu);
-  hipError_t e = s->s.work_for(w, stream, size_t(n), &a.spill, &a.queue, &a.pcount);
+  hipError_t e = s->s.work_for(w, stream, size_t(n), &a.spill, &a.queue, &a.pcount, &a.spill_words);
   if (e != hipSuccess) return hip_fail(e, "work buffer");
   e = lrt::launch_trace(s->s.make_view(), a, reinterpret_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "trace launch");
@@ -653,6 +655,7 @@ lrt_status lrt_set_launch_config(lrt_scene* s, int block, int lds_stack, int xcd
     if (block != 64 && block != 128 && block != 256) return fail(LRT_ERR_INVALID_ARG, "block must be 64, 128 or 256");
     if (lds_stack != 8 && lds_stack != 16 && lds_stack != 32)
       return fail(LRT_ERR_INVALID_ARG, "lds_stack must be 8, 16 or 32");
+    s->s.wide = false;   // a launch shape of the binary walk was asked for
     s->s.block = block;
     s->s.lds_stack = lds_stack;
     s->s.xcd_remap = xcd_remap ? 1 : 0;
@@ -664,6 +667,7 @@ lrt_status lrt_set_tail_config(lrt_scene* s, uint32_t budget, uint32_t tail_wave
   return guarded([&]() -> lrt_status {
     if (!s) return fail(LRT_ERR_INVALID_ARG, "null scene");
     if (tail_waves > 65536) return fail(LRT_ERR_INVALID_ARG, "tail_waves must be <= 65536");
+    s->s.wide = false;   // a launch shape of the binary walk was asked for
     s->s.budget = budget;
     s->s.tail_waves = tail_waves ? tail_waves : 1024u;
     return LRT_OK;
@@ -675,6 +679,7 @@ lrt_status lrt_set_ray_interleave(lrt_scene* s, uint32_t lanes_per_group) {
     if (!s) return fail(LRT_ERR_INVALID_ARG, "null scene");
     if (lanes_per_group > 64 || (lanes_per_group & (lanes_per_group - 1)) != 0)
       return fail(LRT_ERR_INVALID_ARG, "lanes_per_group must be 0 or a power of two up to 64");
+    s->s.wide = false;   // a launch shape of the binary walk was asked for
     s->s.ray_groups = lanes_per_group;
     return LRT_OK;
   });
@@ -684,6 +689,7 @@ lrt_status lrt_set_persistent(lrt_scene* s, int on) {
   return guarded([&]() -> lrt_status {
     if (!s) return fail(LRT_ERR_INVALID_ARG, "null scene");
     if (on != 0 && on != 1) return fail(LRT_ERR_INVALID_ARG, "on must be 0 or 1");
+    s->s.wide = false;   // a launch shape of the binary walk was asked for
     s->s.persistent = on;
     return LRT_OK;
   });
@@ -693,6 +699,7 @@ lrt_status lrt_set_leaf_postponement(lrt_scene* s, int mode) {
   return guarded([&]() -> lrt_status {
     if (!s) return fail(LRT_ERR_INVALID_ARG, "null scene");
     if (mode < -1 || mode > 1) return fail(LRT_ERR_INVALID_ARG, "mode must be -1, 0 or 1");
+    if (mode >= 0) s->s.wide = false;
     s->s.leaf_postpone = mode;
     return LRT_OK;
   });
@@ -706,7 +713,8 @@ lrt_status lrt_autotune(lrt_scene* s, const float* pos_near, const float* dir_fa
     if (!pos_near || !dir_far || !hits || n == 0) return fail(LRT_ERR_INVALID_ARG, "autotune needs a non-empty ray batch");
     lrt::Scene& sc = s->s;
     const lrt::TuneConfig start{sc.block, sc.lds_stack, sc.xcd_remap, sc.budget, sc.tail_waves,
-                                sc.postpone_triangles() ? 1 : 0, sc.ray_groups, sc.persistent};
+                                sc.postpone_triangles() ? 1 : 0, sc.ray_groups, sc.persistent, sc.wide ? 1 : 0};
+    const bool tune_wide = !sc.wideBlocks.empty();
     // the option only exists for triangle-only scenes
     const bool tune_postpone = sc.leaf_kinds() == lrt::LK_TRI;
     auto apply = [&](const lrt::TuneConfig& c) {
@@ -717,6 +725,7 @@ lrt_status lrt_autotune(lrt_scene* s, const float* pos_near, const float* dir_fa
       sc.tail_waves = c.tail_waves;
       sc.ray_groups = c.ray_groups;
       sc.persistent = c.persistent;
+      sc.wide = c.wide != 0;
       if (tune_postpone) sc.leaf_postpone = c.postpone;
     };
     lrt_status st = LRT_OK;
@@ -727,7 +736,7 @@ lrt_status lrt_autotune(lrt_scene* s, const float* pos_near, const float* dir_fa
     };
     lrt::TuneResult r{};
     const int start_mode = sc.leaf_postpone;
-    const hipError_t e = lrt::autotune(launch, reinterpret_cast<hipStream_t>(stream), start, tune_postpone, 3, &r);
+    const hipError_t e = lrt::autotune(launch, reinterpret_cast<hipStream_t>(stream), start, tune_postpone, tune_wide, 3, &r);
     if (e != hipSuccess) {
       apply(start);
       sc.leaf_postpone = start_mode;
@@ -1061,6 +1070,22 @@ lrt_status lrt_get_array(lrt_scene* s, const char* name, void* dst, size_t* byte
     const std::string n = name;
     const void* src = nullptr;
     size_t sz = 0;
+    // the six-wide tree: what the kernels read, or (not committed to a device) what a commit would upload
+    std::vector<lrt::WideBlock> wide_copy;
+    if (n == "wide_blocks" || n == "wide_root") {
+      if (!c.committed && !s->s.tlas.empty()) {
+        s->s.build_device_layout();
+        s->s.build_wide();
+      }
+      wide_copy = c.wideBlocks;
+      if (c.committed && !wide_copy.empty()) {
+        const hipError_t e = hipMemcpy(wide_copy.data(), c.dev.at("wide").ptr(), wide_copy.size() * sizeof(lrt::WideBlock),
+                                       hipMemcpyDeviceToHost);
+        if (e != hipSuccess) return hip_fail(e, "wide tree copy");
+      }
+      if (n == "wide_blocks") { src = wide_copy.data(); sz = wide_copy.size() * sizeof(lrt::WideBlock); }
+      else { src = &c.wideRoot; sz = sizeof(c.wideRoot); }
+    }
 #define ARR(key, vec)                                   \
   if (n == key) { src = vec.data(); sz = vec.size() * sizeof(vec[0]); }
     ARR("nodes", c.nodePairs) ARR("tlas", c.tlas) ARR("instances", c.instances) ARR("geoms", c.geomData)
@@ -1099,7 +1124,7 @@ lrt_status lrt_get_array(lrt_scene* s, const char* name, void* dst, size_t* byte
                                     "orig_nodes", "frame_nodes", "frame_roots", "frame_tex_nodes", "frame_tex_roots",
                                     "sbs_nodes", "sbs_data",
                                     "sbs_data_f", "sbs_roots", "sbs_headers", "multi_nodes", "multi_values", "preset", "orig_indices", "svs_nodes", "svs_roots", "tlas_parent", "grid_data", "grid_offsets", "grid_sizes", "gprim_headers", "gprim_points", "coct_data", "coct_geoms", "coct_mods", "dag_nodes", "dag_child_edges", "dag_data_edges", "dag_distances", "dag_geoms", "dag_mods", "rot_add", "scom2_data", "scom2_headers", "scom2_mods",
-                                    "sbs_mask"};
+                                    "sbs_mask", "wide_blocks"};
       bool ok = false;
       for (const char* k : known) ok = ok || n == k;
       if (!ok) return fail(LRT_ERR_INVALID_ARG, "unknown array '" + n + "'");

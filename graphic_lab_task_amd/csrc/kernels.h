@@ -32,6 +32,8 @@ struct TraceArgs {
                               // (power of two; 0 or 64: rays in thread order)
   uint32_t      persistent;   // 1: one persistent single-pass kernel with per-lane ray refill
   uint32_t*     pcount;       // its two counters (device, zero between calls)
+  uint64_t      spill_words;  // words of the spill
+  uint32_t      wide;         // 1: the six-wide walk where the scene has a wide tree
 };
 // Rays beyond n that the work buffer's spill covers, so that a persistent grid (whole blocks of
 // resident lanes, at most ceil(n / block) blocks) can index it by lane slot.
@@ -155,6 +157,15 @@ hipError_t launch_tlas_refit(BVHNode* tlas, uint32_t n_nodes, const uint32_t* pa
                              uint32_t* counters, hipStream_t stream);
 
 hipError_t launch_trace(const SceneView& s, const TraceArgs& a, hipStream_t stream);
+// Largest batch of the wide walk: its counter runs past the batch by a chunk a wave.
+constexpr uint32_t WIDE_MAX_RAYS = 0xF0000000u;
+// The wide walk of a scene with a wide tree (trace_wide.hip) and the sequential pass over the rays it queues.
+hipError_t launch_trace_wide(const SceneView& s, const TraceArgs& a, hipStream_t stream);
+// Wide instance level after a TLAS refit: instance blocks from the instances, node planes from the TLAS
+// boxes. sources: six TLAS node indices per block (0xFFFFFFFF: none) for the first n_blocks blocks; no
+// blocks for a scene of one instance, whose instance is at block 0.
+hipError_t launch_wide_refit(WideBlock* blocks, uint32_t n_blocks, const uint32_t* sources, const BVHNode* tlas,
+                             const InstanceData* inst, hipStream_t stream);
 // launch_trace with the library's fixed per-device work array as queue and spill (a.queue and
 // a.spill are ignored): at most LRT_NOALLOC_MAX_RAYS rays, no counters; `device` is current.
 hipError_t launch_trace_noalloc(const SceneView& s, TraceArgs a, int device, hipStream_t stream);

@@ -43,7 +43,7 @@ Scene::StreamWork& Scene::stream_work(void* stream) {
 }
 
 hipError_t Scene::work_for(StreamWork& w, void* stream, size_t n, uint32_t** spill, TailQueue** queue,
-                           uint32_t** pcount) {
+                           uint32_t** pcount, uint64_t* spill_words) {
   // 256-B header: the tail queue's counters and list pointer at 0, the persistent kernel's two
   // counters at byte 64; then the queue list (4 B per ray) and the spill, sized for the smallest
   // LDS part so that a later launch-config change never overruns it, and for a persistent grid's
@@ -73,6 +73,7 @@ hipError_t Scene::work_for(StreamWork& w, void* stream, size_t n, uint32_t** spi
   *queue = static_cast<TailQueue*>(w.buf.ptr());
   *pcount = reinterpret_cast<uint32_t*>(static_cast<char*>(w.buf.ptr()) + 64);
   *spill = reinterpret_cast<uint32_t*>(static_cast<char*>(w.buf.ptr()) + head + (w.cap_rays * 4 + 255) / 256 * 256);
+  if (spill_words) *spill_words = uint64_t(w.cap_rays + SPILL_SLACK_RAYS) * (STACK_SIZE - 8);
   return hipSuccess;
 }
 
@@ -715,12 +716,66 @@ hipError_t Scene::commit_instances() {
     if (e != hipSuccess) return e;
     lastCommitKind = 2;
   }
+  if (!wideBlocks.empty()) {
+    WideBlock* blocks = static_cast<WideBlock*>(dev["wide"].ptr());
+    if (rebuild) {
+      uint32_t levels = 0;
+      if (build_wide_instances(&levels) && levels + wideBlasLevels <= WIDE_MAX_LEVELS) {
+        wideLevels = levels + wideBlasLevels;
+        e = hipMemcpy(blocks, wideBlocks.data(), 3 * instances.size() * sizeof(WideBlock), hipMemcpyHostToDevice);
+        if (e != hipSuccess) return e;
+        e = dev["wide_sources"].upload(wideSources.data(), wideSources.size() * sizeof(uint32_t));
+        if (e != hipSuccess) return e;
+      } else {
+        wideBlocks.clear();
+      }
+    } else {
+      e = launch_wide_refit(blocks, uint32_t(wideSources.size() / WIDE_CHILDREN),
+                            static_cast<const uint32_t*>(dev["wide_sources"].ptr()), static_cast<const BVHNode*>(dev["tlas"].ptr()),
+                            static_cast<const InstanceData*>(dev["instances"].ptr()), nullptr);
+      if (e != hipSuccess) return e;
+    }
+  }
   update_cache_geom();
   e = hipDeviceSynchronize();
   if (e != hipSuccess) return e;
   committed = true;
   return hipSuccess;
 }
+
+namespace {
+// Stores the first triangle index of every pair's right side in right.escapeIndex (the BLAS walks do not
+// read escape indices). False unless every left side's indices come before its right side's.
+bool mark_right_sides(BVHNodePair* pairs, uint32_t count) {
+  struct Visit { uint32_t pair; bool done; };
+  std::vector<Visit> stack{{0u, false}};
+  std::vector<uint2> range(count);   // first index and one past the last
+  while (!stack.empty()) {
+    const Visit v = stack.back();
+    stack.pop_back();
+    BVHNodePair& p = pairs[v.pair];
+    if (!v.done) {
+      stack.push_back({v.pair, true});
+      for (const BVHNode* ch : {&p.left, &p.right})
+        if (!(ch->leftOffset & LEAF_BIT)) stack.push_back({ch->leftOffset, false});
+      continue;
+    }
+    uint2 side[2];
+    int k = 0;
+    for (const BVHNode* ch : {&p.left, &p.right}) {
+      if (ch->leftOffset == LEAF_NORMAL) side[k] = uint2{0xFFFFFFFFu, 0xFFFFFFFFu};   // an empty leaf, on the right
+      else if (ch->leftOffset & LEAF_BIT)
+        side[k] = uint2{extract_start(ch->leftOffset), extract_start(ch->leftOffset) + extract_count(ch->leftOffset)};
+      else side[k] = range[ch->leftOffset];
+      ++k;
+    }
+    if (side[0].y > side[1].x) return false;
+    p.right.escapeIndex = side[1].x;
+    range[v.pair] = uint2{side[0].x, side[1].x == 0xFFFFFFFFu ? side[0].y : side[1].y};
+  }
+  return true;
+}
+}  // namespace
 
 // Derives the arrays the kernels read from the reference-layout host arrays. The traversal
 // visits the same nodes in the same order and tests the same floats, so hits are unchanged:
@@ -733,6 +788,7 @@ hipError_t Scene::commit_instances() {
 //  * frame-octree leaf boxes carry their 8 corner distances in one 64-byte record.
 void Scene::build_device_layout() {
   devNodes = nodePairs;
+  devOrdered.assign(geomData.size(), 0u);
   // pair ranges per geometry (geometries append their pairs in order)
   std::vector<std::pair<uint32_t, uint32_t>> ranges(geomData.size());
   for (size_t g = 0; g < geomData.size(); ++g) {
@@ -776,6 +832,7 @@ void Scene::build_device_layout() {
       }
       devNodes[b + k] = pr;
     }
+    if (tri) devOrdered[g] = mark_right_sides(devNodes.data() + b, c) ? 1 : 0;
   }
   // triangle soup in leaf order
   triSoup.assign(indices.size(), float4{0, 0, 0, 0});
@@ -857,6 +914,7 @@ hipError_t Scene::commit() {
   invalidate();   // buffers below may move
   build_host();
   build_device_layout();
+  build_wide();
   // occupancy-mask layout: per brick 1 summary word + ceil(bs^3 / 32) bit words
   sbsMaskGeoms.clear();
   sbsMaskBase.assign(sbsRoots.size(), 0u);
@@ -875,6 +933,7 @@ hipError_t Scene::commit() {
 #define UP(name, vec)                                                        \
   e = dev[name].upload(vec.data(), vec.size() * sizeof(vec[0]));             \
   if (e != hipSuccess) return e;
+  UP("wide", wideBlocks) UP("wide_sources", wideSources)
   UP("nodes", devNodes) UP("tri_soup", triSoup) UP("frame_leaves", frameLeaves) UP("frame_tex", frameTex) UP("tlas", tlas) UP("instances", instances) UP("geoms", geomData) UP("geom_tags", geomTags)
   UP("start_end", startEnd) UP("prim_id_count", primIdCount) UP("vert_pos", vertPos) UP("vert_norm", vertNorm)
   UP("indices", indices) UP("prim_indices", primIndices) UP("orig_nodes", origNodes) UP("frame_nodes", frameNodes)
@@ -928,6 +987,9 @@ SceneView Scene::make_view() const {
   v.tri_soup = (const float4*)P("tri_soup");
   v.frame_leaves = (const FrameLeaf*)P("frame_leaves");
   v.frame_tex = (const float4*)P("frame_tex");
+  v.wide = wideBlocks.empty() ? nullptr : (const WideBlock*)P("wide");
+  v.wide_root = wideRoot;
+  v.wide_levels = wideLevels;
   v.instances = (const InstanceData*)P("instances");
   v.geoms = (const GeomData*)P("geoms");
   v.geom_tags = (const uint32_t*)P("geom_tags");

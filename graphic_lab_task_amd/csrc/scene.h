@@ -92,10 +92,17 @@ struct Scene {
 
   // Device layout derived at commit (same traversal, fewer dependent loads per step).
   std::vector<BVHNodePair> devNodes;
+  std::vector<uint8_t> devOrdered;   // per mesh: 1 if leaf triangle indices grow from left to right
   std::vector<float4> triSoup;
   std::vector<FrameLeaf> frameLeaves;
   std::vector<float4> frameTex;      // 4 float4 per textured frame-octree leaf
   uint32_t cacheGeom = 0xFFFFFFFFu, cachePairs = 0;
+  // Six-wide tree (wide_bvh.h): three blocks per instance for the instance level, then the
+  // geometries; empty where the wide walk does not apply.
+  std::vector<WideBlock> wideBlocks;
+  std::vector<uint32_t> wideSources;   // six TLAS node indices per block of the instance level
+  std::vector<uint32_t> wideRoots;     // per geometry
+  uint32_t wideRoot = 0, wideBlasLevels = 0, wideLevels = 0;
 
   bool committed = false;
   int device = 0;
@@ -108,6 +115,7 @@ struct Scene {
   // Triangle leaf postponement in pass 1: -1 automatic (on for a triangle-only scene with one
   // instance), 0 off, 1 on.
   int leaf_postpone = -1;
+  bool wide = true;     // the six-wide walk where the scene has its tree; off once a launch shape is asked for
   int persistent = 0;   // 1: persistent single-pass trace kernel with per-lane ray refill
 
   // BLAS builder: false the host binned SAH, true the GPU linear BVH (build names "gpu...").
@@ -138,8 +146,10 @@ struct Scene {
   std::mutex work_mu;   // guards the map only
   std::map<void*, std::unique_ptr<StreamWork>> work;
   StreamWork& stream_work(void* stream);
-  // With w.mu held: queue, spill and persistent-kernel counters for n rays on `stream`.
-  hipError_t work_for(StreamWork& w, void* stream, size_t n, uint32_t** spill, TailQueue** queue, uint32_t** pcount);
+  // With w.mu held: queue, spill (of *spill_words words) and persistent-kernel counters for n rays on
+  // `stream`.
+  hipError_t work_for(StreamWork& w, void* stream, size_t n, uint32_t** spill, TailQueue** queue, uint32_t** pcount,
+                      uint64_t* spill_words = nullptr);
   // With w.mu held: the stream's occupancy-mask buffer.
   hipError_t mask_for(StreamWork& w, void* stream, uint32_t** mask);
 
@@ -185,6 +195,8 @@ struct Scene {
   hipError_t commit_instances();   // commit after instance updates only (geometry unchanged)
   void update_cache_geom();
   void build_device_layout();
+  void build_wide();
+  bool build_wide_instances(uint32_t* levels);
   hipError_t commit(); // device upload of every array
   void set_preset(const MultiRenderPreset& p);
   uint32_t leaf_kinds() const;

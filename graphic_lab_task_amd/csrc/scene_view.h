@@ -1,6 +1,7 @@
 // Plain device-pointer view of a committed scene, passed to kernels by value.
 #pragma once
 #include "lrt_types.h"
+#include "wide_bvh.h"
 
 namespace lrt {
 
@@ -107,6 +108,11 @@ struct SceneView {
   const SCom2Header*        scom2_headers; // m_SCom2Headers (GeomData.offset.y), offsets made global
   const int4*               scom2_mods;    // 3 x 48 index modifiers per tree
   uint32_t                  scom2_fast;    // 1: SCom2 leaves take the fast traversal (support_fast_scom_traversal)
+
+  // six-wide tree of the scene (wide_bvh.h), null where the wide walk does not apply
+  const WideBlock* wide;
+  uint32_t         wide_root;
+  uint32_t         wide_levels;     // most nodes on a path
 
   MultiRenderPreset preset;
   float    lod_thr;                 // m_precomputedLoDThr

@@ -429,14 +429,12 @@ __device__ __forceinline__ float frame_tex_interp(const float tc[16], float3 dp,
 // TEX (kernels taking LK_FRAME_TEX) a textured octree's hit also takes its texture coordinates
 // (LocalSurfaceIntersection, :689-710).
 template <bool TEX = false>
-__device__ __forceinline__ void frame_node_intersect(const SceneView& s, const GeomRef& g, float3 ray_pos, float3 ray_dir,
-                                                     float tNear, uint32_t instId, uint32_t geomId,
-                                                     uint32_t bvhNodeId, CRT_Hit& hit) {
-  const uint32_t type = g.type;
+__device__ __forceinline__ void frame_leaf_intersect(const SceneView& s, uint32_t type, const FrameLeaf* leaf,
+                                                     float3 ray_pos, float3 ray_dir, float tNear, uint32_t instId,
+                                                     uint32_t geomId, CRT_Hit& hit) {
   // frame octrees and sparse voxel sets (BVH2Common.cpp:141-218): one leaf record per BLAS leaf
   if (type != TYPE_SDF_FRAME_OCTREE && type != TYPE_SDF_SVS && (!TEX || type != TYPE_SDF_FRAME_OCTREE_TEX)) return;
-  const uint2 go = g.offset;   // y: first leaf record of this geometry
-  const float4* q = reinterpret_cast<const float4*>(s.frame_leaves + go.y + bvhNodeId);
+  const float4* q = reinterpret_cast<const float4*>(leaf);
   const float4 r0 = q[0], r1 = q[1], r2 = q[2], r3 = q[3];
   const float3 min_pos = make3(r0.x, r0.y, r0.z);
   const float3 max_pos = make3(r0.w, r1.x, r1.y);
@@ -465,6 +463,15 @@ __device__ __forceinline__ void frame_node_intersect(const SceneView& s, const G
     hit.coords[0] = frame_tex_interp(tc, dp, 0);
     hit.coords[1] = frame_tex_interp(tc, dp, 1);
   }
+}
+
+template <bool TEX = false>
+__device__ __forceinline__ void frame_node_intersect(const SceneView& s, const GeomRef& g, float3 ray_pos, float3 ray_dir,
+                                                     float tNear, uint32_t instId, uint32_t geomId,
+                                                     uint32_t bvhNodeId, CRT_Hit& hit) {
+  // offset.y: first leaf record of this geometry
+  frame_leaf_intersect<TEX>(s, g.type, s.frame_leaves + g.offset.y + bvhNodeId, ray_pos, ray_dir, tNear, instId, geomId,
+                            hit);
 }
 
 // BVHRT::load_distance_values (BVH2Common.cpp:846-882); returns the minimum value.

@@ -76,7 +76,9 @@ __global__ void k_eye_rays(EyeRayParams prm, const float2* __restrict__ jitter, 
 hipError_t launch_trace(const SceneView& s, const TraceArgs& a, hipStream_t stream) {
   const uint32_t k = s.leaf_kinds & ~(LK_SBS_SMOOTH | LK_TRICUBIC);
   hipError_t e;
-  if (s.leaf_kinds & LK_TRICUBIC)
+  if (a.wide && s.wide && !a.counts && a.queue && a.pcount && a.n <= WIDE_MAX_RAYS)
+    e = launch_trace_wide(s, a, stream);
+  else if (s.leaf_kinds & LK_TRICUBIC)
     e = k == LK_SBS ? launch_trace_sbs_tricubic(s, a, stream) : launch_trace_mixed_tricubic(s, a, stream);
   else if (s.leaf_kinds & LK_SBS_SMOOTH)
     e = k == LK_SBS ? launch_trace_sbs_smooth(s, a, stream) : launch_trace_mixed_smooth(s, a, stream);
@@ -97,7 +99,7 @@ hipError_t launch_trace(const SceneView& s, const TraceArgs& a, hipStream_t stre
   else
     e = launch_trace_mixed(s, a, stream);
   // a call whose second pass did not launch must not leave queued rays to the next call
-  if (e != hipSuccess && a.budget != 0 && a.queue != nullptr && a.counts == nullptr) {
+  if (e != hipSuccess && a.queue != nullptr && a.counts == nullptr) {
     hipLaunchKernelGGL(k_queue_reset, dim3(1), dim3(64), 0, stream, a.queue);
     (void)hipGetLastError();
   }
@@ -133,6 +135,7 @@ hipError_t launch_trace_noalloc(const SceneView& s, TraceArgs a, int device, hip
   a.pcount = base + 16;
   uint32_t* list = base + NOALLOC_HEAD_WORDS;
   a.spill = list + LRT_NOALLOC_MAX_RAYS;
+  a.spill_words = NOALLOC_WORDS - NOALLOC_HEAD_WORDS - LRT_NOALLOC_MAX_RAYS;
   hipLaunchKernelGGL(k_queue_init, dim3(1), dim3(64), 0, stream, a.queue, list, a.pcount);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   return launch_trace(s, a, stream);

@@ -29,13 +29,13 @@ hipError_t time_one(const std::function<hipError_t(const TuneConfig&)>& launch, 
 bool same_config(const TuneConfig& a, const TuneConfig& b) {
   return a.block == b.block && a.lds_stack == b.lds_stack && a.xcd_remap == b.xcd_remap && a.budget == b.budget &&
          a.tail_waves == b.tail_waves && a.postpone == b.postpone && a.ray_groups == b.ray_groups &&
-         a.persistent == b.persistent;
+         a.persistent == b.persistent && a.wide == b.wide;
 }
 
 }  // namespace
 
 hipError_t autotune(const std::function<hipError_t(const TuneConfig&)>& launch, hipStream_t stream,
-                    const TuneConfig& start, bool tune_postpone, int reps, TuneResult* out) {
+                    const TuneConfig& start, bool tune_postpone, bool tune_wide, int reps, TuneResult* out) {
   hipEvent_t e0 = nullptr, e1 = nullptr;
   hipError_t e = hipEventCreate(&e0);
   if (e == hipSuccess) e = hipEventCreate(&e1);
@@ -56,6 +56,11 @@ hipError_t autotune(const std::function<hipError_t(const TuneConfig&)>& launch, 
     return hipSuccess;
   };
   const int n_postpone = tune_postpone ? 2 : 1;
+  if (tune_wide && e == hipSuccess) {
+    TuneConfig c = start;
+    c.wide = 1;
+    e = consider(c, false);
+  }
   for (int pp = 0; pp < n_postpone && e == hipSuccess; ++pp) {
     for (uint32_t groups : {0u, 8u, 32u}) {
       for (int block : {64, 128, 256}) {
@@ -66,6 +71,7 @@ hipError_t autotune(const std::function<hipError_t(const TuneConfig&)>& launch, 
           c.budget = 0;
           c.ray_groups = groups;
           c.persistent = 0;
+          c.wide = 0;
           if (tune_postpone) c.postpone = pp;
           if ((e = consider(c, true)) != hipSuccess) break;
           if (groups == 0) {   // the persistent kernel takes rays in order: no interleaving

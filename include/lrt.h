@@ -286,7 +286,14 @@ lrt_status lrt_query_one(lrt_scene* s, const float* pos_near4, const float* dir_
 lrt_status lrt_eye_rays_dev(const float* proj_inv16, const float* world_view_inv16, uint32_t width, uint32_t height,
                             const float* jitter, uint32_t order, float* pos_near, float* dir_far, void* stream);
 
-/* Kernel configuration used by the trace calls: block size (64/128/256), number of traversal
+/* Scenes of triangle meshes, and scenes of one frame-octree or sparse-voxel-set instance, are traced by
+ * a six-wide walk built at commit that has no launch shape to choose (other scenes, counted calls and
+ * the INTERSECTION_COUNT mode take the binary walk). Each of the launch-shape calls below
+ * (lrt_set_launch_config, lrt_set_tail_config, lrt_set_leaf_postponement with 0 or 1,
+ * lrt_set_ray_interleave, lrt_set_persistent) moves the scene to the binary walk in that shape;
+ * lrt_autotune tries both and keeps the faster. Same hit records either way.
+ *
+ * Kernel configuration used by the trace calls: block size (64/128/256), number of traversal
  * stack entries kept in LDS (8/16/32), XCD-contiguous block mapping (0/1). */
 lrt_status lrt_set_launch_config(lrt_scene* s, int block, int lds_stack, int xcd_remap);
 
@@ -434,7 +441,8 @@ lrt_status lrt_stack_overflow_count(lrt_scene* s, uint64_t* out, int reset);
  * "svs_nodes" (SdfSVSNode), "svs_roots", "tlas_parent" (uint32: parent node of each TLAS node),
  * "grid_data" (float), "grid_offsets", "grid_sizes" (uint32, 3 per grid),
  * "gprim_headers" (GraphicsPrimHeader), "gprim_points" (float4),
- * "preset", and "sbs_mask" (uint32: the committed voxel occupancy
+ * "preset", "wide_blocks" and "wide_root" (uint32: the six-wide tree, 16 words a block, as a commit
+ * uploads it; empty where the scene is traced by the binary walk), and "sbs_mask" (uint32: the committed voxel occupancy
  * masks, per brick set in order and per brick one summary word then ceil(bs^3/32) bit words,
  * bit v set when the minimum of voxel v's 8 corner values is <= 0; copied from the device).
  * With dst == NULL only *bytes is written. */

@@ -1,0 +1,247 @@
+"""The wide walk (trace_wide.hip, the default on triangle scenes and single ordered frame octrees)
+against the binary walk, record for record: tile and batch edges, instances, first-hit and any-hit rays,
+rays and scenes that fall back to the sequential walk, a tree deeper than the LDS stack, the refitted
+instance level, graph replay and the allocation-free entry point."""
+import numpy as np
+import pytest
+
+from conftest import raw_equal
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch_dev():
+    import torch
+    assert torch.cuda.is_available()
+    torch.cuda.set_device(0)
+    return torch
+
+
+def trace(torch, g, s, pos, dirs, fn="trace_closest"):
+    hits = torch.full((pos.shape[0], 8), -5, dtype=torch.int32, device="cuda")
+    getattr(s, fn)(pos, dirs, hits)
+    torch.cuda.synchronize()
+    return hits.cpu().numpy().view(g.HIT_DTYPE).reshape(-1)
+
+
+def flags(torch, s, pos, dirs):
+    out = torch.full((pos.shape[0],), 7, dtype=torch.int32, device="cuda")
+    s.trace_any(pos, dirs, out)
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+class Both:
+    """The same scene twice: the default (wide) walk and the binary walk."""
+
+    def __init__(self, g, build):
+        self.g = g
+        self.wide, self.binary = build(), build()
+        self.binary.set_launch_config(256, 16, True)
+        self.binary.set_tail_config(0, 1024)
+        assert self.wide.get_array("wide_blocks").size
+
+    def check(self, torch, pos, dirs, fn="trace_closest", any_hit=True):
+        a, b = (trace(torch, self.g, s, pos, dirs, fn) for s in (self.wide, self.binary))
+        assert raw_equal(a, b), int((a.view(np.uint8).reshape(-1, 32) != b.view(np.uint8).reshape(-1, 32)).any(1).sum())
+        if any_hit:
+            assert np.array_equal(flags(torch, self.wide, pos, dirs), flags(torch, self.binary, pos, dirs))
+        return a
+
+
+def mesh(g, n, mats=(None,), seed=1, build="cbvh_embree2"):
+    def make():
+        s = g.SceneRT(build_name=build)
+        gid = s.AddGeom_Triangles3f(*g.gen_geodesic(n, 0.05, 4.0, seed))
+        for m in mats:
+            s.AddInstance(gid, m)
+        s.CommitScene()
+        return s
+    return make
+
+
+def random_rays(torch, n, seed, extent=1.5, far=100.0):
+    rng = np.random.default_rng(seed)
+    pos = np.concatenate([rng.uniform(-extent, extent, (n, 3)), np.full((n, 1), 1e-4)], 1).astype(np.float32)
+    d = rng.normal(size=(n, 3))
+    dirs = np.concatenate([d / np.linalg.norm(d, axis=1, keepdims=True), np.full((n, 1), far)], 1).astype(np.float32)
+    return torch.from_numpy(pos).cuda(), torch.from_numpy(dirs).cuda()
+
+
+def mats(n, seed, extent):
+    rng = np.random.default_rng(seed)
+    out = []
+    for _ in range(n):
+        m = np.eye(4, dtype=np.float32)
+        q, r = np.linalg.qr(rng.normal(size=(3, 3)))
+        m[:3, :3] = q * rng.uniform(0.5, 2.0)
+        m[:3, 3] = rng.uniform(-extent, extent, 3)
+        out.append(m)
+    return out
+
+
+@pytest.mark.parametrize("n_rays", [1, 63, 64, 65, 4097, 700001])
+@pytest.mark.parametrize("n", [1, 7, 64])
+def test_mesh(lrt, torch_dev, n, n_rays):
+    b = Both(lrt, mesh(lrt, n))
+    pos, dirs = random_rays(torch_dev, n_rays, n_rays)
+    hits = b.check(torch_dev, pos, dirs)
+    if n_rays > 60:
+        assert 0 < (hits["primId"] != lrt.MISS).sum()
+
+
+@pytest.mark.parametrize("build", ["cbvh_embree1", "cbvh_embree4", "gpu_lbvh2"])
+def test_builders(lrt, torch_dev, build):
+    Both(lrt, mesh(lrt, 20, build=build)).check(torch_dev, *random_rays(torch_dev, 50000, 3))
+
+
+@pytest.mark.parametrize("n_inst", [2, 6, 7, 300])
+def test_instances(lrt, torch_dev, n_inst):
+    b = Both(lrt, mesh(lrt, 12, mats(n_inst, n_inst, 4.0)))
+    b.check(torch_dev, *random_rays(torch_dev, 200003, 5, extent=5.0))
+
+
+def test_first_hit_and_short_rays(lrt, torch_dev):
+    b = Both(lrt, mesh(lrt, 12, mats(20, 4, 3.0)))
+    pos, dirs = random_rays(torch_dev, 30000, 6, extent=4.0, far=0.7)
+    dirs[::3, 3] *= -1   # stops at the sequential walk's first hit
+    dirs[::7, 3] = 0.0
+    b.check(torch_dev, pos, dirs)
+    pos[:, 3] = 0.5   # near plane inside the scene
+    b.check(torch_dev, pos, dirs)
+
+
+def test_special_rays(lrt, torch_dev):
+    b = Both(lrt, mesh(lrt, 9, mats(3, 4, 1.0) + [None]))
+    pos, dirs = random_rays(torch_dev, 9000, 7)
+    dirs[0::9, 0] = 0.0
+    dirs[1::9, :2] = 0.0
+    dirs[2::9, 1] = -0.0
+    dirs[3::9, 2] = 1e-30
+    pos[4::9, 0] = float("inf")
+    pos[5::9, 1] = float("nan")
+    dirs[6::9, 2] = float("nan")
+    dirs[7::9, 3] = float("inf")
+    pos[8::9, 3] = -1.0
+    b.check(torch_dev, pos, dirs)
+
+
+def test_ties(lrt, torch_dev):
+    """Every surface twice, and coplanar tessellations: equal distances are the sequential walk's call."""
+    v, f = lrt.gen_geodesic(8, 0.05, 4.0, 2)
+
+    def make():
+        s = lrt.SceneRT()
+        gid = s.AddGeom_Triangles3f(np.concatenate([v, v]), np.concatenate([f, f + v.shape[0]]))
+        s.AddInstance(gid)
+        s.AddInstance(gid)
+        x, y = np.meshgrid(np.arange(9, dtype=np.float32), np.arange(9, dtype=np.float32), indexing="ij")
+        grid = np.stack([x.ravel() - 4, y.ravel() - 4, np.full(81, 0.25, np.float32)], 1)
+        q = (np.arange(8)[:, None] * 9 + np.arange(8)).ravel()
+        tri = np.concatenate([np.stack([q, q + 9, q + 1], 1), np.stack([q + 1, q + 9, q + 10], 1)]).astype(np.uint32)
+        s.AddInstance(s.AddGeom_Triangles3f(grid, tri))
+        s.CommitScene()
+        return s
+
+    b = Both(lrt, make)
+    pos, dirs = random_rays(torch_dev, 40000, 8, extent=3.0)
+    b.check(torch_dev, pos, dirs)
+    # through the lattice's vertices and edges
+    t = np.random.default_rng(1).integers(-4, 5, (5000, 2)).astype(np.float32)
+    p = pos[:5000].clone()
+    d = torch_dev.from_numpy(np.concatenate([t, np.full((5000, 1), 0.25, np.float32)], 1)).cuda() - p[:, :3]
+    dirs[:5000, :3] = d / d.norm(dim=1, keepdim=True)
+    b.check(torch_dev, p, dirs[:5000].contiguous())
+
+
+def test_deep_tree(lrt, torch_dev):
+    """Triangles whose sizes fall by half each: a chain of nodes, more levels than stack entries in LDS."""
+    n = 66
+    k = 0.5 ** np.arange(n)
+    v = np.stack([np.stack([k, k * 0, k], 1), np.stack([k, k, -k], 1), np.stack([k, -k, k * 0], 1)], 1)
+    v = v.reshape(-1, 3).astype(np.float32)
+    f = np.arange(3 * n, dtype=np.uint32).reshape(-1, 3)
+
+    def make():
+        s = lrt.SceneRT()
+        s.AddInstance(s.AddGeom_Triangles3f(v, f))
+        s.CommitScene()
+        return s
+
+    b = Both(lrt, make)
+    rng = np.random.default_rng(3)
+    pos, dirs = random_rays(torch_dev, 20000, 9, extent=0.2)
+    target = torch_dev.from_numpy((rng.normal(size=(20000, 3)) * 0.5 ** rng.uniform(0, 30, (20000, 1))).astype(np.float32))
+    d = target.cuda() - pos[:, :3]
+    dirs[:, :3] = d / d.norm(dim=1, keepdim=True)
+    b.check(torch_dev, pos, dirs)
+
+
+@pytest.mark.parametrize("depth", [2, 5, 8])
+def test_frame_octree(lrt, torch_dev, depth):
+    rng = np.random.default_rng(2)
+    sph = np.concatenate([rng.uniform(-0.8, 0.8, (24, 3)), rng.uniform(0.1, 0.3, (24, 1))], 1).astype(np.float32)
+    nodes = lrt.sdf_spheres_frame_octree(sph, depth)
+
+    for mode in (lrt.SDF_OCTREE_NODE_INTERSECT_ANALYTIC, lrt.SDF_OCTREE_NODE_INTERSECT_BBOX):
+        for m in (None, mats(1, 3, 0.3)[0]):
+            def make():
+                s = lrt.SceneRT()
+                s.AddInstance(s.AddGeom_SdfFrameOctree(nodes), m)
+                p = lrt.default_preset()
+                p["sdf_node_intersect"] = mode
+                s.SetPreset(p)
+                s.CommitScene()
+                return s
+
+            b = Both(lrt, make)
+            pos, dirs = random_rays(torch_dev, 100003, 10, extent=2.0)
+            dirs[::5, 3] *= -1
+            dirs[::11, 0] = 0.0
+            hits = b.check(torch_dev, pos, dirs)
+            assert (hits["primId"] != lrt.MISS).sum() > 100
+
+
+def test_instance_updates(lrt, torch_dev):
+    start, moved, far_off = mats(40, 1, 4.0), mats(40, 2, 4.0), mats(40, 3, 60.0)
+    b = Both(lrt, mesh(lrt, 10, start))
+    pos, dirs = random_rays(torch_dev, 60000, 11, extent=5.0)
+    b.check(torch_dev, pos, dirs)
+    for step, kind in ((moved, 1), (far_off, 2), (start, None)):
+        for s in (b.wide, b.binary):
+            for i, m in enumerate(step):
+                s.UpdateInstance(i, m)
+            s.CommitScene()
+        if kind is not None:
+            assert b.wide.commit_info()["kind"] == kind
+        b.check(torch_dev, pos, dirs)
+    one = Both(lrt, mesh(lrt, 10, start[:1]))
+    for s in (one.wide, one.binary):
+        s.UpdateInstance(0, moved[0])
+        s.CommitScene()
+    one.check(torch_dev, pos, dirs)
+
+
+def test_graph_replay_and_noalloc(lrt, torch_dev):
+    torch = torch_dev
+    b = Both(lrt, mesh(lrt, 16, mats(9, 1, 2.0)))
+    pos, dirs = random_rays(torch, 60000, 12, extent=3.0)
+    dirs[::17, 1] = 0.0   # some rays take the second pass
+    want = b.check(torch, pos, dirs)
+    assert raw_equal(trace(torch, lrt, b.wide, pos, dirs, "trace_closest_noalloc"), want)
+    hits = torch.zeros((pos.shape[0], 8), dtype=torch.int32, device="cuda")
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        b.wide.trace_closest(pos, dirs, hits, stream=side.cuda_stream)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            b.wide.trace_closest(pos, dirs, hits, stream=torch.cuda.current_stream().cuda_stream)
+    for k in range(3):
+        hits.fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert raw_equal(hits.cpu().numpy().view(lrt.HIT_DTYPE).reshape(-1), want)
+        pos2, dirs2 = random_rays(torch, 1000 + k, k)
+        b.check(torch, pos2, dirs2)
