@@ -743,40 +743,6 @@ hipError_t Scene::commit_instances() {
   return hipSuccess;
 }
 
-namespace {
-// Stores the first triangle index of every pair's right side in right.escapeIndex (the BLAS walks do not
-// read escape indices). False unless every left side's indices come before its right side's.
-bool mark_right_sides(BVHNodePair* pairs, uint32_t count) {
-  struct Visit { uint32_t pair; bool done; };
-  std::vector<Visit> stack{{0u, false}};
-  std::vector<uint2> range(count);   // first index and one past the last
-  while (!stack.empty()) {
-    const Visit v = stack.back();
-    stack.pop_back();
-    BVHNodePair& p = pairs[v.pair];
-    if (!v.done) {
-      stack.push_back({v.pair, true});
-      for (const BVHNode* ch : {&p.left, &p.right})
-        if (!(ch->leftOffset & LEAF_BIT)) stack.push_back({ch->leftOffset, false});
-      continue;
-    }
-    uint2 side[2];
-    int k = 0;
-    for (const BVHNode* ch : {&p.left, &p.right}) {
-      if (ch->leftOffset == LEAF_NORMAL) side[k] = uint2{0xFFFFFFFFu, 0xFFFFFFFFu};   // an empty leaf, on the right
-      else if (ch->leftOffset & LEAF_BIT)
-        side[k] = uint2{extract_start(ch->leftOffset), extract_start(ch->leftOffset) + extract_count(ch->leftOffset)};
-      else side[k] = range[ch->leftOffset];
-      ++k;
-    }
-    if (side[0].y > side[1].x) return false;
-    p.right.escapeIndex = side[1].x;
-    range[v.pair] = uint2{side[0].x, side[1].x == 0xFFFFFFFFu ? side[0].y : side[1].y};
-  }
-  return true;
-}
-}  // namespace
-
 // Derives the arrays the kernels read from the reference-layout host arrays. The traversal
 // visits the same nodes in the same order and tests the same floats, so hits are unchanged:
 //  * each geometry's pairs are renumbered: its top BFS levels first (they are staged in LDS
@@ -788,7 +754,6 @@ bool mark_right_sides(BVHNodePair* pairs, uint32_t count) {
 //  * frame-octree leaf boxes carry their 8 corner distances in one 64-byte record.
 void Scene::build_device_layout() {
   devNodes = nodePairs;
-  devOrdered.assign(geomData.size(), 0u);
   // pair ranges per geometry (geometries append their pairs in order)
   std::vector<std::pair<uint32_t, uint32_t>> ranges(geomData.size());
   for (size_t g = 0; g < geomData.size(); ++g) {
@@ -832,7 +797,6 @@ void Scene::build_device_layout() {
       }
       devNodes[b + k] = pr;
     }
-    if (tri) devOrdered[g] = mark_right_sides(devNodes.data() + b, c) ? 1 : 0;
   }
   // triangle soup in leaf order
   triSoup.assign(indices.size(), float4{0, 0, 0, 0});

@@ -92,7 +92,6 @@ struct Scene {
 
   // Device layout derived at commit (same traversal, fewer dependent loads per step).
   std::vector<BVHNodePair> devNodes;
-  std::vector<uint8_t> devOrdered;   // per mesh: 1 if leaf triangle indices grow from left to right
   std::vector<float4> triSoup;
   std::vector<FrameLeaf> frameLeaves;
   std::vector<float4> frameTex;      // 4 float4 per textured frame-octree leaf

@@ -205,7 +205,8 @@ __device__ __forceinline__ float3 eval_grad_trilinear(const float v[8], float3 q
 // sign follow the start distance, as SURFACE mode does. OCTREE_TYPES compiles in what only the
 // multi-octree, DAG and SCom2 types use: the compact types' wider stopping distance on surface
 // nodes and the channel render modes' hit-point quotients (the other callers stay free of it).
-template <bool OCTREE_TYPES = false>
+// Without NORMAL the record's normal is that of an unlit render mode (callers that need only t).
+template <bool OCTREE_TYPES = false, bool NORMAL = true>
 __device__ bool local_surface_intersection(const SceneView& s, uint32_t type, float3 ray_dir, uint32_t instId,
                                            uint32_t geomId, const float values[8], uint32_t primId, float d,
                                            float qNear, float qFar, float2 fNearFar, float3 start_q,
@@ -362,7 +363,7 @@ __device__ bool local_surface_intersection(const SceneView& s, uint32_t type, fl
   const float tReal = fNearFar.x + d * t;
   if (t <= qFar && hitp && tReal < hit.t) {
     float3 norm = make3(0, 0, 1);
-    if (preset_needs_normal(s.preset.render_mode)) {
+    if (NORMAL && preset_needs_normal(s.preset.render_mode)) {
       if (early_hit && mode == SDF_OCTREE_NODE_INTERSECT_BBOX) {
         norm = make3(0, 0, 0);
         const float3 v = make3(fmax_ref(start_q.x, 1 - start_q.x), fmax_ref(start_q.y, 1 - start_q.y),
@@ -475,10 +476,9 @@ __device__ __forceinline__ void frame_node_intersect(const SceneView& s, const G
 }
 
 // BVHRT::load_distance_values (BVH2Common.cpp:846-882); returns the minimum value.
-__device__ __forceinline__ float sbs_load_values(const SceneView& s, const SdfSBSHeader& h, uint32_t nodeId,
-                                                 float3 voxelPos, uint32_t v_size, float sz_inv, float values[8]) {
+__device__ __forceinline__ float sbs_load_values_at(const SceneView& s, const SdfSBSHeader& h, uint32_t v_off,
+                                                    float3 voxelPos, uint32_t v_size, float sz_inv, float values[8]) {
   float vmin = 1e6f;
-  const uint32_t v_off = s.sbs_nodes[nodeId].data_offset;
   const uint32_t vx = uint32_t(voxelPos.x), vy = uint32_t(voxelPos.y), vz = uint32_t(voxelPos.z);
   if (h.aux_data == SDF_SBS_NODE_LAYOUT_ID32F_IRGB32F || h.aux_data == SDF_SBS_NODE_LAYOUT_ID32F_IRGB32F_IN) {
 #pragma unroll
@@ -505,6 +505,11 @@ __device__ __forceinline__ float sbs_load_values(const SceneView& s, const SdfSB
     }
   }
   return vmin;
+}
+
+__device__ __forceinline__ float sbs_load_values(const SceneView& s, const SdfSBSHeader& h, uint32_t nodeId,
+                                                 float3 voxelPos, uint32_t v_size, float sz_inv, float values[8]) {
+  return sbs_load_values_at(s, h, s.sbs_nodes[nodeId].data_offset, voxelPos, v_size, sz_inv, values);
 }
 
 // Value of lattice point (x, y, z) (corner coordinates 0..bs) of a brick, decoded exactly as
@@ -1026,6 +1031,70 @@ struct SbsVoxelRec {
   float t_local;
 };
 
+// Colour or texture coordinates (coords[0..1]) of a brick hit, from the brick's 8 corner entries.
+__device__ __forceinline__ void sbs_brick_coords(const SceneView& s, const SdfSBSHeader& header, uint32_t data_offset,
+                                                 uint32_t v_size, float3 brick_min_pos, float sz, float3 ray_pos,
+                                                 float3 ray_dir, CRT_Hit& hit) {
+  const float3 pos = ray_pos + hit.t * ray_dir;
+  const float3 dp = (pos - brick_min_pos) * (0.5f * sz);
+  const uint32_t aux = header.aux_data;
+  if (aux == SDF_SBS_NODE_LAYOUT_ID32F_IRGB32F || aux == SDF_SBS_NODE_LAYOUT_ID32F_IRGB32F_IN) {
+    const uint32_t t_off = data_offset + v_size * v_size * v_size;
+    float3 col = make3(0, 0, 0);
+    const float w[8] = {(1 - dp.x) * (1 - dp.y) * (1 - dp.z), (1 - dp.x) * (1 - dp.y) * (dp.z),
+                        (1 - dp.x) * (dp.y) * (1 - dp.z),     (1 - dp.x) * (dp.y) * (dp.z),
+                        (dp.x) * (1 - dp.y) * (1 - dp.z),     (dp.x) * (1 - dp.y) * (dp.z),
+                        (dp.x) * (dp.y) * (1 - dp.z),         (dp.x) * (dp.y) * (dp.z)};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t b = s.sbs_data[t_off + i];
+      const float3 c = make3(s.sbs_data_f[b + 0], s.sbs_data_f[b + 1], s.sbs_data_f[b + 2]);
+      col = (i == 0) ? w[0] * c : col + w[i] * c;
+    }
+    col = make3(clamp_ref(floorf(255.0f * col.x + 0.5f), 0.0f, 255.0f),
+                clamp_ref(floorf(255.0f * col.y + 0.5f), 0.0f, 255.0f),
+                clamp_ref(floorf(255.0f * col.z + 0.5f), 0.0f, 255.0f));
+    hit.coords[0] = col.x + col.y / 256.0f;
+    hit.coords[1] = col.z;
+  } else if (aux == SDF_SBS_NODE_LAYOUT_DX_RGB8) {
+    const uint32_t vals_per_int = 4 / header.bytes_per_value;
+    const uint32_t t_off = data_offset + (v_size * v_size * v_size + vals_per_int - 1) / vals_per_int;
+    const float w[8] = {(1 - dp.x) * (1 - dp.y) * (1 - dp.z), (1 - dp.x) * (1 - dp.y) * (dp.z),
+                        (1 - dp.x) * (dp.y) * (1 - dp.z),     (1 - dp.x) * (dp.y) * (dp.z),
+                        (dp.x) * (1 - dp.y) * (1 - dp.z),     (dp.x) * (1 - dp.y) * (dp.z),
+                        (dp.x) * (dp.y) * (1 - dp.z),         (dp.x) * (dp.y) * (dp.z)};
+    float3 col = make3(0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t c = s.sbs_data[t_off + i];
+      const float3 cf = make3(float((c >> 0) & 0xFF), float((c >> 8) & 0xFF), float((c >> 16) & 0xFF));
+      col = (i == 0) ? w[0] * cf : col + w[i] * cf;
+    }
+    col = make3(clamp_ref(floorf(col.x + 0.5f), 0.0f, 255.0f), clamp_ref(floorf(col.y + 0.5f), 0.0f, 255.0f),
+                clamp_ref(floorf(col.z + 0.5f), 0.0f, 255.0f));
+    hit.coords[0] = col.x + col.y / 256.0f;
+    hit.coords[1] = col.z;
+  } else if (aux == SDF_SBS_NODE_LAYOUT_DX_UV16) {
+    const uint32_t vals_per_int = 4 / header.bytes_per_value;
+    const uint32_t t_off = data_offset + (v_size * v_size * v_size + vals_per_int - 1) / vals_per_int;
+    const float w[8] = {(1 - dp.x) * (1 - dp.y) * (1 - dp.z), (1 - dp.x) * (1 - dp.y) * (dp.z),
+                        (1 - dp.x) * (dp.y) * (1 - dp.z),     (1 - dp.x) * (dp.y) * (dp.z),
+                        (dp.x) * (1 - dp.y) * (1 - dp.z),     (dp.x) * (1 - dp.y) * (dp.z),
+                        (dp.x) * (dp.y) * (1 - dp.z),         (dp.x) * (dp.y) * (dp.z)};
+    float u = 0, v = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t c = s.sbs_data[t_off + i];
+      const float tu = w[i] * (1.5259022e-5f * float(c >> 16));
+      const float tv = w[i] * (1.5259022e-5f * float(c & 0xFFFF));
+      u = (i == 0) ? tu : u + tu;
+      v = (i == 0) ? tv : v + tv;
+    }
+    hit.coords[0] = u;
+    hit.coords[1] = v;
+  }
+}
+
 // Sparse-brick-set leaf: BVHRT::OctreeBrickIntersect (BVH2Common.cpp:884-1112), trilinear.
 // Returns the number of voxels whose values were loaded (all voxels stepped without an
 // occupancy mask). `rec` (indexed layouts only) records the hit voxel. SMOOTH compiles in the
@@ -1128,67 +1197,48 @@ __device__ uint32_t sbs_brick_intersect(const SceneView& s, const GeomRef& g, fl
     }
     brick_fNearFar.x += fmax_ref(0.0f, fNearFar.y - brick_fNearFar.x) + 1e-6f;
   }
-  if (hit.t < old_t) {
-    const float3 pos = ray_pos + hit.t * ray_dir;
-    const float3 dp = (pos - brick_min_pos) * (0.5f * sz);
-    const uint32_t aux = header.aux_data;
-    if (aux == SDF_SBS_NODE_LAYOUT_ID32F_IRGB32F || aux == SDF_SBS_NODE_LAYOUT_ID32F_IRGB32F_IN) {
-      const uint32_t t_off = node.data_offset + v_size * v_size * v_size;
-      float3 col = make3(0, 0, 0);
-      const float w[8] = {(1 - dp.x) * (1 - dp.y) * (1 - dp.z), (1 - dp.x) * (1 - dp.y) * (dp.z),
-                          (1 - dp.x) * (dp.y) * (1 - dp.z),     (1 - dp.x) * (dp.y) * (dp.z),
-                          (dp.x) * (1 - dp.y) * (1 - dp.z),     (dp.x) * (1 - dp.y) * (dp.z),
-                          (dp.x) * (dp.y) * (1 - dp.z),         (dp.x) * (dp.y) * (dp.z)};
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const uint32_t b = s.sbs_data[t_off + i];
-        const float3 c = make3(s.sbs_data_f[b + 0], s.sbs_data_f[b + 1], s.sbs_data_f[b + 2]);
-        col = (i == 0) ? w[0] * c : col + w[i] * c;
-      }
-      col = make3(clamp_ref(floorf(255.0f * col.x + 0.5f), 0.0f, 255.0f),
-                  clamp_ref(floorf(255.0f * col.y + 0.5f), 0.0f, 255.0f),
-                  clamp_ref(floorf(255.0f * col.z + 0.5f), 0.0f, 255.0f));
-      hit.coords[0] = col.x + col.y / 256.0f;
-      hit.coords[1] = col.z;
-    } else if (aux == SDF_SBS_NODE_LAYOUT_DX_RGB8) {
-      const uint32_t vals_per_int = 4 / header.bytes_per_value;
-      const uint32_t t_off = node.data_offset + (v_size * v_size * v_size + vals_per_int - 1) / vals_per_int;
-      const float w[8] = {(1 - dp.x) * (1 - dp.y) * (1 - dp.z), (1 - dp.x) * (1 - dp.y) * (dp.z),
-                          (1 - dp.x) * (dp.y) * (1 - dp.z),     (1 - dp.x) * (dp.y) * (dp.z),
-                          (dp.x) * (1 - dp.y) * (1 - dp.z),     (dp.x) * (1 - dp.y) * (dp.z),
-                          (dp.x) * (dp.y) * (1 - dp.z),         (dp.x) * (dp.y) * (dp.z)};
-      float3 col = make3(0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const uint32_t c = s.sbs_data[t_off + i];
-        const float3 cf = make3(float((c >> 0) & 0xFF), float((c >> 8) & 0xFF), float((c >> 16) & 0xFF));
-        col = (i == 0) ? w[0] * cf : col + w[i] * cf;
-      }
-      col = make3(clamp_ref(floorf(col.x + 0.5f), 0.0f, 255.0f), clamp_ref(floorf(col.y + 0.5f), 0.0f, 255.0f),
-                  clamp_ref(floorf(col.z + 0.5f), 0.0f, 255.0f));
-      hit.coords[0] = col.x + col.y / 256.0f;
-      hit.coords[1] = col.z;
-    } else if (aux == SDF_SBS_NODE_LAYOUT_DX_UV16) {
-      const uint32_t vals_per_int = 4 / header.bytes_per_value;
-      const uint32_t t_off = node.data_offset + (v_size * v_size * v_size + vals_per_int - 1) / vals_per_int;
-      const float w[8] = {(1 - dp.x) * (1 - dp.y) * (1 - dp.z), (1 - dp.x) * (1 - dp.y) * (dp.z),
-                          (1 - dp.x) * (dp.y) * (1 - dp.z),     (1 - dp.x) * (dp.y) * (dp.z),
-                          (dp.x) * (1 - dp.y) * (1 - dp.z),     (dp.x) * (1 - dp.y) * (dp.z),
-                          (dp.x) * (dp.y) * (1 - dp.z),         (dp.x) * (dp.y) * (dp.z)};
-      float u = 0, v = 0;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const uint32_t c = s.sbs_data[t_off + i];
-        const float tu = w[i] * (1.5259022e-5f * float(c >> 16));
-        const float tv = w[i] * (1.5259022e-5f * float(c & 0xFFFF));
-        u = (i == 0) ? tu : u + tu;
-        v = (i == 0) ? tv : v + tv;
-      }
-      hit.coords[0] = u;
-      hit.coords[1] = v;
-    }
-  }
+  if (hit.t < old_t) sbs_brick_coords(s, header, node.data_offset, v_size, brick_min_pos, sz, ray_pos, ray_dir, hit);
   return loaded;
+}
+
+// The record of a hit voxel (x-major index `voxel` of brick `primId`), solved again with the march's own
+// arithmetic, which depends on the voxel alone. Returns the hit's t; miss_t where the voxel has none.
+__device__ __forceinline__ float sbs_voxel_rec(const SceneView& s, uint32_t type, uint32_t sdfId, float3 ray_pos,
+                                               float3 ray_dir, uint32_t instId, uint32_t geomId, uint32_t primId,
+                                               uint32_t voxel, CRT_Hit miss, SbsVoxelRec& rec) {
+  const SdfSBSHeader header = s.sbs_headers[sdfId];
+  const uint32_t nodeId = primId + s.sbs_roots[sdfId];
+  const SdfSBSNode node = s.sbs_nodes[nodeId];
+  const uint32_t v_size = header.brick_size + 2 * header.brick_pad + 1;
+  const float px = float(node.pos_xy >> 16);
+  const float py = float(node.pos_xy & 0x0000FFFF);
+  const float pz = float(node.pos_z_lod_size >> 16);
+  const float sz = float(node.pos_z_lod_size & 0x0000FFFF);
+  const float sz_inv = 2.0f / sz;
+  const float bs = float(header.brick_size);
+  const float d = 2.0f / (sz * bs);
+  const float scale = 0.5f * sz * bs;
+  const float3 brick_min_pos = make3(-1, -1, -1) + sz_inv * make3(px, py, pz);
+  const uint32_t vx = voxel / (header.brick_size * header.brick_size), vy = (voxel / header.brick_size) % header.brick_size,
+                 vz = voxel % header.brick_size;
+  const float3 voxelPos = make3(float(vx), float(vy), float(vz));
+  const float3 min_pos = brick_min_pos + d * voxelPos;
+  const float3 max_pos = min_pos + d * make3(1, 1, 1);
+  const float2 fNearFar = ray_box2(ray_pos, safe_inverse(ray_dir), min_pos, max_pos);
+  float values[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const uint32_t vId = (vx + ((i & 4) >> 2) + header.brick_pad) * v_size * v_size +
+                         (vy + ((i & 2) >> 1) + header.brick_pad) * v_size + (vz + (i & 1) + header.brick_pad);
+    rec.idx[i] = s.sbs_data[node.data_offset + vId];
+    values[i] = s.sbs_data_f[rec.idx[i]];
+  }
+  const float3 start_pos = ray_pos + fNearFar.x * ray_dir;
+  rec.start_q = (start_pos - min_pos) * scale;
+  const float qFar = (fNearFar.y - fNearFar.x) * scale;
+  local_surface_intersection<false, false>(s, type, ray_dir, instId, geomId, values, primId, d, 0.0f, qFar, fNearFar,
+                                           rec.start_q, miss, &rec.t_local);
+  return miss.t;
 }
 
 }  // namespace lrt

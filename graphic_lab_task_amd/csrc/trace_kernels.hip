@@ -76,7 +76,7 @@ __global__ void k_eye_rays(EyeRayParams prm, const float2* __restrict__ jitter, 
 hipError_t launch_trace(const SceneView& s, const TraceArgs& a, hipStream_t stream) {
   const uint32_t k = s.leaf_kinds & ~(LK_SBS_SMOOTH | LK_TRICUBIC);
   hipError_t e;
-  if (a.wide && s.wide && !a.counts && a.queue && a.pcount && a.n <= WIDE_MAX_RAYS)
+  if (a.wide && s.wide && k == s.leaf_kinds && !a.counts && a.queue && a.pcount && a.n <= WIDE_MAX_RAYS)
     e = launch_trace_wide(s, a, stream);
   else if (s.leaf_kinds & LK_TRICUBIC)
     e = k == LK_SBS ? launch_trace_sbs_tricubic(s, a, stream) : launch_trace_mixed_tricubic(s, a, stream);

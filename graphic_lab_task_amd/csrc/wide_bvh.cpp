@@ -35,19 +35,12 @@ bool contains(float3 mn, float3 mx, const BVHNode& c) {
          c.boxMax.z <= mx.z;
 }
 
-// A plane between the two boxes: every ray then passes them one after the other.
-bool separated(const BVHNode& a, const BVHNode& b) {
-  return a.boxMax.x <= b.boxMin.x || b.boxMax.x <= a.boxMin.x || a.boxMax.y <= b.boxMin.y || b.boxMax.y <= a.boxMin.y ||
-         a.boxMax.z <= b.boxMin.z || b.boxMax.z <= a.boxMin.z;
-}
-
 // One tree's collapse. Tree opens an inner word into its two binary children; Leaf gives the blocks of a
 // leaf word and writes them.
 template <class Tree, class Leaf>
 struct Collapse {
   const Tree& tree;
   const Leaf& leaf;
-  bool ordered;   // the two children of every binary node must be separated by a plane
 
   // Gathers up to six children of the binary node it.word: the inner child of largest surface area
   // is replaced by its own two children until six are held or none is left.
@@ -57,8 +50,6 @@ struct Collapse {
       BVHNode two[2];
       uint32_t source[2];
       tree.children(word, two, source);
-      if (ordered && two[0].leftOffset != LEAF_NORMAL && two[1].leftOffset != LEAF_NORMAL && !separated(two[0], two[1]))
-        return false;
       bool in_slot = slot < n;
       for (int k = 0; k < 2; ++k) {
         if (two[k].leftOffset == LEAF_NORMAL) continue;   // the empty sibling of a one-leaf tree
@@ -237,15 +228,41 @@ struct TriLeaf {
   }
 };
 
+// Where the sequential walk has an SDF leaf: its rank from the left, and the topmost pair above it whose two
+// sides overlap.
+struct LeafOrder {
+  uint32_t rank = 0, above = WIDE_NO_OVERLAP;
+};
+
+bool same_box(float3 amn, float3 amx, float3 bmn, float3 bmx) {
+  return amn.x == bmn.x && amn.y == bmn.y && amn.z == bmn.z && amx.x == bmx.x && amx.y == bmx.y && amx.z == bmx.z;
+}
+
 struct FrameLeafWriter {
   const FrameLeaf* leaves;   // of the geometry
+  const LeafOrder* order;
   uint32_t blocks(uint32_t) const { return 1; }
   bool write(uint32_t word, float3 mn, float3 mx, WideBlock* out) const {
-    const FrameLeaf& f = leaves[extract_start(word)];
+    FrameLeaf f = leaves[extract_start(word)];
+    const LeafOrder& at = order[extract_start(word)];
+    f.tex = at.rank | (at.above != WIDE_NO_OVERLAP ? WIDE_OVERLAP : 0u);   // untextured leaves have no use for it
     std::memcpy(out, &f, sizeof(f));
     // the leaf routine tests the record's box, the binary walk the node's: they must be the same
-    return f.boxMin.x == mn.x && f.boxMin.y == mn.y && f.boxMin.z == mn.z && f.boxMax.x == mx.x && f.boxMax.y == mx.y &&
-           f.boxMax.z == mx.z;
+    return same_box(f.boxMin, f.boxMax, mn, mx);
+  }
+};
+
+struct BrickLeaf {
+  const SdfSBSNode* nodes;   // of the geometry
+  size_t count;
+  const LeafOrder* order;
+  uint32_t blocks(uint32_t) const { return 1; }
+  bool write(uint32_t word, float3 mn, float3 mx, WideBlock* out) const {
+    const uint32_t prim = extract_start(word);
+    if (prim >= count) return false;   // the dummy box beside a single brick
+    const WideBrick b{mn, mx, prim, order[prim].rank, nodes[prim], order[prim].above, {}};
+    std::memcpy(out, &b, sizeof(b));
+    return true;
   }
 };
 
@@ -261,6 +278,55 @@ struct InstanceLeaf {
     return true;
   }
 };
+
+}  // namespace
+
+namespace {
+
+// Marks a BLAS's device pairs with what the order of its leaves needs (the BLAS walks do not read escape
+// indices): right.escapeIndex the rank of the right side's first leaf, counted from the left (a mesh
+// counts triangles: the rank is the index of the leaf's first one), and left.escapeIndex 1 where no plane
+// separates the two sides. `order` takes a box leaf's rank and the topmost such pair above it. False where
+// a mesh's triangle indices do not grow from left to right.
+bool mark_order(BVHNodePair* pairs, uint32_t n, bool mesh, std::vector<LeafOrder>& order) {
+  std::vector<uint32_t> count(n, 0u), first(n, 0u), above(n, WIDE_NO_OVERLAP);
+  auto leaves = [&](const BVHNode& c) -> uint32_t {
+    if (c.leftOffset == LEAF_NORMAL) return 0u;   // the empty sibling of a one-leaf tree
+    if (c.leftOffset & LEAF_BIT) return mesh ? extract_count(c.leftOffset) : 1u;
+    return count[c.leftOffset];
+  };
+  // children are stored after their parent
+  for (uint32_t p = n; p-- > 0;) {
+    for (const BVHNode* c : {&pairs[p].left, &pairs[p].right})
+      if (!(c->leftOffset & LEAF_BIT) && (c->leftOffset <= p || c->leftOffset >= n)) return false;
+    count[p] = leaves(pairs[p].left) + leaves(pairs[p].right);
+  }
+  order.assign(mesh || n == 0 ? 0u : count[0], LeafOrder{});
+  for (uint32_t p = 0; p < n; ++p) {
+    BVHNode &l = pairs[p].left, &r = pairs[p].right;
+    const bool apart = l.leftOffset == LEAF_NORMAL || r.leftOffset == LEAF_NORMAL || l.boxMax.x <= r.boxMin.x ||
+                       r.boxMax.x <= l.boxMin.x || l.boxMax.y <= r.boxMin.y || r.boxMax.y <= l.boxMin.y ||
+                       l.boxMax.z <= r.boxMin.z || r.boxMax.z <= l.boxMin.z;
+    const uint32_t overlap = above[p] != WIDE_NO_OVERLAP || apart ? above[p] : p;
+    uint32_t at = first[p];
+    for (BVHNode* c : {&l, &r}) {
+      if (c->leftOffset == LEAF_NORMAL) continue;
+      if (!(c->leftOffset & LEAF_BIT)) {
+        first[c->leftOffset] = at;
+        above[c->leftOffset] = overlap;
+      } else if (mesh) {
+        if (extract_start(c->leftOffset) != at) return false;
+      } else {
+        if (extract_start(c->leftOffset) >= order.size()) return false;
+        order[extract_start(c->leftOffset)] = LeafOrder{at, overlap};
+      }
+      at += leaves(*c);
+    }
+    r.escapeIndex = first[p] + leaves(l);
+    l.escapeIndex = apart ? 0u : 1u;
+  }
+  return true;
+}
 
 }  // namespace
 
@@ -295,7 +361,7 @@ bool Scene::build_wide_instances(uint32_t* levels) {
     wideRoot = wide_ref(0, 2, true);
   } else {
     const TlasTree tree{tlas.data()};
-    if (!Collapse<TlasTree, InstanceLeaf>{tree, leaf, false}.run(top, levels, &wideSources)) return false;
+    if (!Collapse<TlasTree, InstanceLeaf>{tree, leaf}.run(top, levels, &wideSources)) return false;
     wideRoot = wide_ref(0, 1, false);
   }
   if (top.size() > room) return false;
@@ -303,16 +369,16 @@ bool Scene::build_wide_instances(uint32_t* levels) {
   return true;
 }
 
-// Builds wideBlocks from the device layout (devNodes, triSoup, frameLeaves) and the TLAS, or leaves it
-// empty where the wide walk does not apply: it takes scenes of triangle meshes only, and scenes of one
-// instance of a frame octree or sparse voxel set whose binary tree is ordered (trace_wide.hip).
+// Builds wideBlocks from the device layout (devNodes, triSoup, frameLeaves, sbsNodes) and the TLAS, or
+// leaves it empty where the wide walk does not apply: it takes scenes of triangle meshes only, and scenes
+// of one instance of a frame octree, sparse voxel set or sparse brick set.
 void Scene::build_wide() {
   wideBlocks.clear();
   wideSources.clear();
   wideRoots.assign(geomData.size(), 0u);
   const uint32_t kinds = leaf_kinds();
-  const bool frame = kinds == LK_FRAME && instances.size() == 1;
-  if ((kinds != LK_TRI && !frame) || instances.empty()) return;
+  const bool sdf = (kinds == LK_FRAME || kinds == LK_SBS) && instances.size() == 1;
+  if ((kinds != LK_TRI && !sdf) || instances.empty()) return;
   std::vector<uint8_t> used(geomData.size(), 0);
   for (const InstanceData& i : instances) used[i.geomId] = 1;
   std::vector<Blocks> geom(geomData.size());
@@ -322,16 +388,22 @@ void Scene::build_wide() {
     if (!used[g]) continue;
     const size_t first = geomData[g].bvhOffset, end = g + 1 < geomData.size() ? geomData[g + 1].bvhOffset : devNodes.size();
     if (first >= end) return;   // an empty mesh
-    if (geomTags[g] == TAG_TRIANGLE && !devOrdered[g]) return;
+    std::vector<LeafOrder> order;
+    if (!mark_order(devNodes.data() + first, uint32_t(end - first), kinds == LK_TRI, order)) return;
     const PairTree tree{devNodes.data() + first};
     uint32_t levels = 0;
     bool ok;
-    if (frame) {
-      const FrameLeafWriter leaf{frameLeaves.data() + geomData[g].offset.y};
-      ok = Collapse<PairTree, FrameLeafWriter>{tree, leaf, true}.run(geom[g], &levels, nullptr);
+    if (kinds == LK_FRAME) {
+      const FrameLeafWriter leaf{frameLeaves.data() + geomData[g].offset.y, order.data()};
+      ok = Collapse<PairTree, FrameLeafWriter>{tree, leaf}.run(geom[g], &levels, nullptr);
+    } else if (kinds == LK_SBS) {
+      const uint32_t set = geomData[g].offset.x;
+      const size_t last = set + 1 < sbsRoots.size() ? sbsRoots[set + 1] : sbsNodes.size();
+      const BrickLeaf leaf{sbsNodes.data() + sbsRoots[set], last - sbsRoots[set], order.data()};
+      ok = Collapse<PairTree, BrickLeaf>{tree, leaf}.run(geom[g], &levels, nullptr);
     } else {
       const TriLeaf leaf{triSoup.data() + geomData[g].offset.x};
-      ok = Collapse<PairTree, TriLeaf>{tree, leaf, false}.run(geom[g], &levels, nullptr);
+      ok = Collapse<PairTree, TriLeaf>{tree, leaf}.run(geom[g], &levels, nullptr);
     }
     wideRoots[g] = wide_ref(uint32_t(total), 1, false);
     total += geom[g].size();

@@ -47,6 +47,26 @@ struct alignas(16) WideTri {
 };
 static_assert(sizeof(WideTri) == 64, "one block");
 
+// SDF leaves carry their rank among the binary tree's leaves from left to right, and whether two sides that
+// no plane separates lie above them: only among the leaves below one such pair can the sequential walk's
+// order differ from the order of box entries along a ray. A frame-octree leaf has both in its FrameLeaf's
+// `tex` (the bit WIDE_OVERLAP), a brick names the topmost such pair (WIDE_NO_OVERLAP: none).
+constexpr uint32_t WIDE_OVERLAP = 0x80000000u;
+constexpr uint32_t WIDE_NO_OVERLAP = 0xFFFFFFFFu;
+
+// One brick of a sparse brick set: its binary leaf's box, its index in the set, its rank, its node record
+// and the pair.
+struct alignas(16) WideBrick {
+  float3     boxMin;
+  float3     boxMax;
+  uint32_t   prim;
+  uint32_t   rank;
+  SdfSBSNode node;
+  uint32_t   overlap;
+  uint32_t   pad[3];
+};
+static_assert(sizeof(WideBrick) == 64, "one block");
+
 // One instance: columns of the inverse transform (rows 0-2), its box in world space, the root of its
 // geometry and the ids a hit reports.
 struct alignas(16) WideInstance {

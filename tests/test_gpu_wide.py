@@ -1,4 +1,4 @@
-"""The wide walk (trace_wide.hip, the default on triangle scenes and single ordered frame octrees)
+"""The wide walk (trace_wide.hip, the default on triangle scenes, single frame octrees and brick sets)
 against the binary walk, record for record: tile and batch edges, instances, first-hit and any-hit rays,
 rays and scenes that fall back to the sequential walk, a tree deeper than the LDS stack, the refitted
 instance level, graph replay and the allocation-free entry point."""
@@ -245,3 +245,36 @@ def test_graph_replay_and_noalloc(lrt, torch_dev):
         assert raw_equal(hits.cpu().numpy().view(lrt.HIT_DTYPE).reshape(-1), want)
         pos2, dirs2 = random_rays(torch, 1000 + k, k)
         b.check(torch, pos2, dirs2)
+
+
+def brick_scene(g, depth, bs, kind, pad=0, m=None, seed=2):
+    rng = np.random.default_rng(seed)
+    sph = np.concatenate([rng.uniform(-0.8, 0.8, (64, 3)), rng.uniform(0.05, 0.2, (64, 1))], 1).astype(np.float32)
+
+    def make():
+        s = g.SceneRT()
+        if kind == "indexed":
+            h, nodes, vals, vf, _ = g.sdf_spheres_sbs_indexed(sph, depth, bs, 3)
+            gid = s.AddGeom_SdfSBS(h, nodes, vals, vf)
+        else:
+            h = np.zeros((), g.SBS_HEADER_DTYPE)
+            h["brick_size"], h["brick_pad"], h["bytes_per_value"] = bs, pad, kind
+            h["aux_data"] = g.SDF_SBS_NODE_LAYOUT_DX_RGB8
+            nodes, vals = g.sdf_spheres_sbs(sph, depth, h, 0, 5)
+            gid = s.AddGeom_SdfSBS(h, nodes, vals)
+        s.AddInstance(gid, m)
+        s.CommitScene()
+        return s
+    return make
+
+
+# depth 5 holds bricks of two sizes, whose binary tree has overlapping siblings
+@pytest.mark.parametrize("depth,bs,kind", [(2, 1, 1), (3, 4, 2), (5, 2, 4), (5, 8, "indexed"), (4, 3, "indexed")])
+def test_bricks(lrt, torch_dev, depth, bs, kind):
+    for m in (None, mats(1, 3, 0.3)[0]):
+        b = Both(lrt, brick_scene(lrt, depth, bs, kind, pad=1 if kind == 2 else 0, m=m))
+        pos, dirs = random_rays(torch_dev, 150001, depth, extent=2.0)
+        dirs[::11, 0] = 0.0
+        dirs[::5, 3] = 0.6
+        hits = b.check(torch_dev, pos, dirs)
+        assert (hits["primId"] != lrt.MISS).sum() > 0

@@ -149,6 +149,48 @@ def test_frame_octree():
     assert sorted(got) == sorted(want["leftOffset"].tolist())
 
 
+@pytest.mark.parametrize("depth", [1, 5])
+def test_bricks(depth):
+    h = np.zeros((), g.SBS_HEADER_DTYPE)
+    h["brick_size"], h["bytes_per_value"], h["aux_data"] = 2, 2, g.SDF_SBS_NODE_LAYOUT_DX
+    nodes, vals = g.sdf_spheres_sbs(spheres(), depth, h)
+    s = g.SceneRT()
+    s.AddInstance(s.AddGeom_SdfSBS(h, nodes, vals))
+    blocks, _ = tree(commit(s))
+    got = []
+
+    def leaf(at, count):
+        w, f = blocks[at], blocks[at].view(np.float32)
+        got.append((int(w[6]), int(w[7]), int(w[12])))
+        assert count == 1 and np.array_equal(w[8:11], [nodes[got[-1][0]][k] for k in ("pos_xy", "pos_z_lod_size", "data_offset")])
+        return f[:3].astype(np.float64), f[3:6].astype(np.float64)
+
+    walk(blocks, int(blocks[0][15]), leaf)
+    # ranks count the binary tree's leaves from left to right
+    # and name the topmost pair above them whose sides no plane separates (0xFFFFFFFF: none), in the device
+    # order of the pairs, where it is the same for the same leaves
+    pairs, order, todo = s.get_array("nodes"), [], [(0, None)]
+    while todo:
+        t, over = todo.pop()
+        if t >> 31:
+            order.append((t & 0x0FFFFFFF, over))
+            continue
+        a, b = pairs[t]["left"], pairs[t]["right"]
+        if over is None and not ((a["boxMax"] <= b["boxMin"]) | (b["boxMax"] <= a["boxMin"])).any():
+            over = t
+        todo += [(int(b["leftOffset"]), over), (int(a["leftOffset"]), over)]
+    assert sorted(p for p, _, _ in got) == list(range(nodes.size))
+    names = {}
+    for p, r, over in got:
+        assert order[r][0] == p and (over == 0xFFFFFFFF) == (order[r][1] is None)
+        assert names.setdefault(over, order[r][1]) == order[r][1]
+    assert len(set(names.values())) == len(names) and (len(names) > 1) == (depth == 5)
+    # a single brick has a dummy box beside it, which is no brick
+    one = g.SceneRT()
+    one.AddInstance(one.AddGeom_SdfSBS(h, nodes[:1], vals))
+    assert tree(commit(one))[0].size == 0
+
+
 def test_scenes_outside_the_terms_have_no_tree():
     v, f = g.gen_geodesic(3, 0.05, 4.0, 3)
     nodes = g.sdf_spheres_frame_octree(spheres(), 4)
