@@ -24,9 +24,10 @@ struct lrt_sbs_batch {
   // destruction of the scene invalidates the device pointers the plan holds)
   std::vector<std::weak_ptr<uint64_t>> scene_gen;
   std::vector<uint64_t> gen_at_create;
-  lrt::DevBuf d_items, d_begins, d_masks, d_spill, d_counter;
+  lrt::DevBuf d_items, d_begins, d_masks, d_spill, d_counter, d_queue;
   lrt::SbsBatchLaunch L{};
   uint32_t resident[6] = {};   // resident blocks per variant: (LDS stack 8 << v/2, record v%2)
+  uint32_t resident_wide = 0;  // of the wide form, 0 unless every item's scene has a wide tree
 };
 
 namespace {
@@ -198,10 +199,12 @@ lrt_status sbs_diff_common(lrt_scene* s, uint32_t geom_id, const float* params, 
   uint32_t* pcount = nullptr;
   hipError_t e = s->s.work_for(w, stream, size_t(n), &a.spill, &q, &pcount);
   if (e != hipSuccess) return hip_fail(e, "work buffer");
+  a.queue = q;
   // occupancy masks from the caller's parameters (they differ from the committed values)
   lrt::SceneView v = s->s.make_view();
   v.sbs_data_f = params;
   v.sbs_mask = nullptr;
+  if (!s->s.wide) v.wide = nullptr;
   uint32_t* mask = nullptr;
   e = s->s.mask_for(w, stream, &mask);
   if (e != hipSuccess) return hip_fail(e, "mask buffer");
@@ -843,6 +846,7 @@ lrt_status lrt_sbs_batch_create(const lrt_sbs_batch_item* items, uint32_t n_item
       it.view.sbs_data_f = in.params;
       it.view.cache_pairs = 0;
       it.view.cache_geom = 0xFFFFFFFFu;
+      if (!sc.wide) it.view.wide = nullptr;
       it.args.pos = reinterpret_cast<const lrt::float4*>(in.pos_near);
       it.args.dir = reinterpret_cast<const lrt::float4*>(in.dir_far);
       it.args.n = uint32_t(in.n_rays);
@@ -890,6 +894,19 @@ lrt_status lrt_sbs_batch_create(const lrt_sbs_batch_item* items, uint32_t n_item
       b->resident[v] = uint32_t(std::max(1, cus * std::max(1, per_cu)));
       max_grid = std::max(max_grid, b->resident[v]);
     }
+    const uint64_t slots = uint64_t(chunk_begin.back()) * lrt::SBS_BATCH_CHUNK;
+    bool wide = n_items > 0 && slots > 0 && slots <= 0xFFFFFFFFull;
+    for (uint32_t k = 0; k < n_items; ++k) wide = wide && b->items[k].view.wide != nullptr;
+    if (wide) {
+      int per_cu = 0;
+      if ((e = lrt::sbs_batch_wide_blocks_per_cu(&per_cu)) != hipSuccess) return hip_fail(e, "occupancy");
+      b->resident_wide = uint32_t(std::max(1, cus * std::max(1, per_cu)));
+      max_grid = std::max(max_grid, b->resident_wide);
+      if ((e = b->d_queue.reserve(256 + slots * 4)) != hipSuccess) return hip_fail(e, "batch queue");
+      const lrt::TailQueue q{0u, 0u, reinterpret_cast<uint32_t*>(static_cast<char*>(b->d_queue.ptr()) + 256)};
+      if ((e = hipMemcpy(b->d_queue.ptr(), &q, sizeof(q), hipMemcpyHostToDevice)) != hipSuccess)
+        return hip_fail(e, "batch queue");
+    }
     const uint32_t grid = b->resident[2];   // LDS stack 16, hit brick marched again
     const size_t n1 = size_t(n_items) + 1;
     if ((e = b->d_items.upload(b->items.data(), b->items.size() * sizeof(lrt::SbsBatchItem))) != hipSuccess)
@@ -910,6 +927,9 @@ lrt_status lrt_sbs_batch_create(const lrt_sbs_batch_item* items, uint32_t n_item
     L.spill = static_cast<uint32_t*>(b->d_spill.ptr());
     L.grid = grid;
     L.lds_stack = 16;
+    L.wide = wide ? 1u : 0u;
+    L.wide_grid = b->resident_wide;
+    L.queue = static_cast<lrt::TailQueue*>(b->d_queue.ptr());
     L.record = 0;
     auto blocks = [](uint64_t work, uint64_t cap) { return uint32_t(std::min<uint64_t>(cap, (work + 255) / 256)); };
     L.zero_blocks = blocks(max_zero4, 1024);
@@ -952,6 +972,20 @@ lrt_status lrt_sbs_batch_autotune(lrt_sbs_batch* b, void* stream, lrt_sbs_batch_
     lrt::SbsBatchLaunch best = start;
     float best_ms = 1e30f;
     uint32_t tried = 0;
+    auto time_run = [&](const lrt::SbsBatchLaunch& c, float* ms) -> hipError_t {
+      hipError_t te = lrt::launch_sbs_batch(c, hs);   // warm-up
+      *ms = 1e30f;
+      for (int r = 0; r < 3 && te == hipSuccess; ++r) {
+        float t = 0.0f;
+        if ((te = hipEventRecord(e0, hs)) != hipSuccess) break;
+        if ((te = lrt::launch_sbs_batch(c, hs)) != hipSuccess) break;
+        if ((te = hipEventRecord(e1, hs)) != hipSuccess) break;
+        if ((te = hipEventSynchronize(e1)) != hipSuccess) break;
+        if ((te = hipEventElapsedTime(&t, e0, e1)) != hipSuccess) break;
+        *ms = std::min(*ms, t);
+      }
+      return te;
+    };
     // LDS stack 8 / 16 / 32 entries x voxel record off / on x 1/2, 3/4 or all of the resident blocks
     for (int v = 0; v < 6 && e == hipSuccess; ++v) {
       for (int quarters : {2, 3, 4}) {
@@ -959,23 +993,26 @@ lrt_status lrt_sbs_batch_autotune(lrt_sbs_batch* b, void* stream, lrt_sbs_batch_
         c.lds_stack = 8 << (v / 2);
         c.record = v % 2;
         c.grid = std::max<uint32_t>(1u, b->resident[v] * uint32_t(quarters) / 4u);
+        c.wide = 0;
         float ms = 1e30f;
-        if ((e = lrt::launch_sbs_batch(c, hs)) != hipSuccess) break;   // warm-up
-        for (int r = 0; r < 3 && e == hipSuccess; ++r) {
-          float t = 0.0f;
-          if ((e = hipEventRecord(e0, hs)) != hipSuccess) break;
-          if ((e = lrt::launch_sbs_batch(c, hs)) != hipSuccess) break;
-          if ((e = hipEventRecord(e1, hs)) != hipSuccess) break;
-          if ((e = hipEventSynchronize(e1)) != hipSuccess) break;
-          if ((e = hipEventElapsedTime(&t, e0, e1)) != hipSuccess) break;
-          ms = std::min(ms, t);
-        }
+        e = time_run(c, &ms);
         if (e != hipSuccess) break;
         ++tried;
         if (ms < best_ms) {
           best_ms = ms;
           best = c;
         }
+      }
+    }
+    // the wide form is kept where it is faster than the best of these, which is reported all the same
+    if (e == hipSuccess && b->resident_wide) {
+      lrt::SbsBatchLaunch c = best;
+      c.wide = 1;
+      float ms = 1e30f;
+      e = time_run(c, &ms);
+      if (e == hipSuccess && ms < best_ms) {
+        best_ms = ms;
+        best = c;
       }
     }
     if (e0) (void)hipEventDestroy(e0);
@@ -1007,6 +1044,7 @@ lrt_status lrt_sbs_batch_configure(lrt_sbs_batch* b, int lds_stack, int record, 
     b->L.lds_stack = lds_stack;
     b->L.record = record;
     b->L.grid = grid;
+    b->L.wide = 0;
     return LRT_OK;
   });
 }

@@ -9,8 +9,10 @@
 // where q is the hit point in voxel coordinates, w the trilinear weights, f the trilinear
 // distance and G = dL/dC (given, or 2(C - T) for the fused L2 loss): the hit point moves along
 // the ray when a corner distance changes (implicit function theorem on f(q(t)) = 0).
+#include <algorithm>
+
 #include "kernels.h"
-#include "traverse.h"
+#include "wide_walk.h"
 
 namespace lrt {
 
@@ -48,8 +50,8 @@ __device__ bool recompute_hit_voxel(const SceneView& s, uint32_t diff_geom, floa
 // MODE 0 forward, 1 backward with dL/dC, 2 backward of the L2 loss against a target, 3 both the
 // forward colour and the L2 backward. Returns the ray's loss term |C - T|^2 (modes 2, 3).
 // `rec`: the voxel record the traversal's own brick march left (t_local NaN if it recorded none);
-// without one the hit brick is marched once more.
-template <int MODE>
+// without one the hit brick is marched once more (REMARCH).
+template <int MODE, bool REMARCH = true>
 __device__ __forceinline__ float diff_ray(const SceneView& s, const SbsDiffArgs& a, uint32_t i, const CRT_Hit& h,
                                           SbsVoxelRec& rec) {
   const float4 p = a.pos[i];
@@ -57,7 +59,7 @@ __device__ __forceinline__ float diff_ray(const SceneView& s, const SbsDiffArgs&
   float3 dir_l = make3(0, 0, 0);
   bool hit = false;
   if (h.geomId != 0xFFFFFFFFu && (h.geomId & GEOM_ID_MASK) == a.geom_id) {
-    if (rec.t_local == rec.t_local) {   // recorded by the traversal
+    if (!REMARCH || rec.t_local == rec.t_local) {   // recorded by the traversal
       float m[16];
       load_mat(s.instances[h.instId].transformInv, m);
       dir_l = matmul3x3(m, xyz(d));
@@ -155,6 +157,126 @@ __global__ __launch_bounds__(BLOCK) void k_sbs_diff(SceneView s, SbsDiffArgs a) 
     loss = wave_sum(loss);
     if (__lane_id() == 0) atomicAdd(a.loss, loss);
   }
+}
+
+// The wide walk's form (scenes of one brick-set instance with a wide tree, traverse and adjoint in one
+// wave): the wave's 64 rays are walked by all its lanes, the hit's voxel index alone being kept, then the
+// voxel is solved once more for the record and each lane does the rest for its own ray. `first` (LDS, 3
+// words a lane) takes the walk's result of each ray. A ray the wide walk leaves to the sequential one
+// (zero or non-finite components) is queued as `code` for a second kernel (walked here, its code took the
+// kernel from 4 waves a SIMD to 3: the batch of 12 x 4 x 128 x 128 rays 0.88 ms instead of 0.66).
+// What bounds it: vector instructions of solves and node steps at a sixth and half of the lanes, and the
+// waves with the most grazing rays. Whole calls, masks included, against one ray a lane of the binary walk:
+// 8 x 256 x 256 rays into 256^3 voxels 0.79 ms against 0.86, 3 x 201 x 201 rays into 128^3, forward and
+// backward apart, 0.68 against 0.87, the batch above 0.68 against 0.90.
+template <int MODE>
+__device__ __forceinline__ float diff_wave(const SceneView& s, const SbsDiffArgs& a, bool mine, uint32_t ray,
+                                           wide_lds* lds, wide_lds* result, uint32_t* spill,
+                                           TailQueue* queue, uint32_t code) {
+  constexpr int BLOCK = WIDE_BLOCK;
+  const uint32_t lane = threadIdx.x;
+  auto fetch = [&](bool, uint32_t, uint32_t, uint32_t& i, bool& exhausted) -> bool {
+    exhausted = true;
+    i = ray;
+    return mine;
+  };
+  auto done = [&](uint32_t, CRT_Hit& hit, uint32_t voxel, bool again) {
+    result[lane] = __float_as_uint(hit.t);
+    result[BLOCK + lane] = hit.primId;
+    result[2 * BLOCK + lane] = again ? 0xFFFFFFFFu : voxel;
+  };
+  wide_walk<WIDE_BRICK, false, true>(s, a.pos, a.dir, lds, nullptr, spill, true, fetch, done);
+  __syncthreads();
+  if (!mine) return 0.0f;
+  const uint32_t i = ray;
+  const float4 p = a.pos[i], d = a.dir[i];
+  CRT_Hit h = miss_hit(fabs_ref(d.w));
+  SbsVoxelRec rec;
+  rec.t_local = __int_as_float(0x7fc00000);
+  const float t = __uint_as_float(result[lane]);
+  const uint32_t prim = result[BLOCK + lane], voxel = result[2 * BLOCK + lane];
+  if (voxel == 0xFFFFFFFFu) {
+    queue->list[atomicAdd(&queue->count, 1u)] = code;
+    return 0.0f;
+  }
+  if (prim != 0xFFFFFFFFu) {
+    const WideInstance* w = reinterpret_cast<const WideInstance*>(s.wide);
+    const GeomRef g = geom_ref(s, w->geom_id);
+    float3 lo, ld;
+    wide_local_ray(w, xyz(p), xyz(d), lo, ld);
+    const float again = sbs_voxel_rec(s, g.type, g.offset.x, lo, ld, w->inst_id, w->geom_id, prim, voxel, h, rec);
+    if (__float_as_uint(again) == __float_as_uint(t)) {
+      h.t = t;
+      h.primId = prim;
+      h.instId = w->inst_id;
+      h.geomId = w->geom_id | (g.type << SH_TYPE);
+    } else if (a.counters) {
+      atomicAdd(a.counters, 1u);
+    }
+  }
+  return diff_ray<MODE, false>(s, a, i, h, rec);
+}
+
+template <int MODE>
+__global__ __launch_bounds__(WIDE_BLOCK, 4) void k_sbs_diff_wide(SceneView s, SbsDiffArgs a) {
+  __shared__ uint32_t lds[2 * WIDE_LDS_STACK * WIDE_BLOCK];
+  __shared__ uint32_t result[3 * WIDE_BLOCK];
+  // groups of 8 neighbours from distant parts of the batch, as the trace kernel
+  const uint32_t lane = threadIdx.x, i = (lane / 8u * gridDim.x + blockIdx.x) * 8u + lane % 8u;
+  float loss = diff_wave<MODE>(s, a, i < a.n, i, (wide_lds*)(lds), (wide_lds*)(result),
+                               a.spill + size_t(blockIdx.x * WIDE_BLOCK + lane) * (STACK_SIZE - 16), a.queue, i);
+  if (MODE >= 2 && a.loss) {
+    loss = wave_sum(loss);
+    if (lane == 0) atomicAdd(a.loss, loss);
+  }
+}
+
+// One ray of the sequential walk and its adjoint.
+template <int MODE>
+__device__ __forceinline__ float diff_sequential(const SceneView& s, const SbsDiffArgs& a, uint32_t i, lds_u32* lds,
+                                                 uint32_t* spill) {
+  LaneStack<16, WIDE_BLOCK> st;
+  st.col = lds + threadIdx.x;
+  st.spill = spill;
+  uint32_t overflow = 0;
+  RayCounts cnt{};
+  bool aborted = false;
+  SbsVoxelRec rec;
+  rec.t_local = __int_as_float(0x7fc00000);
+  const CRT_Hit h = ray_query_nearest<LK_SBS, 16, WIDE_BLOCK, false, false>(s, a.pos[i], a.dir[i], st, overflow, cnt, nullptr,
+                                                                            0u, aborted, nullptr, nullptr, &rec);
+  return diff_ray<MODE>(s, a, i, h, rec);
+}
+
+// The waves of a kernel over a queue: wave w takes entries [64 w, 64 w + 64) and so on in steps of the grid;
+// waves without entries leave without touching it, the others count themselves out and the last clears it.
+template <class F>
+__device__ __forceinline__ void for_queued(TailQueue* queue, F&& f) {
+  const uint32_t total = __atomic_load_n(&queue->count, __ATOMIC_RELAXED);
+  const uint32_t waves = min(gridDim.x, (total + WIDE_BLOCK - 1) / WIDE_BLOCK);
+  if (blockIdx.x >= waves) return;
+  for (uint32_t first = blockIdx.x * WIDE_BLOCK; first < total; first += gridDim.x * WIDE_BLOCK)
+    f(first + threadIdx.x < total, first + threadIdx.x);
+  __syncthreads();
+  if (threadIdx.x == 0 && atomicAdd(&queue->next, 1u) == waves - 1) {
+    queue->count = 0;
+    queue->next = 0;
+  }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(WIDE_BLOCK) void k_sbs_diff_queued(SceneView s, SbsDiffArgs a) {
+  __shared__ uint32_t lds[16 * WIDE_BLOCK];
+  for_queued(a.queue, [&](bool mine, uint32_t k) {
+    float loss = 0.0f;
+    if (mine)
+      loss = diff_sequential<MODE>(s, a, a.queue->list[k], (lds_u32*)(lds),
+                                   a.spill + size_t(blockIdx.x * WIDE_BLOCK + threadIdx.x) * (STACK_SIZE - 16));
+    if (MODE >= 2 && a.loss) {
+      loss = wave_sum(loss);
+      if (threadIdx.x == 0) atomicAdd(a.loss, loss);
+    }
+  });
 }
 
 // ---- batched launch ----
@@ -275,13 +397,66 @@ __global__ __launch_bounds__(BLOCK) void k_sbs_batch(SbsBatchLaunch L) {
   }
 }
 
+// The wide form: one-wave blocks again, every item with a wide tree. A wave's chunks are dealt out for
+// three quarters of the batch, the rest comes from the counter (an atomic on one address takes about 16
+// ns, and with one for each of the 12,288 chunks of 12 x 4 x 128 x 128 rays that was 0.2 ms).
+__global__ __launch_bounds__(WIDE_BLOCK, 4) void k_sbs_batch_wide(SbsBatchLaunch L) {
+  __shared__ uint32_t lds[2 * WIDE_LDS_STACK * WIDE_BLOCK];
+  __shared__ uint32_t result[3 * WIDE_BLOCK];
+  const uint32_t lane = threadIdx.x;
+  const uint32_t turns = uint32_t(uint64_t(L.total_chunks) * 3u / 4u / gridDim.x);
+  for (uint32_t turn = 0;; ++turn) {
+    uint32_t chunk = turn * gridDim.x + blockIdx.x;
+    if (turn >= turns) {
+      uint32_t got = 0;
+      if (lane == 0) got = atomicAdd(L.counter, 1u);
+      chunk = turns * gridDim.x + __builtin_amdgcn_readfirstlane(got);
+    }
+    if (chunk >= L.total_chunks) break;   // the same for the whole wave
+    const uint32_t it = __builtin_amdgcn_readfirstlane(find_item(L.chunk_begin, L.n_items, chunk));
+    const SbsBatchItem& item = L.items[it];
+    const uint32_t i = (chunk - L.chunk_begin[it]) * SBS_BATCH_CHUNK + lane;
+    float loss = diff_wave<3>(item.view, item.args, i < item.args.n, i, (wide_lds*)(lds), (wide_lds*)(result),
+                              L.spill + size_t(blockIdx.x * WIDE_BLOCK + lane) * (STACK_SIZE - 8), L.queue,
+                              chunk * SBS_BATCH_CHUNK + lane);
+    loss = wave_sum(loss);
+    if (lane == 0 && item.args.loss) atomicAdd(item.args.loss, loss);
+    __syncthreads();
+  }
+}
+
+__global__ __launch_bounds__(WIDE_BLOCK) void k_sbs_batch_queued(SbsBatchLaunch L) {
+  __shared__ uint32_t lds[16 * WIDE_BLOCK];
+  for_queued(L.queue, [&](bool mine, uint32_t k) {
+    if (!mine) return;
+    const uint32_t code = L.queue->list[k];   // chunk and ray
+    const uint32_t it = find_item(L.chunk_begin, L.n_items, code / SBS_BATCH_CHUNK);
+    const SbsBatchItem& item = L.items[it];
+    const uint32_t i = code - L.chunk_begin[it] * SBS_BATCH_CHUNK;
+    const float loss = diff_sequential<3>(item.view, item.args, i, (lds_u32*)(lds),
+                                          L.spill + size_t(blockIdx.x * WIDE_BLOCK + threadIdx.x) * (STACK_SIZE - 8));
+    if (item.args.loss) atomicAdd(item.args.loss, loss);
+  });
+}
+
 template <int S, bool REC>
 const void* batch_kernel() {
   return reinterpret_cast<const void*>(k_sbs_batch<S, SBS_BATCH_BLOCK, REC>);
 }
 
+// Grid of the kernels over a queue: 8 blocks a CU of 256 (their 160 registers allow 12)
+constexpr uint32_t QUEUED_BLOCKS = 2048;
+
 template <int MODE>
 hipError_t launch_mode(const SceneView& s, const SbsDiffArgs& a, hipStream_t stream) {
+  if (s.wide) {
+    hipLaunchKernelGGL((k_sbs_diff_wide<MODE>), dim3((a.n + WIDE_BLOCK - 1) / WIDE_BLOCK), dim3(WIDE_BLOCK), 0, stream, s,
+                       a);
+    // mostly nothing is queued; as many blocks as fit at once take it if everything is
+    hipLaunchKernelGGL((k_sbs_diff_queued<MODE>), dim3(std::min((a.n + WIDE_BLOCK - 1) / WIDE_BLOCK, QUEUED_BLOCKS)),
+                       dim3(WIDE_BLOCK), 0, stream, s, a);
+    return hipGetLastError();
+  }
   constexpr int S = 16, BLOCK = 128;
   const uint32_t grid = (a.n + BLOCK - 1) / BLOCK;
   hipLaunchKernelGGL((k_sbs_diff<MODE, S, BLOCK>), dim3(grid), dim3(BLOCK), 0, stream, s, a);
@@ -304,6 +479,10 @@ hipError_t sbs_batch_blocks_per_cu(int lds_stack, int record, int* blocks) {
   return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks, k, SBS_BATCH_BLOCK, 0);
 }
 
+hipError_t sbs_batch_wide_blocks_per_cu(int* blocks) {
+  return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks, reinterpret_cast<const void*>(k_sbs_batch_wide), WIDE_BLOCK, 0);
+}
+
 hipError_t launch_sbs_batch(const SbsBatchLaunch& L, hipStream_t stream) {
   if (L.n_items == 0) return hipSuccess;
   // x extents sized for the largest item (smaller items leave blocks idle)
@@ -313,6 +492,13 @@ hipError_t launch_sbs_batch(const SbsBatchLaunch& L, hipStream_t stream) {
   } else if (L.total_bricks) {   // very large bricks: one thread per voxel bit, then the summary words
     hipLaunchKernelGGL(k_batch_mask_words, dim3(L.mask_blocks, L.n_items), dim3(256), 0, stream, L);
     hipLaunchKernelGGL(k_batch_mask_summary, dim3(L.summary_blocks, L.n_items), dim3(256), 0, stream, L);
+  }
+  if (L.wide) {
+    hipLaunchKernelGGL(k_sbs_batch_wide, dim3(std::min(L.wide_grid, std::max(1u, L.total_chunks))), dim3(WIDE_BLOCK), 0,
+                       stream, L);
+    hipLaunchKernelGGL(k_sbs_batch_queued, dim3(std::min(std::min(L.wide_grid, L.total_chunks), QUEUED_BLOCKS)),
+                       dim3(WIDE_BLOCK), 0, stream, L);
+    return hipGetLastError();
   }
   const dim3 g(L.grid), b(SBS_BATCH_BLOCK);
   switch (L.lds_stack * 2 + (L.record ? 1 : 0)) {

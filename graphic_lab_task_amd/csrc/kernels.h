@@ -66,7 +66,8 @@ struct SbsDiffArgs {
   float*        grad;         // backward: dL/dparams, accumulated (scene-sized)
   float*        loss;         // fused L2: sum over rays of |C - T|^2, accumulated (nullable)
   uint32_t*     counters;     // nullable: [0] += rays whose recomputed hit differed from the walk
-  uint32_t*     spill;        // n * (STACK_SIZE - 16) words
+  uint32_t*     spill;        // (n + 63) * (STACK_SIZE - 16) words
+  TailQueue*    queue;        // rays the wide form leaves to the sequential walk (empty between calls)
   uint32_t      xcd_remap;
 };
 
@@ -112,6 +113,9 @@ struct SbsBatchLaunch {
   uint32_t* spill;               // grid * BLOCK * (STACK_SIZE - 8) words
   uint32_t grid;                 // persistent blocks (at most the resident blocks of the variant)
   int lds_stack;                 // stack entries in LDS: 8, 16 or 32
+  uint32_t wide;                 // 1: the wide form, on wide_grid blocks (grid, lds_stack and record are the binary one's)
+  uint32_t wide_grid;
+  TailQueue* queue;              // of the wide form: chunk * SBS_BATCH_CHUNK + ray (empty between runs)
   int record;                    // 1: the walk records the hit voxel; 0: the hit brick is marched again
 };
 constexpr int SBS_BATCH_BLOCK = 64;
@@ -119,6 +123,7 @@ constexpr int SBS_BATCH_CHUNK = 64;   // rays per work item of the persistent ba
 hipError_t launch_sbs_batch(const SbsBatchLaunch& L, hipStream_t stream);
 // Resident blocks per CU of the persistent batch kernel variant (occupancy query).
 hipError_t sbs_batch_blocks_per_cu(int lds_stack, int record, int* blocks);
+hipError_t sbs_batch_wide_blocks_per_cu(int* blocks);
 
 // Light (core/IRenderer.h:72-78), 32 B
 struct ResolveLight {

@@ -383,8 +383,9 @@ lrt_status lrt_sbs_batch_run(lrt_sbs_batch* b, void* stream);
 /* Chooses the batch kernel's shape by timing runs of the plan on `stream` (which overwrite its
  * outputs): stack entries in LDS (8/16/32), whether the walk records the hit voxel or the hit
  * brick is marched again, and the persistent grid (1/2, 3/4 or all of the resident blocks). The
- * fastest shape is kept in the plan. Gradients agree to float rounding across shapes (the atomic
- * accumulation order differs). No counterpart in the reference. */
+ * fastest shape is kept in the plan, and, where every scene has the six-wide walk, used only if it beats
+ * the form on that walk (the plan's initial one). Gradients agree to float rounding across shapes (the
+ * atomic accumulation order differs). No counterpart in the reference. */
 typedef struct lrt_sbs_batch_tune_result {
   int32_t lds_stack, record;
   uint32_t grid;
@@ -393,8 +394,8 @@ typedef struct lrt_sbs_batch_tune_result {
 } lrt_sbs_batch_tune_result;
 lrt_status lrt_sbs_batch_autotune(lrt_sbs_batch* b, void* stream, lrt_sbs_batch_tune_result* out);
 /* Sets the batch kernel variant and persistent grid directly (a configuration lrt_sbs_batch_autotune
- * reported earlier): lds_stack 8, 16 or 32, record 0 or 1, grid 1 .. the variant's resident
- * blocks. No counterpart in the reference. */
+ * reported earlier) and moves the plan to the binary walk: lds_stack 8, 16 or 32, record 0 or 1, grid
+ * 1 .. the variant's resident blocks. No counterpart in the reference. */
 lrt_status lrt_sbs_batch_configure(lrt_sbs_batch* b, int lds_stack, int record, uint32_t grid);
 lrt_status lrt_sbs_batch_destroy(lrt_sbs_batch* b);
 

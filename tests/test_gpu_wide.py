@@ -278,3 +278,61 @@ def test_bricks(lrt, torch_dev, depth, bs, kind):
         dirs[::5, 3] = 0.6
         hits = b.check(torch_dev, pos, dirs)
         assert (hits["primId"] != lrt.MISS).sum() > 0
+
+
+@pytest.mark.parametrize("depth,n", [(3, 1), (3, 63), (4, 4097), (5, 50000)])
+def test_adjoint(lrt, torch_dev, depth, n):
+    """Colour bit for bit, gradient and loss up to the order of the atomics (fp32 sums of up to 50,000 terms
+    in another order: 1e-5 of the norm)."""
+    torch = torch_dev
+    b = Both(lrt, brick_scene(lrt, depth, 8, "indexed"))
+    pos, dirs = random_rays(torch, n, depth, extent=2.0)
+    dirs[::13, 1] = 0.0
+    params = torch.from_numpy(b.wide.get_array("sbs_data_f")).cuda()
+    params += 0.002 * torch.randn(params.shape, device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    target = torch.rand((n, 4), device="cuda", generator=torch.Generator("cuda").manual_seed(2))
+    got = []
+    for s in (b.wide, b.binary):
+        c = [torch.full((n, 4), -7.0, device="cuda") for _ in range(2)]
+        grads = [torch.zeros_like(params) for _ in range(3)]
+        loss = [torch.zeros(1, device="cuda") for _ in range(2)]
+        s.sbs_forward(0, params, pos, dirs, c[0])
+        s.sbs_backward(0, params, pos, dirs, target, grads[0])
+        s.sbs_l2_backward(0, params, pos, dirs, target, grads[1], loss[0])
+        s.sbs_render_l2_backward(0, params, pos, dirs, target, c[1], grads[2], loss[1])
+        torch.cuda.synchronize()
+        assert s.sbs_recompute_misses() == 0
+        got.append((c, grads, loss))
+    for x, y in zip(got[0][0], got[1][0]):
+        assert torch.equal(x, y)
+    for x, y in zip(got[0][1] + got[0][2], got[1][1] + got[1][2]):
+        assert float((x - y).norm()) <= 1e-5 * float(y.norm()) + 1e-12
+
+
+def test_batch_forms_agree(lrt, torch_dev):
+    """The batched run in the wide form (its default) against the binary one."""
+    torch = torch_dev
+    items = []
+    for k, (depth, n) in enumerate([(3, 1000), (5, 6400), (2, 1), (4, 0), (4, 65)]):
+        s = brick_scene(lrt, depth, 8, "indexed", seed=k)()
+        pos, dirs = random_rays(torch, max(n, 1), k, extent=2.0)
+        pos, dirs = pos[:n].contiguous(), dirs[:n].contiguous()
+        dirs[::9, 2] = 0.0
+        params = torch.from_numpy(s.get_array("sbs_data_f")).cuda()
+        items.append({"scene": s, "geom_id": 0, "params": params, "grad": torch.full_like(params, 9.0),
+                      "loss": torch.full((1,), 9.0, device="cuda"), "pos": pos, "dir": dirs,
+                      "target": torch.full((n, 4), 0.3, device="cuda"), "colour": torch.full((n, 4), -7.0, device="cuda")})
+    runs = []
+    for wide in (True, False):
+        if not wide:
+            for it in items:
+                it["scene"].set_launch_config(256, 16, True)
+        batch = lrt.SbsBatch(items)
+        for _ in range(2):
+            batch.run()
+        torch.cuda.synchronize()
+        runs.append([[it[k].clone() for k in ("colour", "grad", "loss")] for it in items])
+    for a, b in zip(*runs):
+        assert torch.equal(a[0], b[0])
+        for x, y in zip(a[1:], b[1:]):
+            assert float((x - y).norm()) <= 1e-5 * float(y.norm()) + 1e-12
