@@ -717,7 +717,7 @@ lrt_status lrt_autotune(lrt_scene* s, const float* pos_near, const float* dir_fa
     lrt::Scene& sc = s->s;
     const lrt::TuneConfig start{sc.block, sc.lds_stack, sc.xcd_remap, sc.budget, sc.tail_waves,
                                 sc.postpone_triangles() ? 1 : 0, sc.ray_groups, sc.persistent, sc.wide ? 1 : 0};
-    const bool tune_wide = !sc.wideBlocks.empty();
+    const bool tune_wide = !sc.wideBlocks.empty() || sc.make_view().leaf_kinds == lrt::LK_MULTI;
     // the option only exists for triangle-only scenes
     const bool tune_postpone = sc.leaf_kinds() == lrt::LK_TRI;
     auto apply = [&](const lrt::TuneConfig& c) {

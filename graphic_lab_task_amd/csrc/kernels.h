@@ -33,7 +33,7 @@ struct TraceArgs {
   uint32_t      persistent;   // 1: one persistent single-pass kernel with per-lane ray refill
   uint32_t*     pcount;       // its two counters (device, zero between calls)
   uint64_t      spill_words;  // words of the spill
-  uint32_t      wide;         // 1: the six-wide walk where the scene has a wide tree
+  uint32_t      wide;         // 1: the default form of the scene's kind (wide tree, multi-octrees) where it has one
 };
 // Rays beyond n that the work buffer's spill covers, so that a persistent grid (whole blocks of
 // resident lanes, at most ceil(n / block) blocks) can index it by lane slot.
@@ -162,7 +162,7 @@ hipError_t launch_tlas_refit(BVHNode* tlas, uint32_t n_nodes, const uint32_t* pa
                              uint32_t* counters, hipStream_t stream);
 
 hipError_t launch_trace(const SceneView& s, const TraceArgs& a, hipStream_t stream);
-// Largest batch of the wide walk: its counter runs past the batch by a chunk a wave.
+// Largest batch of the kernels that share rays by a counter, which runs past the batch by a chunk a wave.
 constexpr uint32_t WIDE_MAX_RAYS = 0xF0000000u;
 // The wide walk of a scene with a wide tree (trace_wide.hip) and the sequential pass over the rays it queues.
 hipError_t launch_trace_wide(const SceneView& s, const TraceArgs& a, hipStream_t stream);

@@ -1271,16 +1271,20 @@ __device__ __forceinline__ int ot_new_node(float txm, int x, float tym, int y, f
   return (txm < tym) ? (txm < tzm ? x : z) : (tym < tzm ? y : z);
 }
 
-// A stack entry of the octree walk, 8 bytes: the node and where it sits under its parent. The
+// A stack entry of the octree walk, 8 bytes packed: the node and where it sits under its parent. The
 // node's position is not stored: every entry's parent is an ancestor (or itself) of the node the
 // walk expanded last (a depth-first stack holds deeper levels above shallower ones, and a level's
 // entries all come from its most recent expansion), so it is that node's position shifted down
 // to the parent's level, times two, plus the entry's octant bits.
+// It also has the node's children, so that a step waits for one load, their records (28 bits each for the
+// node and the children, both counted from the root).
 struct OTEntry {
   uint32_t node_id;
+  uint32_t children;
   uint32_t meta;   // bits 0-2 octant (x<<2 | y<<1 | z), bits 3-6 level, bit 7 leaf with data (info > 0)
 };
 constexpr int OT_STACK = 32;
+constexpr uint32_t OT_MASK = (1u << 28) - 1;
 constexpr int OT_LDS = 16;   // entries kept in LDS when the caller provides room (2 words each)
 
 // The walk's stack: entries below OT_LDS in the caller's LDS columns (entry k, word j at
@@ -1289,160 +1293,193 @@ constexpr int OT_LDS = 16;   // entries kept in LDS when the caller provides roo
 template <int BLOCK>
 struct OTStack {
   lds_u32* col;
-  OTEntry priv[OT_STACK];
+  uint2 priv[OT_STACK];
   __device__ __forceinline__ OTEntry get(int k) const {
-    if (col && k < OT_LDS) return OTEntry{col[(2 * k) * BLOCK], col[(2 * k + 1) * BLOCK]};
-    return priv[k];
+    const uint2 w = col && k < OT_LDS ? uint2{col[(2 * k) * BLOCK], col[(2 * k + 1) * BLOCK]} : priv[k];
+    return OTEntry{w.x & OT_MASK, w.y & OT_MASK, w.x >> 28 | (w.y >> 28) << 4};
   }
   __device__ __forceinline__ void set(int k, const OTEntry& e) {
+    const uint2 w{e.node_id | e.meta << 28, e.children | (e.meta >> 4) << 28};
     if (col && k < OT_LDS) {
-      col[(2 * k) * BLOCK] = e.node_id;
-      col[(2 * k + 1) * BLOCK] = e.meta;
+      col[(2 * k) * BLOCK] = w.x;
+      col[(2 * k + 1) * BLOCK] = w.y;
     } else {
-      priv[k] = e;
+      priv[k] = w;
     }
   }
 };
 
-// Walks the octree in front-to-back child order with mirrored coordinates (octant mask `a`)
-// and stops at the first leaf whose surface is hit. `ot_col`: LDS columns for the top of the
-// stack (OT_LDS x 2 words per lane, stride BLOCK; may be null: all in private memory).
-// Returns the bytes read from the octree in 16-byte units (node records and voxel values).
+// A ray in an octree walk: mirrored coordinates (octant mask `a`), the root's entry distances and extents per
+// axis, and the position and level of the node expanded last (16 bits each; the root's until then).
+struct OTRay {
+  float3 t0, len;
+  uint32_t a, xy, zl;
+};
+
+__device__ __forceinline__ OTRay ot_ray(float3 pos, float3 dir) {
+  OTRay r;
+  r.a = 0;
+  if (dir.x < 0) { pos.x *= -1; dir.x *= -1; r.a |= 4; }
+  if (dir.y < 0) { pos.y *= -1; dir.y *= -1; r.a |= 2; }
+  if (dir.z < 0) { pos.z *= -1; dir.z *= -1; r.a |= 1; }
+  pos = -1.0f * pos;
+  const float3 inv = safe_inverse(dir);
+  r.t0 = pos * inv - inv;
+  r.len = (pos * inv + inv) - r.t0;
+  r.xy = r.zl = 0;
+  return r;
+}
+
+// Position, level and span of a stack entry.
+struct OTCell {
+  uint32_t x, y, z, level;
+  float3 t0, t1;
+};
+
+__device__ __forceinline__ OTCell ot_cell(const OTRay& r, const OTEntry& e) {
+  OTCell c;
+  c.level = (e.meta >> 3) & 0xFu;
+  c.x = c.y = c.z = 0;
+  if (c.level > 0) {
+    const uint32_t sh = (r.zl >> 16) - (c.level - 1);
+    c.x = (((r.xy & 0xFFFFu) >> sh) << 1) | ((e.meta >> 2) & 1u);
+    c.y = (((r.xy >> 16) >> sh) << 1) | ((e.meta >> 1) & 1u);
+    c.z = (((r.zl & 0xFFFFu) >> sh) << 1) | (e.meta & 1u);
+  }
+  const float d = 1.0f / float(1u << c.level);
+  const float3 p = make3(float(c.x), float(c.y), float(c.z));
+  c.t0 = r.t0 + d * p * r.len;
+  c.t1 = r.t0 + d * (p + 1.0f) * r.len;
+  return c;
+}
+
+// Target node size at distance 1 of the preset's level of detail.
+__device__ __forceinline__ float ot_lod_size(const SceneView& s) { return powf(2.0f, s.preset.level_of_detail) - 0.01f; }
+
+// One step of the walk (children front to back): drops or expands the top entry. True: it is a leaf to be
+// solved, and still on top. `units`: the bytes read from the octree in 16-byte units.
+template <int BLOCK>
+__device__ __forceinline__ bool ot_step(const SceneView& s, uint32_t root, OTRay& r, OTStack<BLOCK>& stack, int& top,
+                                        float tNear, float lod_size, uint32_t& units) {
+  const SdfMultiOctreeNode* nodes = s.multi_nodes + root;
+  const OTEntry e = stack.get(top);
+  const OTCell c = ot_cell(r, e);
+  if (fmin_ref(fmin_ref(c.t1.x, c.t1.y), c.t1.z) < tNear) {
+    top--;
+    return false;
+  }
+  if (e.meta & 0x80u) return true;
+  const float t = s.preset.fixed_lod > 0 ? 1.0f : fmax_ref(c.t0.x, fmax_ref(c.t0.y, c.t0.z));
+  if (float(1u << c.level) > lod_size / t) {
+    units++;
+    if (nodes[e.node_id].voxel_count > 0) return true;
+    top--;
+    return false;
+  }
+  // The children on the ray (at most 4: each step sets another octant bit) in its order, 4 bits each; their
+  // records, which do not decide the order, are then loaded at once.
+  const float3 tm = 0.5f * (c.t0 + c.t1);
+  int curr = ot_first_node(c.t0, tm);
+  uint32_t order = 0, count = 0;
+  do {
+    order |= uint32_t(curr) << (4 * count++);
+    curr = ot_new_node((curr & 4) ? c.t1.x : tm.x, (curr & 4) ? 8 : curr | 4, (curr & 2) ? c.t1.y : tm.y,
+                       (curr & 2) ? 8 : curr | 2, (curr & 1) ? c.t1.z : tm.z, (curr & 1) ? 8 : curr | 1);
+  } while (curr < 8);
+  units += count;
+  // a child is kept (8) if it has voxels or children, as a leaf (16) if it has data and no children: a leaf
+  // entry of the reference carries info = its data offset and counts as a leaf only when info > 0
+  uint32_t kind[4], below[4];
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) {
+    const uint32_t curr_k = (order >> (4 * (k < count ? k : 0u))) & 7u;
+    const SdfMultiOctreeNode n = nodes[e.children + (curr_k ^ r.a)];
+    kind[k] = curr_k;
+    below[k] = n.children_offset > 0 ? n.children_offset - root : 0u;
+    if (k < count && (n.voxel_count > 0 || n.children_offset > 0)) kind[k] |= 8u;
+    if (n.children_offset == 0 && n.data_offset > 0) kind[k] |= 16u;
+  }
+  r.xy = c.x | c.y << 16;
+  r.zl = c.z | c.level << 16;
+  // they replace the current entry, the first one on top; entries past the stack are dropped
+  top += int(((kind[0] >> 3) & 1u) + ((kind[1] >> 3) & 1u) + ((kind[2] >> 3) & 1u) + ((kind[3] >> 3) & 1u)) - 1;
+  int at = top;
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k)
+    if (kind[k] & 8u) {
+      if (at < OT_STACK)
+        stack.set(at, OTEntry{e.children + ((kind[k] & 7u) ^ r.a), below[k],
+                              (kind[k] & 7u) | ((c.level + 1) << 3) | (kind[k] & 16u) << 3});
+      --at;
+    }
+  if (top >= OT_STACK) top = OT_STACK - 1;
+  return false;
+}
+
+// The surface in the voxels of a leaf on top of the stack.
+__device__ __forceinline__ void ot_solve(const SceneView& s, const OTRay& r, const OTEntry& e, uint32_t root, float3 ray_pos,
+                                         float3 ray_dir, float tNear, uint32_t instId, uint32_t geomId, CRT_Hit& hit,
+                                         uint32_t& units) {
+  const OTCell c = ot_cell(r, e);
+  const float old_t = hit.t;
+  const float tmin = fmax_ref(c.t0.x, fmax_ref(c.t0.y, c.t0.z));
+  const float tmax = fmin_ref(c.t1.x, fmin_ref(c.t1.y, c.t1.z));
+  const uint32_t level_sz = 1u << c.level, p_mask = level_sz - 1;
+  const uint32_t rx = (r.a & 4) ? (~c.x & p_mask) : c.x;
+  const uint32_t ry = (r.a & 2) ? (~c.y & p_mask) : c.y;
+  const uint32_t rz = (r.a & 1) ? (~c.z & p_mask) : c.z;
+  const float sz = 0.5f * float(level_sz);
+  const float d = 1.0f / sz;
+  const float3 min_pos = make3(-1, -1, -1) + d * make3(float(rx), float(ry), float(rz));
+  float2 fNearFar;
+  fNearFar.x = tmin;
+  fNearFar.y = tmax;
+  const float3 start_pos = ray_pos + fNearFar.x * ray_dir;
+  const float3 start_q = sz * (start_pos - min_pos);
+  const float qNear = fmax_ref(0.0f, sz * (tNear - fNearFar.x));
+  const float qFar = sz * (fNearFar.y - fNearFar.x);
+  const SdfMultiOctreeNode n = s.multi_nodes[root + e.node_id];
+  const uint32_t info = n.data_offset;
+  units += 1 + 2 * n.voxel_count;
+  const bool surface = (n.flags & MULTI_OCTREE_FLAG_SURFACE) != 0;
+  for (uint32_t v = 0; v < n.voxel_count; ++v) {
+    float values[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) values[i] = s.multi_values[info + 8 * v + i];
+    local_surface_intersection<true>(s, TYPE_SDF_MULTI_OCTREE, ray_dir, instId, geomId, values, e.node_id, d, qNear,
+                                     qFar, fNearFar, start_q, hit, nullptr, surface);
+  }
+  if (s.preset.render_mode == MULTI_RENDER_MODE_MO_VOXEL_COUNT) {
+    if (hit.t < old_t) hit.primId = n.voxel_count;
+  } else if (s.preset.render_mode == MULTI_RENDER_MODE_MO_FLAGS) {
+    if (hit.t < old_t) hit.primId = n.flags;
+  }
+}
+
+__device__ __forceinline__ OTEntry ot_root(const SceneView& s, uint32_t root) {
+  const uint32_t children = s.multi_nodes[root].children_offset;
+  return OTEntry{0u, children > 0 ? children - root : 0u, 0u};
+}
+
+// The whole walk of one instance, which stops at the first leaf whose surface is hit. `ot_col`: LDS columns
+// for the top of the stack (OT_LDS x 2 words per lane, stride BLOCK; may be null: all in private memory).
+// Returns `units`.
 template <int BLOCK = 64>
 __device__ uint32_t multi_octree_intersect(const SceneView& s, const GeomRef& g, float3 ray_pos, float3 ray_dir,
                                            float tNear, uint32_t instId, uint32_t geomId, CRT_Hit& hit,
                                            lds_u32* ot_col = nullptr) {
-  float3 pos_ray_pos = ray_pos;
-  float3 pos_ray_dir = ray_dir;
-  uint32_t a = 0;
-  if (ray_dir.x < 0) { pos_ray_pos.x *= -1; pos_ray_dir.x *= -1; a |= 4; }
-  if (ray_dir.y < 0) { pos_ray_pos.y *= -1; pos_ray_dir.y *= -1; a |= 2; }
-  if (ray_dir.z < 0) { pos_ray_pos.z *= -1; pos_ray_dir.z *= -1; a |= 1; }
-  pos_ray_pos = -1.0f * pos_ray_pos;
-  const float3 inv = safe_inverse(pos_ray_dir);
-  const float3 t0_ = pos_ray_pos * inv - inv;
-  const float3 t1_ = pos_ray_pos * inv + inv;
-  const float3 l_ = t1_ - t0_;
-  // nn_indices of the reference, packed as x | y << 4 | z << 8
-  const uint32_t nn[8] = {0x124u, 0x835u, 0x386u, 0x887u, 0x568u, 0x878u, 0x788u, 0x888u};
-
+  OTRay r = ot_ray(ray_pos, ray_dir);
   OTStack<BLOCK> stack;
   stack.col = ot_col;
   int top = 0;
   uint32_t units = 0;
-  const float old_t = hit.t;
-  const uint32_t type = g.type;
+  const float old_t = hit.t, lod_size = ot_lod_size(s);
   const uint32_t root = g.offset.x;
-  // position and level of the node expanded last (the root's until the first expansion)
-  uint32_t cx = 0, cy = 0, cz = 0, cl = 0;
-  stack.set(0, OTEntry{root, 0u});
+  stack.set(0, ot_root(s, root));
   while (top >= 0) {
-    const OTEntry e = stack.get(top);
-    const uint32_t level = (e.meta >> 3) & 0xFu;
-    uint32_t px = 0, py = 0, pz = 0;
-    if (level > 0) {
-      const uint32_t sh = cl - (level - 1);
-      px = ((cx >> sh) << 1) | ((e.meta >> 2) & 1u);
-      py = ((cy >> sh) << 1) | ((e.meta >> 1) & 1u);
-      pz = ((cz >> sh) << 1) | (e.meta & 1u);
-    }
-    const uint32_t level_sz = 1u << level;
-    float d = 1.0f / float(level_sz);
-    const float3 p_f = make3(float(px), float(py), float(pz));
-    const float3 t0 = t0_ + d * p_f * l_;
-    const float3 t1 = t0_ + d * (p_f + 1.0f) * l_;
-    const float t_out = fmin_ref(fmin_ref(t1.x, t1.y), t1.z);
-    if (t_out < tNear) {
-      top--;
-      continue;
-    }
-    bool is_leaf = (e.meta & 0x80u) != 0;
-    SdfMultiOctreeNode n;
-    bool have_node = false;
-    if (!is_leaf) {
-      const float t = s.preset.fixed_lod > 0 ? 1.0f : fmax_ref(t0.x, fmax_ref(t0.y, t0.z));
-      const float target_lod_size = (powf(2.0f, s.preset.level_of_detail) - 0.01f) / t;
-      if (float(level_sz) > target_lod_size) {
-        n = s.multi_nodes[e.node_id];
-        have_node = true;
-        units++;
-        is_leaf = true;
-        if (n.voxel_count == 0) {
-          top--;
-          continue;
-        }
-      }
-    }
-    if (is_leaf) {
-      const float tmin = fmax_ref(t0.x, fmax_ref(t0.y, t0.z));
-      const float tmax = fmin_ref(t1.x, fmin_ref(t1.y, t1.z));
-      const uint32_t p_mask = level_sz - 1;
-      const uint32_t rx = (a & 4) ? (~px & p_mask) : px;
-      const uint32_t ry = (a & 2) ? (~py & p_mask) : py;
-      const uint32_t rz = (a & 1) ? (~pz & p_mask) : pz;
-      const uint32_t node_id = e.node_id;
-      const float sz = 0.5f * float(level_sz);
-      d = 1.0f / sz;
-      const float3 min_pos = make3(-1, -1, -1) + d * make3(float(rx), float(ry), float(rz));
-      float2 fNearFar;
-      fNearFar.x = tmin;
-      fNearFar.y = tmax;
-      const float3 start_pos = ray_pos + fNearFar.x * ray_dir;
-      const float3 start_q = sz * (start_pos - min_pos);
-      const float qNear = fmax_ref(0.0f, sz * (tNear - fNearFar.x));
-      const float qFar = sz * (fNearFar.y - fNearFar.x);
-      if (!have_node) n = s.multi_nodes[node_id];
-      const uint32_t info = n.data_offset;
-      units += 1 + 2 * n.voxel_count;
-      const bool surface = (n.flags & MULTI_OCTREE_FLAG_SURFACE) != 0;
-      const uint32_t primId = node_id - root;
-      for (uint32_t v = 0; v < n.voxel_count; ++v) {
-        float values[8];
-#pragma unroll
-        for (int i = 0; i < 8; i++) values[i] = s.multi_values[info + 8 * v + i];
-        local_surface_intersection<true>(s, TYPE_SDF_MULTI_OCTREE, ray_dir, instId, geomId, values, primId, d, qNear, qFar,
-                                   fNearFar, start_q, hit, nullptr, surface);
-      }
-      if (s.preset.render_mode == MULTI_RENDER_MODE_MO_VOXEL_COUNT) {
-        if (hit.t < old_t) hit.primId = n.voxel_count;
-      } else if (s.preset.render_mode == MULTI_RENDER_MODE_MO_FLAGS) {
-        if (hit.t < old_t) hit.primId = n.flags;
-      }
-      top = (hit.t < old_t) ? -1 : top - 1;
-    } else {
-      OTEntry buf[4];
-      int buf_top = 0;
-      const float3 tm = 0.5f * (t0 + t1);
-      int curr = ot_first_node(t0, tm);
-      const uint32_t children = s.multi_nodes[e.node_id].children_offset;
-      const uint32_t child_level = (level + 1) << 3;
-      do {
-        const uint32_t child = uint32_t(curr) ^ a;
-        const SdfMultiOctreeNode cn = s.multi_nodes[children + child];
-        units++;
-        const bool child_is_node = cn.children_offset > 0;
-        if ((cn.voxel_count > 0 || child_is_node) && buf_top < 4) {
-          // a leaf entry of the reference carries info = its data offset and counts as a leaf
-          // only when that is non-zero (info > 0); a node's info is 0
-          const bool leaf = !child_is_node && cn.data_offset > 0;
-          buf[buf_top].node_id = children + child;
-          buf[buf_top].meta = uint32_t(curr) | child_level | (leaf ? 0x80u : 0u);
-          buf_top++;
-        }
-        const uint32_t ni = nn[curr];
-        curr = ot_new_node((curr & 4) ? t1.x : tm.x, int(ni & 0xF), (curr & 2) ? t1.y : tm.y, int((ni >> 4) & 0xF),
-                           (curr & 1) ? t1.z : tm.z, int(ni >> 8));
-      } while (curr < 8);
-      cx = px;
-      cy = py;
-      cz = pz;
-      cl = level;
-      // children replace the current entry, the first one on top; entries past the stack are dropped
-      for (int i = 0; i < buf_top; i++)
-        if (top + i < OT_STACK) stack.set(top + i, buf[buf_top - i - 1]);
-      top += buf_top - 1;
-      if (top >= OT_STACK) top = OT_STACK - 1;
-    }
+    if (!ot_step(s, root, r, stack, top, tNear, lod_size, units)) continue;
+    ot_solve(s, r, stack.get(top), root, ray_pos, ray_dir, tNear, instId, geomId, hit, units);
+    top = (hit.t < old_t) ? -1 : top - 1;
   }
   return units;
 }

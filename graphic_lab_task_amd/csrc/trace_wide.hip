@@ -33,30 +33,15 @@
 //    of such a set), are compared by the sequential walk's rule at the node where they part
 //    (wide_before), and the walk goes on past the hit's entry as far as such a leaf can begin
 //    (wide_reach).
-#include <algorithm>
-#include <atomic>
-
-#include "kernels.h"
+#include "wave_rays.h"
 #include "wide_walk.h"
 
 namespace lrt {
 namespace {
 
-constexpr int WIDE_DEVICES = 64;
-// Rays the counter hands out at once. Every fetch is an atomic on one address, about 16 ns each: at 32
-// the 1024 x 1024 octree view takes 0.51 ms instead of 0.43, at 128 the last chunks are uneven (0.53).
-constexpr uint32_t WIDE_CHUNK = 64;
-// Neighbouring rays that start in one wave. Slow rays (silhouettes) are neighbours, and a wave steps
-// through the sum of what its lanes wait for: 327,680 triangles, 512 x 512: 258 us in whole waves of
-// neighbours, 210 in groups of 16, 186 in groups of 8.
-constexpr uint32_t WIDE_GROUP = 8;
-
 // Leaf kinds of the sequential walk that answers a kernel's queued rays.
 constexpr uint32_t wide_kinds(WideLeafKind leaf) { return leaf == WIDE_TRI ? LK_TRI : (leaf == WIDE_FRAME ? LK_FRAME : LK_SBS); }
 
-// Persistent one-wave blocks. `per_wave` rays of a wave's own come first (a power of two up to 64, in
-// groups of at most WIDE_GROUP neighbours from distant parts of the batch), `turns` rounds of them, then
-// chunks from the counter.
 template <WideLeafKind LEAF, bool ANY>
 __global__ __launch_bounds__(WIDE_BLOCK, LEAF == WIDE_BRICK ? 4 : 5) void k_trace_wide(
     SceneView s, const float4* __restrict__ pos, const float4* __restrict__ dir, CRT_Hit* __restrict__ out,
@@ -66,46 +51,7 @@ __global__ __launch_bounds__(WIDE_BLOCK, LEAF == WIDE_BRICK ? 4 : 5) void k_trac
   __shared__ uint32_t lds[2 * WIDE_LDS_STACK * BLOCK];
   __shared__ uint32_t keep[LEAF == WIDE_TRI ? 6 * BLOCK : 1];   // world ray of each lane while it is inside an instance
   const uint32_t lane = threadIdx.x;
-  // an atomic on one address takes about 16 ns, so a wave asks the counter for a chunk at a time
-  const uint32_t own = min(n, gridDim.x * per_wave * turns);
-  uint32_t next = 0, end = 0, turn = 0;
-
-  auto fetch = [&](bool idle, uint32_t n_idle, uint32_t rank, uint32_t& i, bool& exhausted) -> bool {
-    if (turn == 0) {
-      turn = 1;
-      const uint32_t group = min(per_wave, WIDE_GROUP);
-      if (n <= own && turns == 1) exhausted = true;
-      i = (lane / group * gridDim.x + blockIdx.x) * group + lane % group;
-      return lane < per_wave && i < own;
-    }
-    if (next == end && turn < turns) {
-      next = (turn * gridDim.x + blockIdx.x) * BLOCK;
-      end = next + BLOCK;
-      ++turn;
-    }
-    if (next == end) {
-      uint32_t got = 0;
-      if (lane == 0) got = atomicAdd(counter, WIDE_CHUNK);
-      got = __builtin_amdgcn_readfirstlane(got);
-      const uint32_t rest = n - own;
-      if (got >= rest) {
-        exhausted = true;
-        // every wave ends on exactly one fetch past the rays; the one that sees the last value of
-        // all clears the counter for the next call on this stream
-        const uint32_t over = (rest + WIDE_CHUNK - 1) / WIDE_CHUNK * WIDE_CHUNK;
-        if (lane == 0 && got == over + WIDE_CHUNK * (gridDim.x - 1)) atomicExch(counter, 0u);
-        return false;
-      }
-      next = own + got;
-      end = rest - got < WIDE_CHUNK ? n : next + WIDE_CHUNK;
-    }
-    const uint32_t count = min(n_idle, end - next);
-    const bool mine = idle && rank < count;
-    if (mine) i = next + rank;
-    next += count;
-    if (next == end && turn == turns && n <= own) exhausted = true;
-    return mine;
-  };
+  WaveRays fetch{n, per_wave, turns, counter};
   auto done = [&](uint32_t i, CRT_Hit& hit, uint32_t, bool again) {
     if (again) {
       queue->list[atomicAdd(&queue->count, 1u)] = i;
@@ -213,49 +159,24 @@ __global__ void k_wide_refit(WideBlock* blocks, uint32_t n_blocks, const uint32_
   }
 }
 
-// Blocks of a kernel that are resident on the current device at once (asked once per device).
-template <class K>
-hipError_t resident_blocks(K kernel, std::atomic<uint32_t>* known, uint32_t* blocks) {
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  uint32_t r = dev < WIDE_DEVICES ? known[dev].load(std::memory_order_relaxed) : 0u;
-  if (r == 0) {
-    int per_cu = 0, cus = 0;
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), WIDE_BLOCK, 0);
-    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e != hipSuccess) return e;
-    r = uint32_t(per_cu > 0 ? per_cu : 1) * uint32_t(cus > 0 ? cus : 1);
-    if (dev < WIDE_DEVICES) known[dev].store(r, std::memory_order_relaxed);
-  }
-  *blocks = r;
-  return hipSuccess;
-}
-
 template <WideLeafKind LEAF, bool ANY>
 hipError_t launch_wide_t(const SceneView& s, const TraceArgs& a, hipStream_t stream) {
-  static std::atomic<uint32_t> known[WIDE_DEVICES], known_queued[WIDE_DEVICES];
+  static std::atomic<uint32_t> known[WAVE_DEVICES], known_queued[WAVE_DEVICES];
   const uint32_t waves = (a.n + WIDE_BLOCK - 1) / WIDE_BLOCK;
   uint32_t resident = 0, resident_queued = 0;
   hipError_t e = resident_blocks(k_trace_wide<LEAF, ANY>, known, &resident);
   if (e == hipSuccess) e = resident_blocks(k_trace_queued<LEAF>, known_queued, &resident_queued);
   if (e != hipSuccess) return e;
-  // A wave's own rays: as many waves as fit at once share the batch, down to one ray a wave, whose other
-  // lanes then walk parts of it. A tree of more levels than the LDS stack spills by lane of the grid.
+  // Lanes without a ray walk parts of the others. A tree of more levels than the LDS stack spills by lane of
+  // the grid.
   uint32_t most = resident, spill_stride = 0;
   if (s.wide_levels > uint32_t(WIDE_LDS_STACK)) {
     spill_stride = 2 * (s.wide_levels - WIDE_LDS_STACK);   // at most 56 words; the spill has 72 a ray
     most = uint32_t(std::min<uint64_t>(most, a.spill_words / (spill_stride * WIDE_BLOCK)));
   }
-  uint32_t per_wave = WIDE_BLOCK;
-  while (per_wave > 1 && a.n / (per_wave / 2) < most) per_wave /= 2;
-  const uint32_t grid = std::min((a.n + per_wave - 1) / per_wave, most);
-  // Whole rounds of own rays while a quarter of the batch is left for the counter, which evens out what
-  // the waves were dealt (1024 x 1024 octree view: 0.43 ms, all by the counter 0.49; 4 M bounce rays: 2.88
-  // ms, none by the counter 3.5).
-  const uint32_t turns = std::max(1u, uint32_t(uint64_t(a.n) * 3 / 4 / (uint64_t(grid) * per_wave)));
-  hipLaunchKernelGGL((k_trace_wide<LEAF, ANY>), dim3(grid), dim3(WIDE_BLOCK), 0, stream, s, a.pos, a.dir, a.out,
-                     a.any_out, a.n, per_wave, turns, a.spill, spill_stride, a.pcount, a.queue);
+  const WaveShares w = wave_shares(a.n, most);
+  hipLaunchKernelGGL((k_trace_wide<LEAF, ANY>), dim3(w.grid), dim3(WIDE_BLOCK), 0, stream, s, a.pos, a.dir, a.out,
+                     a.any_out, a.n, w.per_wave, w.turns, a.spill, spill_stride, a.pcount, a.queue);
   hipLaunchKernelGGL((k_trace_queued<LEAF>), dim3(std::min(waves, resident_queued)), dim3(WIDE_BLOCK), 0, stream, s,
                      a.pos, a.dir, a.out, a.any_out, a.overflow_count, a.spill, a.queue);
   return hipGetLastError();

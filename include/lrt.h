@@ -287,8 +287,8 @@ lrt_status lrt_eye_rays_dev(const float* proj_inv16, const float* world_view_inv
                             const float* jitter, uint32_t order, float* pos_near, float* dir_far, void* stream);
 
 /* Scenes of triangle meshes, and scenes of one frame-octree or sparse-voxel-set instance, are traced by
- * a six-wide walk built at commit that has no launch shape to choose (other scenes, counted calls and
- * the INTERSECTION_COUNT mode take the binary walk). Each of the launch-shape calls below
+ * a six-wide walk built at commit that has no launch shape to choose, scenes of multi-octrees by a kernel
+ * that has none either (other scenes, counted calls and the INTERSECTION_COUNT mode take the binary walk). Each of the launch-shape calls below
  * (lrt_set_launch_config, lrt_set_tail_config, lrt_set_leaf_postponement with 0 or 1,
  * lrt_set_ray_interleave, lrt_set_persistent) moves the scene to the binary walk in that shape;
  * lrt_autotune tries both and keeps the faster. Same hit records either way.

@@ -1,5 +1,5 @@
 """The wide walk (trace_wide.hip, the default on triangle scenes, single frame octrees and brick sets)
-against the binary walk, record for record: tile and batch edges, instances, first-hit and any-hit rays,
+and the multi-octree kernel (trace_multi.hip) against the binary walk, record for record: tile and batch edges, instances, first-hit and any-hit rays,
 rays and scenes that fall back to the sequential walk, a tree deeper than the LDS stack, the refitted
 instance level, graph replay and the allocation-free entry point."""
 import numpy as np
@@ -8,6 +8,7 @@ import pytest
 from conftest import raw_equal
 
 pytestmark = pytest.mark.gpu
+MO_VOXEL_COUNT = 24   # MULTI_RENDER_MODE_MO_VOXEL_COUNT
 
 
 @pytest.fixture(scope="module")
@@ -35,12 +36,12 @@ def flags(torch, s, pos, dirs):
 class Both:
     """The same scene twice: the default (wide) walk and the binary walk."""
 
-    def __init__(self, g, build):
+    def __init__(self, g, build, tree=True):
         self.g = g
         self.wide, self.binary = build(), build()
         self.binary.set_launch_config(256, 16, True)
         self.binary.set_tail_config(0, 1024)
-        assert self.wide.get_array("wide_blocks").size
+        assert bool(self.wide.get_array("wide_blocks").size) == tree
 
     def check(self, torch, pos, dirs, fn="trace_closest", any_hit=True):
         a, b = (trace(torch, self.g, s, pos, dirs, fn) for s in (self.wide, self.binary))
@@ -336,3 +337,52 @@ def test_batch_forms_agree(lrt, torch_dev):
         assert torch.equal(a[0], b[0])
         for x, y in zip(a[1:], b[1:]):
             assert float((x - y).norm()) <= 1e-5 * float(y.norm()) + 1e-12
+
+
+@pytest.mark.parametrize("depth,count,lod,n", [(2, 1, 0.0, 1), (3, 2, 0.0, 63), (6, 1, 3.0, 70000), (7, 3, 0.0, 100001),
+                                               (8, 1, 0.0, 400000)])
+def test_multi_octrees(lrt, torch_dev, depth, count, lod, n):
+    """Small and large batches, several instances, levels of detail, first-hit and any-hit rays, axis-parallel
+    rays, the modes that put node properties into the record, graph replay."""
+    torch, g = torch_dev, lrt
+    rng = np.random.default_rng(4)
+    sph = np.concatenate([rng.uniform(-0.7, 0.7, (48, 3)), rng.uniform(0.05, 0.25, (48, 1))], 1).astype(np.float32)
+    nodes, values = g.sdf_spheres_multi_octree(sph, depth)
+
+    def make():
+        s = g.SceneRT()
+        for _ in range(min(count, 2)):
+            gid = s.AddGeom_SdfMultiOctree(nodes, values)
+        for k, m in enumerate(mats(count, 3, 0.4)):
+            s.AddInstance(k % (gid + 1), m if count > 1 else None)
+        s.CommitScene()
+        return s
+    b = Both(g, make, tree=False)
+    pos, dirs = random_rays(torch, n, depth, extent=2.0)
+    dirs[::11, 0] = 0.0
+    dirs[::5, 3] = 0.6
+    dirs[::7, 3] *= -1.0
+    for mode in (g.MULTI_RENDER_MODE_LAMBERT_NO_TEX, MO_VOXEL_COUNT):
+        preset = g.default_preset()
+        preset["render_mode"] = mode
+        if lod:
+            preset["fixed_lod"], preset["level_of_detail"] = 1, lod
+        for s in (b.wide, b.binary):
+            s.SetPreset(preset)
+        hits = b.check(torch, pos, dirs)
+        assert n < 63 or (hits["geomId"] != g.MISS).sum() > 0
+    if n <= 65536:
+        assert raw_equal(trace(torch, g, b.wide, pos, dirs, "trace_closest_noalloc"), hits)
+    out = torch.zeros((n, 8), dtype=torch.int32, device="cuda")
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        b.wide.trace_closest(pos, dirs, out, stream=side.cuda_stream)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            b.wide.trace_closest(pos, dirs, out, stream=torch.cuda.current_stream().cuda_stream)
+    for _ in range(3):
+        out.fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert raw_equal(out.cpu().numpy().view(g.HIT_DTYPE).reshape(-1), hits)
