@@ -81,6 +81,7 @@ Scene::~Scene() {
   work.clear();
   dev.clear();
   if (d_overflow) (void)hipFree(d_overflow);
+  if (host_pinned) (void)hipHostFree(host_pinned);
 }
 
 namespace {

@@ -156,6 +156,7 @@ struct Scene {
   // only, so a picking loop allocates on its first call and never again.
   std::mutex host_mu;
   DevBuf host_io;
+  void* host_pinned = nullptr;   // pinned host memory for the rays and records of small calls
 
   // Commit generation: bumped by every change that invalidates device pointers handed out
   // earlier (commit, clear, add, instance update). Batch plans record it and refuse to run once

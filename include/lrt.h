@@ -216,8 +216,9 @@ lrt_status lrt_trace_closest_dev(lrt_scene* s, const float* pos_near, const floa
 lrt_status lrt_trace_closest_noalloc_dev(lrt_scene* s, const float* pos_near, const float* dir_far, lrt_hit* hits,
                                          uint64_t n, void* stream);
 
-/* Same over host buffers (copies in, traces, copies out, synchronises). The device staging
- * buffer belongs to the scene and only grows: repeated calls of one size allocate nothing. */
+/* Same over host buffers (copies in, traces, copies out, synchronises). The staging buffers (pinned
+ * host memory for up to 4096 rays, device memory for more) belong to the scene and only grow:
+ * repeated calls of one size allocate nothing. */
 lrt_status lrt_trace_closest_host(lrt_scene* s, const float* pos_near, const float* dir_far, lrt_hit* hits,
                                   uint64_t n);
 

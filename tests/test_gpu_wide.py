@@ -386,3 +386,13 @@ def test_multi_octrees(lrt, torch_dev, depth, count, lod, n):
         graph.replay()
         torch.cuda.synchronize()
         assert raw_equal(out.cpu().numpy().view(g.HIT_DTYPE).reshape(-1), hits)
+
+
+@pytest.mark.parametrize("n", [1, 4096, 4097])
+def test_host_staging(lrt, torch_dev, n):
+    """Host calls staged in pinned memory (up to 4,096 rays) and by copies give the device call's records."""
+    s = mesh(lrt, 12)()
+    pos, dirs = random_rays(torch_dev, n, 3)
+    want = trace(torch_dev, lrt, s, pos, dirs)
+    for _ in range(2):
+        assert raw_equal(s.trace_closest_host(pos.cpu().numpy(), dirs.cpu().numpy()), want)
