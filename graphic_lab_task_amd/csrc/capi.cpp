@@ -92,7 +92,7 @@ lrt::TraceArgs trace_args(lrt_scene* s, const float* pos, const float* dir, lrt_
   a.postpone_tri = s->s.preset.render_mode != lrt::MULTI_RENDER_MODE_INTERSECTION_COUNT && s->s.postpone_triangles();
   a.persistent = s->s.persistent ? 1u : 0u;
   // (the wide walk visits other leaves, too)
-  a.wide = s->s.wide && s->s.preset.render_mode != lrt::MULTI_RENDER_MODE_INTERSECTION_COUNT;
+  a.wide = s->s.wide && s->s.preset.render_mode != lrt::MULTI_RENDER_MODE_INTERSECTION_COUNT && !s->s.rays_crowd(n);
   return a;
 }
 

@@ -162,6 +162,11 @@ hipError_t launch_tlas_refit(BVHNode* tlas, uint32_t n_nodes, const uint32_t* pa
                              uint32_t* counters, hipStream_t stream);
 
 hipError_t launch_trace(const SceneView& s, const TraceArgs& a, hipStream_t stream);
+// Counters by which persistent waves share a batch (wave_rays.h), each in a line of its own behind the
+// persistent kernel's: counter c is word WAVE_COUNTER_AT + c * WAVE_COUNTER_WORDS from there, zero between calls.
+constexpr uint32_t WAVE_COUNTERS = 16, WAVE_COUNTER_WORDS = 64, WAVE_COUNTER_AT = 48;
+// Header of a work buffer: the tail queue at byte 0, the persistent kernel's counters at 64, the waves' at 256.
+constexpr uint32_t WORK_HEAD_BYTES = 256 + WAVE_COUNTERS * WAVE_COUNTER_WORDS * 4;
 // Largest batch of the kernels that share rays by a counter, which runs past the batch by a chunk a wave.
 constexpr uint32_t WIDE_MAX_RAYS = 0xF0000000u;
 // The wide walk of a scene with a wide tree (trace_wide.hip) and the sequential pass over the rays it queues.

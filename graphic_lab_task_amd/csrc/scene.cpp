@@ -44,11 +44,11 @@ Scene::StreamWork& Scene::stream_work(void* stream) {
 
 hipError_t Scene::work_for(StreamWork& w, void* stream, size_t n, uint32_t** spill, TailQueue** queue,
                            uint32_t** pcount, uint64_t* spill_words) {
-  // 256-B header: the tail queue's counters and list pointer at 0, the persistent kernel's two
-  // counters at byte 64; then the queue list (4 B per ray) and the spill, sized for the smallest
+  // header: the tail queue's counters and list pointer at 0, the persistent kernel's two counters at
+  // byte 64, the counters by which waves share rays from byte 256 on; then the queue list (4 B per ray) and the spill, sized for the smallest
   // LDS part so that a later launch-config change never overruns it, and for a persistent grid's
   // lane slots (up to SPILL_SLACK_RAYS past n)
-  const size_t head = 256;
+  const size_t head = WORK_HEAD_BYTES;
   const size_t list_bytes = (n * 4 + 255) / 256 * 256;
   const size_t need = head + list_bytes + (n + SPILL_SLACK_RAYS) * size_t(STACK_SIZE - 8) * 4;
   if (w.cap_rays < n || w.buf.bytes() < need) {
@@ -60,7 +60,7 @@ hipError_t Scene::work_for(StreamWork& w, void* stream, size_t n, uint32_t** spi
       w.cap_rays = 0;
       return e;
     }
-    uint8_t header[256] = {};
+    uint8_t header[WORK_HEAD_BYTES] = {};
     TailQueue q{0u, 0u, reinterpret_cast<uint32_t*>(static_cast<char*>(w.buf.ptr()) + head)};
     std::memcpy(header, &q, sizeof(q));
     e = hipMemcpy(w.buf.ptr(), header, sizeof(header), hipMemcpyHostToDevice);
@@ -633,6 +633,20 @@ uint32_t Scene::leaf_kinds() const {
     else if (t == TAG_SCOM2) k |= LK_SCOM2;
   }
   return k;
+}
+
+// With hundreds of rays a triangle the lanes of a wave go the same way, and a binary step of one shared fetch
+// and two box tests is cheaper than a wide one of six. Camera rays, wide against binary: 500 triangles, 182
+// thousand rays 56 us against 48 and 30 thousand 38 against 48; 1,280 triangles, 990 thousand 150 against 103 and
+// 182 thousand 62 against 61; 5,120 triangles, 990 thousand 178 against 162 and 182 thousand 77 against 98;
+// 20,480 triangles, 990 thousand 217 against 288. So the line is at 128 rays a triangle, and at 65,536 rays,
+// below which the wide walk's shorter chains win for any mesh. Bricks hold some
+// hundred voxels each: 384 bricks, 630 thousand rays 331 against 316 and 30 thousand 87 against 245; 6,144
+// bricks, 480 thousand 580 against 3,000: 1,024 rays a brick.
+bool Scene::rays_crowd(uint64_t n) const {
+  if (n < 65536 || instances.size() != 1 || geomTags.size() != 1) return false;
+  if (geomTags[0] == TAG_TRIANGLE) return n >= 128ull * (indices.size() / 3);
+  return geomTags[0] == TAG_SDF_BRICK && n >= 1024ull * sbsNodes.size();
 }
 
 // Postponed triangle leaves help coherent rays into one mesh (fewer wave-wide waits) and hurt

@@ -130,6 +130,8 @@ struct Scene {
   double tlasAreaNow = 0.0;           // the same after the last refit
   uint32_t lastCommitKind = 0;        // LRT_COMMIT_* of the last commit
   bool postpone_triangles() const;
+  // Many rays into one small mesh or brick set: default calls keep the binary walk.
+  bool rays_crowd(uint64_t n) const;
 
   // Work memory of one stream: the tail queue (256-B header + list), the deep-stack spill and
   // the occupancy masks of calls whose values differ from the committed ones. A call holds

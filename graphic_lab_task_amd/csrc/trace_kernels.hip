@@ -7,12 +7,12 @@
 
 namespace lrt {
 
-// Work memory of the allocation-free trace: a 256-B header (tail queue at word 0, the persistent
-// kernel's counters at word 16), the queue (one word per ray) and the deep-stack spill
+// Work memory of the allocation-free trace: the header (tail queue at word 0, the persistent
+// kernel's counters at word 16, the waves' from word 64), the queue (one word per ray) and the deep-stack spill
 // (STACK_SIZE - 8 words per ray, enough for every LDS stack depth, plus the persistent grid's
 // slack), for at most LRT_NOALLOC_MAX_RAYS rays. Host code never uses this name as an address: each
 // device's copy is resolved once with hipGetSymbolAddress and that pointer is passed on.
-constexpr size_t NOALLOC_HEAD_WORDS = 64;
+constexpr size_t NOALLOC_HEAD_WORDS = WORK_HEAD_BYTES / 4;
 constexpr size_t NOALLOC_WORDS =
     NOALLOC_HEAD_WORDS + LRT_NOALLOC_MAX_RAYS + size_t(LRT_NOALLOC_MAX_RAYS + SPILL_SLACK_RAYS) * (STACK_SIZE - 8);
 static __device__ __align__(256) uint32_t scratch[NOALLOC_WORDS];
@@ -27,6 +27,7 @@ __global__ void k_queue_init(TailQueue* queue, uint32_t* list, uint32_t* pcount)
     pcount[0] = 0;
     pcount[1] = 0;
   }
+  if (threadIdx.x < WAVE_COUNTERS) pcount[WAVE_COUNTER_AT + threadIdx.x * WAVE_COUNTER_WORDS] = 0;
 }
 
 // Clears the tail queue when a call's second pass could not be launched (a kernel rather than a

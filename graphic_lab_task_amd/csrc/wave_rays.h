@@ -8,8 +8,9 @@
 namespace lrt {
 
 constexpr uint32_t WAVE_LANES = 64;
-// Rays the counter hands out at once. Every fetch is an atomic on one address, about 16 ns each: at 32
-// the 1024 x 1024 octree view takes 0.51 ms instead of 0.43, at 128 the last chunks are uneven (0.53).
+// Rays a counter hands out at once. Every fetch is an atomic, about 16 ns each on one address: with one
+// counter, at 32 the 1024 x 1024 octree view takes 0.51 ms instead of 0.43, at 128 the last chunks are
+// uneven (0.53).
 constexpr uint32_t WAVE_CHUNK = 64;
 // Neighbouring rays that start in one wave. Slow rays (silhouettes) are neighbours, and a wave steps
 // through the sum of what its lanes wait for: 327,680 triangles, 512 x 512: 258 us in whole waves of
@@ -17,14 +18,28 @@ constexpr uint32_t WAVE_CHUNK = 64;
 constexpr uint32_t WAVE_GROUP = 8;
 
 // A wave's rays: `per_wave` of its own come first (a power of two up to 64, in groups of at most WAVE_GROUP
-// neighbours from distant parts of the batch), `turns` rounds of them, then chunks from the counter.
+// neighbours from distant parts of the batch), `turns` rounds of them (the later ones of 64, so that more than
+// one takes per_wave 64), then chunks from a counter. Wave w uses counter w mod WAVE_COUNTERS, which has its
+// own part of the rest: with one counter for all, a wave's fetches and its last, failing one queued up for
+// 16 ns each (1100 x 900 rays into 500 triangles: 189 us, now 134; the octree view below 432, now 401).
 struct WaveRays {
   uint32_t n, per_wave, turns;
-  uint32_t* counter;   // 0 between calls
+  uint32_t* counter;                 // the wave's, 0 between calls
+  uint32_t first = 0, rest = 0;      // its part of the batch
+  uint32_t waves = 0;                // that share it
   uint32_t next = 0, end = 0, turn = 0;
 
   __device__ __forceinline__ WaveRays(uint32_t n_, uint32_t per_wave_, uint32_t turns_, uint32_t* counter_)
-      : n(n_), per_wave(per_wave_), turns(turns_), counter(counter_) {}
+      : n(n_), per_wave(per_wave_), turns(turns_) {
+    const uint32_t own = min(n, gridDim.x * per_wave * turns), left = n - own;
+    const uint32_t counters = min(WAVE_COUNTERS, gridDim.x), c = blockIdx.x % counters;
+    const uint32_t part = (left / counters + WAVE_CHUNK) / WAVE_CHUNK * WAVE_CHUNK;   // >= left / counters, whole chunks
+    first = min(left, c * part);
+    rest = min(left - first, part);
+    first += own;
+    waves = (gridDim.x - c + counters - 1) / counters;
+    counter = counter_ + WAVE_COUNTER_AT + c * WAVE_COUNTER_WORDS;
+  }
 
   // Called by all lanes of the wave. Whether the lane (idle, `rank` of the n_idle idle ones) gets a ray, in
   // i; sets `exhausted` (wave-uniform) when no more come.
@@ -43,21 +58,23 @@ struct WaveRays {
       ++turn;
     }
     if (next == end) {
-      // an atomic on one address takes about 16 ns, so a wave asks the counter for a chunk at a time
+      if (rest == 0) {
+        exhausted = true;
+        return false;
+      }
       uint32_t got = 0;
       if (lane == 0) got = atomicAdd(counter, WAVE_CHUNK);
       got = __builtin_amdgcn_readfirstlane(got);
-      const uint32_t rest = n - own;
       if (got >= rest) {
         exhausted = true;
-        // every wave ends on exactly one fetch past the rays; the one that sees the last value of
-        // all clears the counter for the next call on this stream
+        // every wave of the counter ends on exactly one fetch past its rays; the one that sees the last
+        // value of all clears it for the next call on this stream
         const uint32_t over = (rest + WAVE_CHUNK - 1) / WAVE_CHUNK * WAVE_CHUNK;
-        if (lane == 0 && got == over + WAVE_CHUNK * (gridDim.x - 1)) atomicExch(counter, 0u);
+        if (lane == 0 && got == over + WAVE_CHUNK * (waves - 1)) atomicExch(counter, 0u);
         return false;
       }
-      next = own + got;
-      end = rest - got < WAVE_CHUNK ? n : next + WAVE_CHUNK;
+      next = first + got;
+      end = first + (rest - got < WAVE_CHUNK ? rest : got + WAVE_CHUNK);
     }
     const uint32_t count = min(n_idle, end - next);
     const bool mine = idle && rank < count;
@@ -80,7 +97,8 @@ inline WaveShares wave_shares(uint32_t n, uint32_t most) {
   // Whole rounds of own rays while a quarter of the batch is left for the counter, which evens out what
   // the waves were dealt (1024 x 1024 octree view: 0.43 ms, all by the counter 0.49; 4 M bounce rays: 2.88
   // ms, none by the counter 3.5).
-  w.turns = std::max(1u, uint32_t(uint64_t(n) * 3 / 4 / (uint64_t(w.grid) * w.per_wave)));
+  if (w.per_wave == WAVE_LANES)
+    w.turns = std::max(1u, uint32_t(uint64_t(n) * 3 / 4 / (uint64_t(w.grid) * w.per_wave)));
   return w;
 }
 
