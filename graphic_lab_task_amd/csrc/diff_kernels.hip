@@ -12,6 +12,7 @@
 #include <algorithm>
 
 #include "kernels.h"
+#include "wave_rays.h"
 #include "wide_walk.h"
 
 namespace lrt {
@@ -168,7 +169,7 @@ __global__ __launch_bounds__(BLOCK) void k_sbs_diff(SceneView s, SbsDiffArgs a) 
 // What bounds it: vector instructions of solves and node steps at a sixth and half of the lanes, and the
 // waves with the most grazing rays. Whole calls, masks included, against one ray a lane of the binary walk:
 // 8 x 256 x 256 rays into 256^3 voxels 0.79 ms against 0.86, 3 x 201 x 201 rays into 128^3, forward and
-// backward apart, 0.68 against 0.87, the batch above 0.68 against 0.90.
+// backward apart, 0.57 against 0.87, the batch above 0.68 against 0.90.
 template <int MODE>
 __device__ __forceinline__ float diff_wave(const SceneView& s, const SbsDiffArgs& a, bool mine, uint32_t ray,
                                            wide_lds* lds, wide_lds* result, uint32_t* spill,
@@ -218,12 +219,14 @@ __device__ __forceinline__ float diff_wave(const SceneView& s, const SbsDiffArgs
 }
 
 template <int MODE>
-__global__ __launch_bounds__(WIDE_BLOCK, 4) void k_sbs_diff_wide(SceneView s, SbsDiffArgs a) {
+__global__ __launch_bounds__(WIDE_BLOCK, 4) void k_sbs_diff_wide(SceneView s, SbsDiffArgs a, uint32_t per_wave) {
   __shared__ uint32_t lds[2 * WIDE_LDS_STACK * WIDE_BLOCK];
   __shared__ uint32_t result[3 * WIDE_BLOCK];
-  // groups of 8 neighbours from distant parts of the batch, as the trace kernel
-  const uint32_t lane = threadIdx.x, i = (lane / 8u * gridDim.x + blockIdx.x) * 8u + lane % 8u;
-  float loss = diff_wave<MODE>(s, a, i < a.n, i, (wide_lds*)(lds), (wide_lds*)(result),
+  // per_wave rays in groups of at most WAVE_GROUP neighbours from distant parts of the batch, as the trace
+  // kernel; the other lanes walk parts of them
+  const uint32_t lane = threadIdx.x, group = min(per_wave, WAVE_GROUP);
+  const uint32_t i = (lane / group * gridDim.x + blockIdx.x) * group + lane % group;
+  float loss = diff_wave<MODE>(s, a, lane < per_wave && i < a.n, i, (wide_lds*)(lds), (wide_lds*)(result),
                                a.spill + size_t(blockIdx.x * WIDE_BLOCK + lane) * (STACK_SIZE - 16), a.queue, i);
   if (MODE >= 2 && a.loss) {
     loss = wave_sum(loss);
@@ -450,8 +453,16 @@ constexpr uint32_t QUEUED_BLOCKS = 2048;
 template <int MODE>
 hipError_t launch_mode(const SceneView& s, const SbsDiffArgs& a, hipStream_t stream) {
   if (s.wide) {
-    hipLaunchKernelGGL((k_sbs_diff_wide<MODE>), dim3((a.n + WIDE_BLOCK - 1) / WIDE_BLOCK), dim3(WIDE_BLOCK), 0, stream, s,
-                       a);
+    static std::atomic<uint32_t> known[WAVE_DEVICES];
+    uint32_t resident = 0;
+    const hipError_t e = resident_blocks(k_sbs_diff_wide<MODE>, known, &resident);
+    if (e != hipSuccess) return e;
+    // As many waves as are resident share the batch, so that lanes without a ray help (3 x 201 x 201 rays: 0.57
+    // ms a call, 64 rays a wave 0.66). A tree of more levels than the LDS stack spills, and the spill has room
+    // for a lane a ray.
+    const uint32_t per_wave = s.wide_levels > uint32_t(WIDE_LDS_STACK) ? WAVE_LANES : wave_shares(a.n, resident).per_wave;
+    hipLaunchKernelGGL((k_sbs_diff_wide<MODE>), dim3((a.n + per_wave - 1) / per_wave), dim3(WIDE_BLOCK), 0, stream, s, a,
+                       per_wave);
     // mostly nothing is queued; as many blocks as fit at once take it if everything is
     hipLaunchKernelGGL((k_sbs_diff_queued<MODE>), dim3(std::min((a.n + WIDE_BLOCK - 1) / WIDE_BLOCK, QUEUED_BLOCKS)),
                        dim3(WIDE_BLOCK), 0, stream, s, a);
