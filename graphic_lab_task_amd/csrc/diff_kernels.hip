@@ -200,8 +200,10 @@ __device__ __forceinline__ float diff_wave(const SceneView& s, const SbsDiffArgs
     queue->list[atomicAdd(&queue->count, 1u)] = code;
     return 0.0f;
   }
-  if (prim != 0xFFFFFFFFu) {
-    const WideInstance* w = reinterpret_cast<const WideInstance*>(s.wide);
+  // The scene's only instance may be of another set, whose words are no indices into the parameters (they can
+  // be packed 8- or 16-bit codes): its hits have no voxel to differentiate, and colour 0 as on the binary walk.
+  const WideInstance* w = reinterpret_cast<const WideInstance*>(s.wide);
+  if (prim != 0xFFFFFFFFu && w->geom_id == a.geom_id) {
     const GeomRef g = geom_ref(s, w->geom_id);
     float3 lo, ld;
     wide_local_ray(w, xyz(p), xyz(d), lo, ld);

@@ -310,6 +310,57 @@ def test_adjoint(lrt, torch_dev, depth, n):
         assert float((x - y).norm()) <= 1e-5 * float(y.norm()) + 1e-12
 
 
+@pytest.mark.parametrize("other", [1, 2, "indexed"])
+def test_adjoint_of_another_set(lrt, torch_dev, other):
+    """Two brick sets, the first (of packed codes or indices) or the second one instanced, the second one
+    differentiated: rays that hit the first have no colour, no gradient and a loss against 0."""
+    torch, g = torch_dev, lrt
+    rng = np.random.default_rng(2)
+    sph = np.concatenate([rng.uniform(-0.8, 0.8, (64, 3)), rng.uniform(0.05, 0.2, (64, 1))], 1).astype(np.float32)
+
+    def add(s, kind, depth):
+        if kind == "indexed":
+            return s.AddGeom_SdfSBS(*g.sdf_spheres_sbs_indexed(sph, depth, 8, 3)[:4])
+        h = np.zeros((), g.SBS_HEADER_DTYPE)
+        h["brick_size"], h["bytes_per_value"], h["aux_data"] = 4, kind, g.SDF_SBS_NODE_LAYOUT_DX
+        return s.AddGeom_SdfSBS(h, *g.sdf_spheres_sbs(sph, depth, h))
+
+    n = 5001
+    pos, dirs = random_rays(torch, n, 4, extent=2.0)
+    dirs[::13, 1] = 0.0   # some rays take the sequential walk
+    target = torch.rand((n, 4), device="cuda", generator=torch.Generator("cuda").manual_seed(2))
+    for instanced in (0, 1):
+        def make():
+            s = g.SceneRT()
+            s.AddInstance((add(s, other, 3), add(s, "indexed", 4))[instanced])
+            s.CommitScene()
+            return s
+        b = Both(g, make)
+        assert (b.check(torch, pos, dirs)["primId"] != g.MISS).sum() > 300
+        params = torch.from_numpy(b.wide.get_array("sbs_data_f")).cuda()
+        got = []
+        for s in (b.wide, b.binary):
+            c = [torch.full((n, 4), -7.0, device="cuda") for _ in range(2)]
+            grads = [torch.zeros_like(params) for _ in range(3)]
+            loss = [torch.zeros(1, device="cuda") for _ in range(2)]
+            s.sbs_forward(1, params, pos, dirs, c[0])
+            s.sbs_backward(1, params, pos, dirs, target, grads[0])
+            s.sbs_l2_backward(1, params, pos, dirs, target, grads[1], loss[0])
+            s.sbs_render_l2_backward(1, params, pos, dirs, target, c[1], grads[2], loss[1])
+            torch.cuda.synchronize()
+            assert s.sbs_recompute_misses() == 0
+            if instanced == 0:
+                # the loss: an fp32 sum of n terms in any order, each step of which rounds by 2^-24
+                want = float((target[:, :3].double() ** 2).sum())
+                assert all(not x.any() for x in c + grads)
+                assert all(abs(float(x) - want) <= n * 2.0 ** -24 * want for x in loss)
+            got.append((c, grads + loss))
+        for x, y in zip(got[0][0], got[1][0]):
+            assert torch.equal(x, y)
+        for x, y in zip(got[0][1], got[1][1]):
+            assert float((x - y).norm()) <= 1e-5 * float(y.norm()) + 1e-12
+
+
 def test_batch_forms_agree(lrt, torch_dev):
     """The batched run in the wide form (its default) against the binary one."""
     torch = torch_dev
