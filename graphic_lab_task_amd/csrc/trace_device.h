@@ -1456,9 +1456,11 @@ __device__ __forceinline__ void ot_solve(const SceneView& s, const OTRay& r, con
   }
 }
 
+// The root's entry. A root without children is a leaf whatever the level of detail and wherever its data begin
+// (the children field 0 would make it step into its own record and the seven after it).
 __device__ __forceinline__ OTEntry ot_root(const SceneView& s, uint32_t root) {
   const uint32_t children = s.multi_nodes[root].children_offset;
-  return OTEntry{0u, children > 0 ? children - root : 0u, 0u};
+  return children > 0 ? OTEntry{0u, children - root, 0u} : OTEntry{0u, 0u, 0x80u};
 }
 
 // The whole walk of one instance, which stops at the first leaf whose surface is hit. `ot_col`: LDS columns

@@ -1221,7 +1221,9 @@ struct Tracer {
     int top = 0;
     const float old_t = pHit->t;
     const uint32_t root = s.geoms[geomId].offset[0];
-    stack[0] = Elem{root, 0, 0, 0, 0, 1};
+    // a root without children is a leaf (the reference would take nodes 0 to 7 for its children)
+    const bool one_node = s.multi_nodes[root].children_offset == 0;
+    stack[0] = Elem{root, one_node ? s.multi_nodes[root].data_offset : 0u, 0, 0, 0, 1};
     while (top >= 0) {
       Elem& e = stack[top];
       float d = 1.0f / float(e.size);
@@ -1229,7 +1231,7 @@ struct Tracer {
       const f3 t0 = T0 + d * pf * L;
       const f3 t1 = T0 + d * (pf + 1.0f) * L;
       if (std::min(std::min(t1.x, t1.y), t1.z) < tNear) { top--; continue; }
-      bool leaf = e.info > 0;
+      bool leaf = e.info > 0 || one_node;
       if (!leaf) {
         const float t = s.preset.fixed_lod > 0 ? 1.0f : std::max(t0.x, std::max(t0.y, t0.z));
         const float target = (std::pow(2.0f, s.preset.level_of_detail) - 0.01f) / t;

@@ -5,7 +5,7 @@ instance level, graph replay and the allocation-free entry point."""
 import numpy as np
 import pytest
 
-from conftest import raw_equal
+from conftest import assert_sdf_parity, raw_equal, sdf_check
 
 pytestmark = pytest.mark.gpu
 MO_VOXEL_COUNT = 24   # MULTI_RENDER_MODE_MO_VOXEL_COUNT
@@ -437,6 +437,36 @@ def test_multi_octrees(lrt, torch_dev, depth, count, lod, n):
         graph.replay()
         torch.cuda.synchronize()
         assert raw_equal(out.cpu().numpy().view(g.HIT_DTYPE).reshape(-1), hits)
+
+
+@pytest.mark.parametrize("first", [False, True])
+@pytest.mark.parametrize("voxels", [0, 1])
+def test_multi_octree_of_one_node(lrt, orc, torch_dev, first, voxels):
+    """A root without children is a leaf (or empty), as the only octree and behind another one, in the default
+    and the one-ray-a-lane kernels and beside a mesh."""
+    node = np.zeros(1, lrt.MULTI_NODE_DTYPE)
+    node["voxel_count"] = voxels
+    values = np.array([((i >> 2) + (i >> 1 & 1) + (i & 1) - 1.4) * 0.5 for i in range(8)], np.float32)
+    more = lrt.sdf_spheres_multi_octree(np.array([[0.2, 0.1, -0.3, 0.4]], np.float32), 3)
+    for beside in (False, True):
+        def make():
+            s = lrt.SceneRT()
+            if first:
+                s.AddInstance(s.AddGeom_SdfMultiOctree(*more), mats(1, 3, 1.0)[0])
+            s.AddInstance(s.AddGeom_SdfMultiOctree(node, values))
+            if beside:
+                s.AddInstance(s.AddGeom_Triangles3f(*lrt.gen_geodesic(3, 0.05, 4.0, 2)), mats(1, 5, 2.0)[0])
+            s.CommitScene()
+            return s
+        b = Both(lrt, make, tree=False)
+        pos, dirs = random_rays(torch_dev, 20001, 3, extent=2.5)
+        dirs[::11, 0] = 0.0
+        got = b.check(torch_dev, pos, dirs)
+        p, d = pos.cpu().numpy(), dirs.cpu().numpy()
+        want, _ = orc.trace_closest(orc.Scene.from_scene(b.wide), p, d)
+        r = sdf_check(got, want, p, d)
+        assert_sdf_parity(r, got, want)
+        assert bool(((got["geomId"] & lrt.GEOM_ID_MASK) == int(first)).any()) == bool(voxels)
 
 
 @pytest.mark.parametrize("n", [1, 4096, 4097])

@@ -387,3 +387,39 @@ def test_multi_octree_level_of_detail(lrt, orc, camera_batch):
     assert np.sum(a != b) <= 0.002 * a.size
     both = a & b
     assert np.quantile(np.abs(hm["t"][both] - hf["t"][both]), 0.99) < 1e-3 * (2.0 / 32)
+
+
+@pytest.mark.parametrize("first", [False, True])
+@pytest.mark.parametrize("voxels", [0, 1])
+def test_multi_octree_of_one_node(lrt, orc, camera_batch, first, voxels):
+    """A root without children is the whole cube's leaf, as the only octree and behind another one, and an
+    empty one is missed. The values are those of a plane, which the trilinear reproduces."""
+    normal, offset = np.array([0.48, 0.6, 0.64]), 0.2
+    corner = np.array([[(i >> 2) & 1, (i >> 1) & 1, i & 1] for i in range(8)]) * 2.0 - 1.0
+    node = np.zeros(1, lrt.MULTI_NODE_DTYPE)
+    node["voxel_count"] = voxels
+    values = (corner @ normal - offset).astype(np.float32)
+
+    def build(s):
+        if first:
+            s.AddGeom_SdfMultiOctree(*lrt.sdf_spheres_multi_octree(sphere_set(), 3))
+        s.AddInstance(s.AddGeom_SdfMultiOctree(node, values))
+    pos, dir = camera_batch
+    got = orc.trace_closest(orc.Scene.from_scene(host_scene(lrt, build)), pos, dir)[0]
+    p, d = pos[:, :3].astype(np.float64), dir[:, :3].astype(np.float64)
+    # rays that enter the cube on the plane's positive side (the others start in the solid part)
+    a, b = (-1 - p) / d, (1 - p) / d
+    near, far = np.minimum(a, b).max(1), np.maximum(a, b).min(1)
+    t = (offset - p @ normal) / (d @ normal)
+    start = (p + near[:, None] * d) @ normal - offset
+    through = (near < far) & (start > 1e-4) & (t > near) & (t < far - 1e-4)
+    misses = (near > far + 1e-4) | ((start > 1e-4) & ((t < near - 1e-4) | (t > far + 1e-4)))
+    hit = got["primId"] != MISS
+    if not voxels:
+        assert not hit.any()
+        return
+    assert through.sum() > 0.02 * hit.size and hit[through].all() and not hit[misses].any()
+    assert (got["primId"][hit] == 0).all()
+    # the hit lies where the trilinear falls to the walk's stopping distance (at most 1e-6 of the cell's edge) in
+    # fp32 coordinates of a cell of edge 2
+    assert np.abs(got["t"][through] - t[through]).max() < 2e-5
