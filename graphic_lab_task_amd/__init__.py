@@ -156,6 +156,7 @@ TYPE_MESH_TRIANGLE, TYPE_SDF_FRAME_OCTREE, TYPE_SDF_SBS, TYPE_SDF_SBS_COL = 0, 3
 TYPE_SDF_FRAME_OCTREE_TEX = 8
 SH_TYPE, GEOM_ID_MASK = 24, 0x00FFFFFF
 MISS = 0xFFFFFFFF
+WALK_AUTO, WALK_BINARY, WALK_WIDE = -1, 0, 1   # LRT_WALK_* (include/lrt.h)
 NOALLOC_MAX_RAYS = 65536   # LRT_NOALLOC_MAX_RAYS (include/lrt.h)
 SDF_SBS_NODE_LAYOUT_DX = 1 << 24
 SDF_SBS_NODE_LAYOUT_DX_UV16 = 2 << 24
@@ -278,6 +279,11 @@ def lib() -> ctypes.CDLL:
             "lrt_set_persistent": ([vp, i32], i32),
             "lrt_set_tlas_update": ([vp, i32], i32),
             "lrt_get_commit_info": ([vp, ctypes.POINTER(_CommitInfo)], i32),
+            "lrt_set_walk": ([vp, i32], i32),
+            "lrt_get_walk": ([vp, ctypes.POINTER(i32)], i32),
+            "lrt_walk_of_call": ([vp, u64, ctypes.POINTER(i32)], i32),
+            "lrt_sbs_batch_set_walk": ([vp, i32], i32),
+            "lrt_sbs_batch_get_walk": ([vp, ctypes.POINTER(i32)], i32),
             "lrt_autotune": ([vp, vp, vp, vp, u64, vp, vp], i32),
             "lrt_sbs_param_layout": ([vp, u32, ctypes.POINTER(u32), ctypes.POINTER(u32), ctypes.POINTER(u64)], i32),
             "lrt_sbs_forward_dev": ([vp, u32, vp, vp, vp, u64, vp, vp], i32),
@@ -334,6 +340,7 @@ def exported_symbols():
             "lrt_update_instance", "lrt_commit", "lrt_set_preset", "lrt_trace_closest_dev",
             "lrt_trace_closest_host", "lrt_trace_closest_noalloc_dev", "lrt_trace_any_dev", "lrt_trace_closest_counted_dev", "lrt_query_one", "lrt_eye_rays_dev",
             "lrt_set_launch_config", "lrt_set_tail_config", "lrt_set_leaf_postponement", "lrt_set_ray_interleave", "lrt_set_persistent",
+            "lrt_set_walk", "lrt_get_walk", "lrt_walk_of_call", "lrt_sbs_batch_set_walk", "lrt_sbs_batch_get_walk",
             "lrt_set_tlas_update", "lrt_get_commit_info", "lrt_autotune", "lrt_sbs_param_layout",
             "lrt_sbs_forward_dev", "lrt_sbs_backward_dev", "lrt_sbs_l2_backward_dev", "lrt_sbs_render_l2_backward_dev", "lrt_sbs_recompute_misses",
             "lrt_sbs_batch_create", "lrt_sbs_batch_run", "lrt_sbs_batch_autotune", "lrt_sbs_batch_configure", "lrt_sbs_batch_destroy",
@@ -590,11 +597,12 @@ class SceneRT:
                                                    stream))
 
     def autotune(self, pos, dir, hits, stream: int = 0) -> dict:
-        """Times the launch configurations on this device ray batch and keeps the fastest."""
+        """Times the launch configurations on this device ray batch and keeps the fastest ("walk": which walk;
+        the other entries describe the binary one)."""
         n = pos.numel() // 4
         r = _TuneResult()
         _check(lib().lrt_autotune(self._h, _ptr(pos), _ptr(dir), _ptr(hits), n, stream, ctypes.byref(r)))
-        return {f: getattr(r, f) for f, _ in _TuneResult._fields_}
+        return {**{f: getattr(r, f) for f, _ in _TuneResult._fields_}, "walk": self.get_walk()}
 
     # ---- differentiable sparse brick set ----
     def sbs_param_layout(self, geom_id: int):
@@ -652,6 +660,21 @@ class SceneRT:
     def set_persistent(self, on: bool = True):
         """One persistent single-pass kernel with per-lane ray refill (True) or the two-pass grid launch."""
         _check(lib().lrt_set_persistent(self._h, 1 if on else 0))
+
+    def set_walk(self, walk: int = -1):
+        """WALK_AUTO, WALK_BINARY (in the shape set last) or WALK_WIDE (include/lrt.h)."""
+        _check(lib().lrt_set_walk(self._h, walk))
+
+    def get_walk(self) -> int:
+        w = ctypes.c_int32()
+        _check(lib().lrt_get_walk(self._h, ctypes.byref(w)))
+        return w.value
+
+    def walk_of_call(self, n_rays: int) -> int:
+        """The walk (WALK_BINARY or WALK_WIDE) of a closest-hit or any-hit call of n rays."""
+        w = ctypes.c_int32()
+        _check(lib().lrt_walk_of_call(self._h, n_rays, ctypes.byref(w)))
+        return w.value
 
     def set_tlas_update(self, mode: int = 1):
         """Commits after UpdateInstance only: 1 refit the TLAS on the GPU, 0 rebuild it on the host."""
@@ -712,10 +735,20 @@ class SbsBatch:
         _check(lib().lrt_sbs_batch_run(self._h, stream))
 
     def autotune(self, stream: int = 0) -> dict:
-        """Times the batch kernel's shapes on this plan (overwriting its outputs) and keeps the fastest."""
+        """Times the batch kernel's shapes on this plan (overwriting its outputs) and keeps the fastest ("walk":
+        which walk; the other entries describe the binary one)."""
         r = _BatchTuneResult()
         _check(lib().lrt_sbs_batch_autotune(self._h, stream, ctypes.byref(r)))
-        return {f: getattr(r, f) for f, _ in _BatchTuneResult._fields_}
+        return {**{f: getattr(r, f) for f, _ in _BatchTuneResult._fields_}, "walk": self.get_walk()}
+
+    def set_walk(self, walk: int):
+        """WALK_BINARY, or the form on the six-wide walk where every scene has it."""
+        _check(lib().lrt_sbs_batch_set_walk(self._h, walk))
+
+    def get_walk(self) -> int:
+        w = ctypes.c_int32()
+        _check(lib().lrt_sbs_batch_get_walk(self._h, ctypes.byref(w)))
+        return w.value
 
     def configure(self, lds_stack: int, record: int, grid: int):
         """Sets the kernel variant (LDS stack entries, hit-voxel record) and persistent grid."""

@@ -92,8 +92,20 @@ lrt::TraceArgs trace_args(lrt_scene* s, const float* pos, const float* dir, lrt_
   a.postpone_tri = s->s.preset.render_mode != lrt::MULTI_RENDER_MODE_INTERSECTION_COUNT && s->s.postpone_triangles();
   a.persistent = s->s.persistent ? 1u : 0u;
   // (the wide walk visits other leaves, too)
-  a.wide = s->s.wide && s->s.preset.render_mode != lrt::MULTI_RENDER_MODE_INTERSECTION_COUNT && !s->s.rays_crowd(n);
+  a.wide = s->s.preset.render_mode != lrt::MULTI_RENDER_MODE_INTERSECTION_COUNT &&
+           (s->s.walk == LRT_WALK_WIDE || (s->s.walk == LRT_WALK_AUTO && !s->s.rays_crowd(n)));
   return a;
+}
+
+// Whether a closest-hit or any-hit call of n rays takes the wide form, its queue and counters being there.
+bool call_is_wide(lrt_scene* s, uint64_t n) {
+  if (n > 0xFFFFFFFFull) return false;
+  lrt::TraceArgs a = trace_args(s, nullptr, nullptr, nullptr, nullptr, n, nullptr);
+  lrt::TailQueue queue{};
+  uint32_t counters = 0;
+  a.queue = &queue;
+  a.pcount = &counters;
+  return lrt::takes_wide_form(s->s.make_view(), a);
 }
 
 // Host calls of up to this many rays are traced from and into pinned host memory: the kernels read a ray
@@ -210,7 +222,7 @@ lrt_status sbs_diff_common(lrt_scene* s, uint32_t geom_id, const float* params, 
   lrt::SceneView v = s->s.make_view();
   v.sbs_data_f = params;
   v.sbs_mask = nullptr;
-  if (!s->s.wide) v.wide = nullptr;
+  if (s->s.walk == LRT_WALK_BINARY) v.wide = nullptr;
   uint32_t* mask = nullptr;
   e = s->s.mask_for(w, stream, &mask);
   if (e != hipSuccess) return hip_fail(e, "mask buffer");
@@ -684,7 +696,7 @@ lrt_status lrt_set_launch_config(lrt_scene* s, int block, int lds_stack, int xcd
     if (block != 64 && block != 128 && block != 256) return fail(LRT_ERR_INVALID_ARG, "block must be 64, 128 or 256");
     if (lds_stack != 8 && lds_stack != 16 && lds_stack != 32)
       return fail(LRT_ERR_INVALID_ARG, "lds_stack must be 8, 16 or 32");
-    s->s.wide = false;   // a launch shape of the binary walk was asked for
+    s->s.walk = LRT_WALK_BINARY;   // a launch shape of the binary walk was asked for
     s->s.block = block;
     s->s.lds_stack = lds_stack;
     s->s.xcd_remap = xcd_remap ? 1 : 0;
@@ -696,7 +708,7 @@ lrt_status lrt_set_tail_config(lrt_scene* s, uint32_t budget, uint32_t tail_wave
   return guarded([&]() -> lrt_status {
     if (!s) return fail(LRT_ERR_INVALID_ARG, "null scene");
     if (tail_waves > 65536) return fail(LRT_ERR_INVALID_ARG, "tail_waves must be <= 65536");
-    s->s.wide = false;   // a launch shape of the binary walk was asked for
+    s->s.walk = LRT_WALK_BINARY;   // a launch shape of the binary walk was asked for
     s->s.budget = budget;
     s->s.tail_waves = tail_waves ? tail_waves : 1024u;
     return LRT_OK;
@@ -708,7 +720,7 @@ lrt_status lrt_set_ray_interleave(lrt_scene* s, uint32_t lanes_per_group) {
     if (!s) return fail(LRT_ERR_INVALID_ARG, "null scene");
     if (lanes_per_group > 64 || (lanes_per_group & (lanes_per_group - 1)) != 0)
       return fail(LRT_ERR_INVALID_ARG, "lanes_per_group must be 0 or a power of two up to 64");
-    s->s.wide = false;   // a launch shape of the binary walk was asked for
+    s->s.walk = LRT_WALK_BINARY;   // a launch shape of the binary walk was asked for
     s->s.ray_groups = lanes_per_group;
     return LRT_OK;
   });
@@ -718,7 +730,7 @@ lrt_status lrt_set_persistent(lrt_scene* s, int on) {
   return guarded([&]() -> lrt_status {
     if (!s) return fail(LRT_ERR_INVALID_ARG, "null scene");
     if (on != 0 && on != 1) return fail(LRT_ERR_INVALID_ARG, "on must be 0 or 1");
-    s->s.wide = false;   // a launch shape of the binary walk was asked for
+    s->s.walk = LRT_WALK_BINARY;   // a launch shape of the binary walk was asked for
     s->s.persistent = on;
     return LRT_OK;
   });
@@ -728,8 +740,35 @@ lrt_status lrt_set_leaf_postponement(lrt_scene* s, int mode) {
   return guarded([&]() -> lrt_status {
     if (!s) return fail(LRT_ERR_INVALID_ARG, "null scene");
     if (mode < -1 || mode > 1) return fail(LRT_ERR_INVALID_ARG, "mode must be -1, 0 or 1");
-    if (mode >= 0) s->s.wide = false;
+    if (mode >= 0) s->s.walk = LRT_WALK_BINARY;
     s->s.leaf_postpone = mode;
+    return LRT_OK;
+  });
+}
+
+lrt_status lrt_set_walk(lrt_scene* s, int walk) {
+  return guarded([&]() -> lrt_status {
+    if (!s) return fail(LRT_ERR_INVALID_ARG, "null scene");
+    if (walk < LRT_WALK_AUTO || walk > LRT_WALK_WIDE)
+      return fail(LRT_ERR_INVALID_ARG, "walk must be LRT_WALK_AUTO, LRT_WALK_BINARY or LRT_WALK_WIDE");
+    s->s.walk = walk;
+    return LRT_OK;
+  });
+}
+
+lrt_status lrt_get_walk(lrt_scene* s, int* walk) {
+  return guarded([&]() -> lrt_status {
+    if (!s || !walk) return fail(LRT_ERR_INVALID_ARG, "null argument");
+    *walk = s->s.walk;
+    return LRT_OK;
+  });
+}
+
+lrt_status lrt_walk_of_call(lrt_scene* s, uint64_t n, int* walk) {
+  return guarded([&]() -> lrt_status {
+    if (!s || !walk) return fail(LRT_ERR_INVALID_ARG, "null argument");
+    if (!s->s.committed) return fail(LRT_ERR_NOT_COMMITTED, "scene is not committed");
+    *walk = call_is_wide(s, n) ? LRT_WALK_WIDE : LRT_WALK_BINARY;
     return LRT_OK;
   });
 }
@@ -742,8 +781,8 @@ lrt_status lrt_autotune(lrt_scene* s, const float* pos_near, const float* dir_fa
     if (!pos_near || !dir_far || !hits || n == 0) return fail(LRT_ERR_INVALID_ARG, "autotune needs a non-empty ray batch");
     lrt::Scene& sc = s->s;
     const lrt::TuneConfig start{sc.block, sc.lds_stack, sc.xcd_remap, sc.budget, sc.tail_waves,
-                                sc.postpone_triangles() ? 1 : 0, sc.ray_groups, sc.persistent, sc.wide ? 1 : 0};
-    const bool tune_wide = !sc.wideBlocks.empty() || sc.make_view().leaf_kinds == lrt::LK_MULTI;
+                                sc.postpone_triangles() ? 1 : 0, sc.ray_groups, sc.persistent,
+                                sc.walk != LRT_WALK_BINARY ? 1 : 0};
     // the option only exists for triangle-only scenes
     const bool tune_postpone = sc.leaf_kinds() == lrt::LK_TRI;
     auto apply = [&](const lrt::TuneConfig& c) {
@@ -754,7 +793,7 @@ lrt_status lrt_autotune(lrt_scene* s, const float* pos_near, const float* dir_fa
       sc.tail_waves = c.tail_waves;
       sc.ray_groups = c.ray_groups;
       sc.persistent = c.persistent;
-      sc.wide = c.wide != 0;
+      sc.walk = c.wide ? LRT_WALK_WIDE : LRT_WALK_BINARY;   // (explicit: rays_crowd has no say in what is timed)
       if (tune_postpone) sc.leaf_postpone = c.postpone;
     };
     lrt_status st = LRT_OK;
@@ -764,11 +803,15 @@ lrt_status lrt_autotune(lrt_scene* s, const float* pos_near, const float* dir_fa
       return st == LRT_OK ? hipSuccess : hipErrorLaunchFailure;
     };
     lrt::TuneResult r{};
-    const int start_mode = sc.leaf_postpone;
+    const int start_mode = sc.leaf_postpone, start_walk = sc.walk;
+    sc.walk = LRT_WALK_WIDE;
+    const bool tune_wide = call_is_wide(s, n);
+    sc.walk = start_walk;
     const hipError_t e = lrt::autotune(launch, reinterpret_cast<hipStream_t>(stream), start, tune_postpone, tune_wide, 3, &r);
     if (e != hipSuccess) {
       apply(start);
       sc.leaf_postpone = start_mode;
+      sc.walk = start_walk;
       return st != LRT_OK ? st : hip_fail(e, "autotune");
     }
     apply(r.best);
@@ -872,7 +915,7 @@ lrt_status lrt_sbs_batch_create(const lrt_sbs_batch_item* items, uint32_t n_item
       it.view.sbs_data_f = in.params;
       it.view.cache_pairs = 0;
       it.view.cache_geom = 0xFFFFFFFFu;
-      if (!sc.wide) it.view.wide = nullptr;
+      if (sc.walk == LRT_WALK_BINARY) it.view.wide = nullptr;
       it.args.pos = reinterpret_cast<const lrt::float4*>(in.pos_near);
       it.args.dir = reinterpret_cast<const lrt::float4*>(in.dir_far);
       it.args.n = uint32_t(in.n_rays);
@@ -1082,6 +1125,24 @@ lrt_status lrt_sbs_batch_run(lrt_sbs_batch* b, void* stream) {
     if (st != LRT_OK) return st;
     const hipError_t e = lrt::launch_sbs_batch(b->L, reinterpret_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "batch launch");
+    return LRT_OK;
+  });
+}
+
+lrt_status lrt_sbs_batch_set_walk(lrt_sbs_batch* b, int walk) {
+  return guarded([&]() -> lrt_status {
+    if (!b) return fail(LRT_ERR_INVALID_ARG, "null batch");
+    if (walk < LRT_WALK_AUTO || walk > LRT_WALK_WIDE)
+      return fail(LRT_ERR_INVALID_ARG, "walk must be LRT_WALK_AUTO, LRT_WALK_BINARY or LRT_WALK_WIDE");
+    b->L.wide = walk != LRT_WALK_BINARY && b->resident_wide ? 1u : 0u;
+    return LRT_OK;
+  });
+}
+
+lrt_status lrt_sbs_batch_get_walk(lrt_sbs_batch* b, int* walk) {
+  return guarded([&]() -> lrt_status {
+    if (!b || !walk) return fail(LRT_ERR_INVALID_ARG, "null argument");
+    *walk = b->L.wide ? LRT_WALK_WIDE : LRT_WALK_BINARY;
     return LRT_OK;
   });
 }

@@ -162,6 +162,8 @@ hipError_t launch_tlas_refit(BVHNode* tlas, uint32_t n_nodes, const uint32_t* pa
                              uint32_t* counters, hipStream_t stream);
 
 hipError_t launch_trace(const SceneView& s, const TraceArgs& a, hipStream_t stream);
+// Whether launch_trace takes the wide form (the wide walk, or the multi-octree kernel) for a call.
+bool takes_wide_form(const SceneView& s, const TraceArgs& a);
 // Counters by which persistent waves share a batch (wave_rays.h), each in a line of its own behind the
 // persistent kernel's: counter c is word WAVE_COUNTER_AT + c * WAVE_COUNTER_WORDS from there, zero between calls.
 constexpr uint32_t WAVE_COUNTERS = 16, WAVE_COUNTER_WORDS = 64, WAVE_COUNTER_AT = 48;

@@ -8,6 +8,7 @@
 #include <string>
 #include <vector>
 
+#include "../../include/lrt.h"
 #include "bvh_build.h"
 #include "kernels.h"
 #include "scene_view.h"
@@ -114,7 +115,8 @@ struct Scene {
   // Triangle leaf postponement in pass 1: -1 automatic (on for a triangle-only scene with one
   // instance), 0 off, 1 on.
   int leaf_postpone = -1;
-  bool wide = true;     // the six-wide walk where the scene has its tree; off once a launch shape is asked for
+  // LRT_WALK_*: automatic is the wide form where the scene has one and rays_crowd does not hold
+  int walk = LRT_WALK_AUTO;
   int persistent = 0;   // 1: persistent single-pass trace kernel with per-lane ray refill
 
   // BLAS builder: false the host binned SAH, true the GPU linear BVH (build names "gpu...").

@@ -74,10 +74,16 @@ __global__ void k_eye_rays(EyeRayParams prm, const float2* __restrict__ jitter, 
   dir[idx] = make4(rd.x, rd.y, rd.z, 1e9f);
 }
 
+bool takes_wide_form(const SceneView& s, const TraceArgs& a) {
+  if (!a.wide || a.counts || !a.queue || !a.pcount || a.n > WIDE_MAX_RAYS) return false;
+  // (smoothed and tricubic brick sets have kinds of their own)
+  return s.leaf_kinds == LK_MULTI || (s.wide && !(s.leaf_kinds & (LK_SBS_SMOOTH | LK_TRICUBIC)));
+}
+
 hipError_t launch_trace(const SceneView& s, const TraceArgs& a, hipStream_t stream) {
   const uint32_t k = s.leaf_kinds & ~(LK_SBS_SMOOTH | LK_TRICUBIC);
   hipError_t e;
-  if (a.wide && s.wide && k == s.leaf_kinds && !a.counts && a.queue && a.pcount && a.n <= WIDE_MAX_RAYS)
+  if (k != LK_MULTI && takes_wide_form(s, a))
     e = launch_trace_wide(s, a, stream);
   else if (s.leaf_kinds & LK_TRICUBIC)
     e = k == LK_SBS ? launch_trace_sbs_tricubic(s, a, stream) : launch_trace_mixed_tricubic(s, a, stream);

@@ -134,7 +134,7 @@ hipError_t launch_multi_default(const SceneView& s, const TraceArgs& a, hipStrea
 
 // The one-ray-a-lane kernels answer counted calls and launch shapes that the caller chose.
 hipError_t launch_trace_multi(const SceneView& s, const TraceArgs& a, hipStream_t stream) {
-  if (a.wide && !a.counts && a.pcount && a.n <= WIDE_MAX_RAYS) return launch_multi_default(s, a, stream);
+  if (takes_wide_form(s, a)) return launch_multi_default(s, a, stream);
   return launch_kinds<LK_MULTI>(s, a, stream);
 }
 

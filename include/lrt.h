@@ -287,14 +287,29 @@ lrt_status lrt_query_one(lrt_scene* s, const float* pos_near4, const float* dir_
 lrt_status lrt_eye_rays_dev(const float* proj_inv16, const float* world_view_inv16, uint32_t width, uint32_t height,
                             const float* jitter, uint32_t order, float* pos_near, float* dir_far, void* stream);
 
-/* Scenes of triangle meshes, and scenes of one frame-octree or sparse-voxel-set instance, are traced by
- * a six-wide walk built at commit that has no launch shape to choose, scenes of multi-octrees by a kernel
- * that has none either (other scenes, counted calls and the INTERSECTION_COUNT mode take the binary walk). Each of the launch-shape calls below
- * (lrt_set_launch_config, lrt_set_tail_config, lrt_set_leaf_postponement with 0 or 1,
+/* Scenes of triangle meshes, and scenes of one instance of a frame octree, sparse voxel set or sparse brick
+ * set, are traced by a six-wide walk built at commit that has no launch shape to choose, scenes of
+ * multi-octrees by a kernel that has none either: the wide form. Other scenes, counted calls and the
+ * INTERSECTION_COUNT mode take the binary walk, and so, by default, do large batches (65,536 rays or more) into one small
+ * mesh or brick set (128 rays a triangle, 1,024 a brick), which it is faster on. Each of the launch-shape
+ * calls below (lrt_set_launch_config, lrt_set_tail_config, lrt_set_leaf_postponement with 0 or 1,
  * lrt_set_ray_interleave, lrt_set_persistent) moves the scene to the binary walk in that shape;
- * lrt_autotune tries both and keeps the faster. Same hit records either way.
+ * lrt_autotune tries both and keeps the faster for every batch; lrt_set_walk chooses. Same hit records
+ * either way.
  *
- * Kernel configuration used by the trace calls: block size (64/128/256), number of traversal
+ * lrt_set_walk: LRT_WALK_AUTO (the default, as above), LRT_WALK_BINARY (in the shape set last), or
+ * LRT_WALK_WIDE (the wide form for batches of any size, where the scene has one). The differentiable calls
+ * take the wide form, where it applies, unless the walk is LRT_WALK_BINARY. lrt_get_walk: the setting,
+ * which lrt_autotune leaves at WIDE or BINARY: a tuned configuration is stored as its lrt_tune_result and
+ * this, and restored by the launch-shape calls and then lrt_set_walk. lrt_walk_of_call: the walk (BINARY or
+ * WIDE) that a closest-hit or any-hit call of n rays into the committed scene takes, with the present
+ * setting and preset. No counterparts in the reference. */
+enum { LRT_WALK_AUTO = -1, LRT_WALK_BINARY = 0, LRT_WALK_WIDE = 1 };
+lrt_status lrt_set_walk(lrt_scene* s, int walk);
+lrt_status lrt_get_walk(lrt_scene* s, int* walk);
+lrt_status lrt_walk_of_call(lrt_scene* s, uint64_t n, int* walk);
+
+/* Kernel configuration used by the trace calls: block size (64/128/256), number of traversal
  * stack entries kept in LDS (8/16/32), XCD-contiguous block mapping (0/1). */
 lrt_status lrt_set_launch_config(lrt_scene* s, int block, int lds_stack, int xcd_remap);
 
@@ -398,12 +413,18 @@ lrt_status lrt_sbs_batch_autotune(lrt_sbs_batch* b, void* stream, lrt_sbs_batch_
  * reported earlier) and moves the plan to the binary walk: lds_stack 8, 16 or 32, record 0 or 1, grid
  * 1 .. the variant's resident blocks. No counterpart in the reference. */
 lrt_status lrt_sbs_batch_configure(lrt_sbs_batch* b, int lds_stack, int record, uint32_t grid);
+/* The walk of a plan: LRT_WALK_BINARY, in the shape set last, or (AUTO or WIDE) the form on the six-wide walk
+ * where every scene has it, which is a new plan's default. lrt_sbs_batch_get_walk: WIDE or BINARY, which
+ * with the shape is the whole configuration that lrt_sbs_batch_autotune chose. */
+lrt_status lrt_sbs_batch_set_walk(lrt_sbs_batch* b, int walk);
+lrt_status lrt_sbs_batch_get_walk(lrt_sbs_batch* b, int* walk);
 lrt_status lrt_sbs_batch_destroy(lrt_sbs_batch* b);
 
 /* Rays whose recomputed hit voxel did not reproduce the walk's hit (expected 0). */
 lrt_status lrt_sbs_recompute_misses(lrt_scene* s, uint64_t* out, int reset);
 
-/* Result of lrt_autotune. */
+/* Result of lrt_autotune: the shape of the binary walk. Where the wide form was the fastest (lrt_get_walk
+ * then gives LRT_WALK_WIDE) best_ms is its time and the shape is the one the scene had before. */
 typedef struct lrt_tune_result {
   int32_t block, lds_stack, xcd_remap;
   uint32_t budget, tail_waves;

@@ -144,3 +144,25 @@ def test_differentiable_calls_refuse_mixed_scenes(lrt):
     with pytest.raises(lrt.LrtError) as e:
         mixed.sbs_param_layout(0)
     assert e.value.code == 4 and "brick sets" in str(e.value)
+
+
+def test_walk_setting(lrt):
+    """The walk of a scene: automatic at first, binary once a launch shape is asked for, and back."""
+    s = lrt.SceneRT()
+    assert s.get_walk() == lrt.WALK_AUTO
+    for shape in (lambda: s.set_launch_config(256, 16, True), lambda: s.set_tail_config(64, 1024),
+                  lambda: s.set_ray_interleave(32), lambda: s.set_persistent(False),
+                  lambda: s.set_leaf_postponement(1)):
+        s.set_walk(lrt.WALK_WIDE)
+        assert s.get_walk() == lrt.WALK_WIDE
+        shape()
+        assert s.get_walk() == lrt.WALK_BINARY
+    s.set_leaf_postponement(-1)
+    assert s.get_walk() == lrt.WALK_BINARY
+    s.set_walk()
+    assert s.get_walk() == lrt.WALK_AUTO
+    for bad in (-2, 2):
+        with pytest.raises(lrt.LrtError):
+            s.set_walk(bad)
+    with pytest.raises(lrt.LrtError):   # not committed
+        s.walk_of_call(1)

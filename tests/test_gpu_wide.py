@@ -388,6 +388,18 @@ def test_batch_forms_agree(lrt, torch_dev):
         assert torch.equal(a[0], b[0])
         for x, y in zip(a[1:], b[1:]):
             assert float((x - y).norm()) <= 1e-5 * float(y.norm()) + 1e-12
+    batch.set_walk(lrt.WALK_WIDE)
+    assert batch.get_walk() == lrt.WALK_BINARY   # the plan of scenes on the binary walk has no other
+    for it in items:
+        it["scene"].set_walk(lrt.WALK_AUTO)
+    batch = lrt.SbsBatch(items)
+    assert batch.get_walk() == lrt.WALK_WIDE
+    r = batch.autotune()
+    assert r["walk"] == batch.get_walk()
+    batch.configure(r["lds_stack"], r["record"], r["grid"])
+    assert batch.get_walk() == lrt.WALK_BINARY
+    batch.set_walk(r["walk"])
+    assert batch.get_walk() == r["walk"]
 
 
 @pytest.mark.parametrize("depth,count,lod,n", [(2, 1, 0.0, 1), (3, 2, 0.0, 63), (6, 1, 3.0, 70000), (7, 3, 0.0, 100001),
@@ -437,6 +449,55 @@ def test_multi_octrees(lrt, torch_dev, depth, count, lod, n):
         graph.replay()
         torch.cuda.synchronize()
         assert raw_equal(out.cpu().numpy().view(g.HIT_DTYPE).reshape(-1), hits)
+
+
+# the lines of Scene::rays_crowd: 65,536 rays, 128 a triangle, 1,024 a brick
+@pytest.mark.parametrize("kind,size,line", [("mesh", 1, 65536), ("mesh", 6, 92160), ("bricks", 2, 65536)])
+def test_crowded_batches(lrt, torch_dev, kind, size, line):
+    """Both sides of the line where default calls leave the wide walk, and batches beyond it with the walk set."""
+    b = Both(lrt, mesh(lrt, size) if kind == "mesh" else brick_scene(lrt, size, 1, 1))
+    for n in (line - 1, line):
+        assert b.wide.walk_of_call(n) == (lrt.WALK_WIDE if n < line else lrt.WALK_BINARY)
+        pos, dirs = random_rays(torch_dev, n, 1)
+        b.check(torch_dev, pos, dirs)
+    b.wide.set_walk(lrt.WALK_WIDE)
+    assert b.wide.walk_of_call(line) == lrt.WALK_WIDE
+    b.check(torch_dev, pos, dirs)
+
+
+@pytest.mark.parametrize("kind", ["crowded mesh", "instances", "multi", "mixed"])
+def test_tuned_walk_is_kept(lrt, torch_dev, kind):
+    """The tuner times the walk it names and a scene of the same make takes its result over: shape, then walk."""
+    torch = torch_dev
+
+    def make():
+        s = lrt.SceneRT()
+        if kind in ("multi", "mixed"):
+            s.AddInstance(s.AddGeom_SdfMultiOctree(*lrt.sdf_spheres_multi_octree(
+                np.array([[0.2, 0.1, -0.3, 0.4], [-0.3, 0.1, 0.3, 0.3]], np.float32), 4)))
+        if kind != "multi":
+            gid = s.AddGeom_Triangles3f(*lrt.gen_geodesic(2, 0.05, 4.0, 2))
+            for m in mats(9 if kind == "instances" else 1, 4, 2.0):
+                s.AddInstance(gid, m)
+        s.CommitScene()
+        return s
+    n = 70001
+    pos, dirs = random_rays(torch, n, 2, extent=2.5)
+    s, other = make(), make()
+    assert (s.walk_of_call(n) == lrt.WALK_WIDE) == (kind in ("instances", "multi"))
+    want = trace(torch, lrt, s, pos, dirs)
+    hits = torch.zeros((n, 8), dtype=torch.int32, device="cuda")
+    r = s.autotune(pos, dirs, hits)
+    assert r["walk"] == s.get_walk() == s.walk_of_call(n) != lrt.WALK_AUTO
+    assert kind != "mixed" or r["walk"] == lrt.WALK_BINARY
+    other.set_launch_config(r["block"], r["lds_stack"], bool(r["xcd_remap"]))
+    other.set_tail_config(r["budget"], r["tail_waves"])
+    other.set_ray_interleave(r["ray_interleave"])
+    other.set_persistent(bool(r["persistent"]))
+    other.set_walk(r["walk"])
+    assert other.walk_of_call(n) == r["walk"]
+    for x in (s, other):
+        assert raw_equal(trace(torch, lrt, x, pos, dirs), want)
 
 
 @pytest.mark.parametrize("first", [False, True])
