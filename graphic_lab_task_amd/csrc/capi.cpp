@@ -110,9 +110,10 @@ bool call_is_wide(lrt_scene* s, uint64_t n) {
 
 // Host calls of up to this many rays are traced from and into pinned host memory: the kernels read a ray
 // and write a record of 32 bytes each over the bus, while each of the three copies of the general way takes
-// about 10 us whatever its size. Into 81,920 triangles: 1 ray 46 -> 22 us, 256 rays 71 -> 50, 4,096 rays 95 ->
-// 86. Beyond, the gain shrinks (16,384 rays: 145 -> 121) and the pinned memory (64 bytes a ray) grows.
-constexpr uint64_t HOST_PINNED_RAYS = 4096;
+// about 10 us whatever its size. lrt_trace_closest_host on 81,920 triangles, called from C: 1 ray 46 -> 22 us,
+// 256 rays 71 -> 50, 4,096 rays 95 -> 86 (a pick through the Python package 72 -> 38). Beyond, the gain shrinks
+// (16,384 rays: 145 -> 121) and the pinned memory (64 bytes a ray) grows.
+constexpr uint64_t HOST_PINNED_RAYS = lrt::PINNED_BYTES / 64;   // 4,096
 
 // Queries this library does not answer: tricubic interpolation of a brick set without padding
 // (the 4^3 samples start one voxel before the brick, BVH2Common.cpp:790-844: the reference reads
@@ -538,13 +539,9 @@ lrt_status lrt_trace_closest_host(lrt_scene* s, const float* pos_near, const flo
     lrt::DevBuf& io = s->s.host_io;
     hipError_t e;
     if (n <= HOST_PINNED_RAYS) {
-      void*& mem = s->s.host_pinned;
-      if (!mem && hipHostMalloc(&mem, HOST_PINNED_RAYS * 64, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
-        mem = nullptr;
-        (void)hipGetLastError();   // the copies below do without
-      }
-      if (mem) {
-        char* base = static_cast<char*>(mem);
+      const lrt::PinnedBlock mem;
+      if (mem.ptr()) {   // (the copies below do without)
+        char* base = static_cast<char*>(mem.ptr());
         std::memcpy(base, pos_near, n * 16);
         std::memcpy(base + n * 16, dir_far, n * 16);
         const lrt_status st = trace_common(s, reinterpret_cast<float*>(base), reinterpret_cast<float*>(base + n * 16),

@@ -77,11 +77,65 @@ hipError_t Scene::work_for(StreamWork& w, void* stream, size_t n, uint32_t** spi
   return hipSuccess;
 }
 
+namespace {
+struct PinnedPool {
+  std::mutex mu;
+  std::vector<void*> kept;   // has room for one a scene
+  size_t n_scenes = 0;
+};
+// never destroyed: a scene may outlive the static objects of the library
+PinnedPool& pinned_pool() {
+  static PinnedPool* p = new PinnedPool;
+  return *p;
+}
+}  // namespace
+
+PinnedBlock::PinnedBlock() {
+  PinnedPool& pool = pinned_pool();
+  {
+    std::lock_guard<std::mutex> lock(pool.mu);
+    if (!pool.kept.empty()) {
+      p_ = pool.kept.back();
+      pool.kept.pop_back();
+    }
+  }
+  if (!p_ && hipHostMalloc(&p_, PINNED_BYTES, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
+    p_ = nullptr;
+    (void)hipGetLastError();
+  }
+}
+
+PinnedBlock::~PinnedBlock() {
+  if (!p_) return;
+  PinnedPool& pool = pinned_pool();
+  {
+    std::lock_guard<std::mutex> lock(pool.mu);
+    if (pool.kept.size() < pool.n_scenes) {
+      pool.kept.push_back(p_);
+      return;
+    }
+  }
+  (void)hipHostFree(p_);
+}
+
+Scene::Scene() {
+  PinnedPool& pool = pinned_pool();
+  std::lock_guard<std::mutex> lock(pool.mu);
+  pool.kept.reserve(pool.n_scenes + 1);
+  ++pool.n_scenes;
+}
+
 Scene::~Scene() {
   work.clear();
   dev.clear();
   if (d_overflow) (void)hipFree(d_overflow);
-  if (host_pinned) (void)hipHostFree(host_pinned);
+  PinnedPool& pool = pinned_pool();
+  std::lock_guard<std::mutex> lock(pool.mu);
+  --pool.n_scenes;
+  while (pool.kept.size() > pool.n_scenes) {
+    (void)hipHostFree(pool.kept.back());
+    pool.kept.pop_back();
+  }
 }
 
 namespace {

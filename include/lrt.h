@@ -216,9 +216,9 @@ lrt_status lrt_trace_closest_dev(lrt_scene* s, const float* pos_near, const floa
 lrt_status lrt_trace_closest_noalloc_dev(lrt_scene* s, const float* pos_near, const float* dir_far, lrt_hit* hits,
                                          uint64_t n, void* stream);
 
-/* Same over host buffers (copies in, traces, copies out, synchronises). The staging buffers (pinned
- * host memory for up to 4096 rays, device memory for more) belong to the scene and only grow:
- * repeated calls of one size allocate nothing. */
+/* Same over host buffers (copies in, traces, copies out, synchronises). The staging buffers
+ * only grow, so repeated calls of one size allocate nothing: pinned host memory for up to 4096 rays, from a
+ * pool of the process with at most one block of 256 KB per scene, and device memory of the scene for more. */
 lrt_status lrt_trace_closest_host(lrt_scene* s, const float* pos_near, const float* dir_far, lrt_hit* hits,
                                   uint64_t n);
 
@@ -274,7 +274,7 @@ lrt_status lrt_resolve_dev(lrt_scene* s, const lrt_hit* gbuffer, const lrt_resol
 lrt_status lrt_tonemap_dev(const float* colour, uint64_t n, uint32_t sample_count, uint32_t* rgba8, void* stream);
 
 /* Single-ray RayQuery_NearestHit for picking (demo_app/plugins/MRFull/execute_commands.cpp:189);
- * runs the same gfx950 kernel on one ray and synchronises. Uses the scene's staging buffer of
+ * runs the same gfx950 kernel on one ray and synchronises. Uses the staging memory of
  * lrt_trace_closest_host: after the first call, a picking loop allocates nothing. */
 lrt_status lrt_query_one(lrt_scene* s, const float* pos_near4, const float* dir_far4, lrt_hit* out);
 

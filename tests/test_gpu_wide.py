@@ -538,3 +538,30 @@ def test_host_staging(lrt, torch_dev, n):
     want = trace(torch_dev, lrt, s, pos, dirs)
     for _ in range(2):
         assert raw_equal(s.trace_closest_host(pos.cpu().numpy(), dirs.cpu().numpy()), want)
+
+
+def test_host_staging_across_scenes_and_threads(lrt, torch_dev):
+    """Scenes that come and go share the staging memory of host calls, one block a call: threads on scenes of
+    their own, on one scene, and calls after most scenes are gone give the device call's records."""
+    import threading
+    pos, dirs = random_rays(torch_dev, 300, 3)
+    p, d = pos.cpu().numpy(), dirs.cpu().numpy()
+    scenes = [mesh(lrt, 3 + k)() for k in range(6)]
+    want = [trace(torch_dev, lrt, s, pos, dirs) for s in scenes]
+    bad = []
+
+    def work(k, own):
+        for r in range(20):
+            s = mesh(lrt, 3 + k)() if own else scenes[k]
+            if not raw_equal(s.trace_closest_host(p, d), want[k]):
+                bad.append((k, own, r))
+    threads = [threading.Thread(target=work, args=(k % 6, k % 4 == 3)) for k in range(12)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+    del scenes[1:]
+    assert raw_equal(scenes[0].trace_closest_host(p, d), want[0])
+    scenes.clear()   # the last scene gives the memory back
+    assert raw_equal(mesh(lrt, 4)().trace_closest_host(p, d), want[1])
