@@ -1199,11 +1199,16 @@ lrt_status lrt_get_array(lrt_scene* s, const char* name, void* dst, size_t* byte
         s->s.build_device_layout();
         s->s.build_wide();
       }
-      wide_copy = c.wideBlocks;
+      wide_copy.resize(c.wideCount);
       if (c.committed && !wide_copy.empty()) {
         const hipError_t e = hipMemcpy(wide_copy.data(), c.dev.at("wide").ptr(), wide_copy.size() * sizeof(lrt::WideBlock),
                                        hipMemcpyDeviceToHost);
         if (e != hipSuccess) return hip_fail(e, "wide tree copy");
+      } else if (c.wideBuild) {
+        std::copy_n(c.wideBuild.get(), wide_copy.size(), wide_copy.begin());
+        s->s.wideBuild.reset();
+      } else {
+        wide_copy.clear();
       }
       if (n == "wide_blocks") { src = wide_copy.data(); sz = wide_copy.size() * sizeof(lrt::WideBlock); }
       else { src = &c.wideRoot; sz = sizeof(c.wideRoot); }

@@ -785,18 +785,18 @@ hipError_t Scene::commit_instances() {
     if (e != hipSuccess) return e;
     lastCommitKind = 2;
   }
-  if (!wideBlocks.empty()) {
+  if (wideCount) {
     WideBlock* blocks = static_cast<WideBlock*>(dev["wide"].ptr());
     if (rebuild) {
       uint32_t levels = 0;
       if (build_wide_instances(&levels) && levels + wideBlasLevels <= WIDE_MAX_LEVELS) {
         wideLevels = levels + wideBlasLevels;
-        e = hipMemcpy(blocks, wideBlocks.data(), 3 * instances.size() * sizeof(WideBlock), hipMemcpyHostToDevice);
+        e = hipMemcpy(blocks, wideTop.data(), wideTop.size() * sizeof(WideBlock), hipMemcpyHostToDevice);
         if (e != hipSuccess) return e;
         e = dev["wide_sources"].upload(wideSources.data(), wideSources.size() * sizeof(uint32_t));
         if (e != hipSuccess) return e;
       } else {
-        wideBlocks.clear();
+        wideCount = 0;
       }
     } else {
       e = launch_wide_refit(blocks, uint32_t(wideSources.size() / WIDE_CHILDREN),
@@ -966,7 +966,15 @@ hipError_t Scene::commit() {
 #define UP(name, vec)                                                        \
   e = dev[name].upload(vec.data(), vec.size() * sizeof(vec[0]));             \
   if (e != hipSuccess) return e;
-  UP("wide", wideBlocks) UP("wide_sources", wideSources)
+  e = dev["wide"].upload(wideBuild.get(), wideCount * sizeof(WideBlock));
+  wideBuild.reset();
+  if (e == hipErrorOutOfMemory) {   // the binary walk does without
+    (void)hipGetLastError();
+    wideCount = 0;
+  } else if (e != hipSuccess) {
+    return e;
+  }
+  UP("wide_sources", wideSources)
   UP("nodes", devNodes) UP("tri_soup", triSoup) UP("frame_leaves", frameLeaves) UP("frame_tex", frameTex) UP("tlas", tlas) UP("instances", instances) UP("geoms", geomData) UP("geom_tags", geomTags)
   UP("start_end", startEnd) UP("prim_id_count", primIdCount) UP("vert_pos", vertPos) UP("vert_norm", vertNorm)
   UP("indices", indices) UP("prim_indices", primIndices) UP("orig_nodes", origNodes) UP("frame_nodes", frameNodes)
@@ -1020,7 +1028,7 @@ SceneView Scene::make_view() const {
   v.tri_soup = (const float4*)P("tri_soup");
   v.frame_leaves = (const FrameLeaf*)P("frame_leaves");
   v.frame_tex = (const float4*)P("frame_tex");
-  v.wide = wideBlocks.empty() ? nullptr : (const WideBlock*)P("wide");
+  v.wide = wideCount == 0 ? nullptr : (const WideBlock*)P("wide");
   v.wide_root = wideRoot;
   v.wide_levels = wideLevels;
   v.instances = (const InstanceData*)P("instances");

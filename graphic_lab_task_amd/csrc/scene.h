@@ -39,7 +39,6 @@ class DevBuf {
   size_t used_ = 0;
 };
 
-// Mirrors the member arrays of BVHRT (MultiRenderer/BVH2Common.h:262-365).
 // Pinned host memory for the rays and records of one small host call, from a pool of the process. With a block of
 // its own a scene paid for pinning and unpinning: 20,480 triangles, first pick 108 us and the scene's end 75 us, 60
 // and 16 with a block of the pool. A call holds a block while it runs, and a scene runs one such call at a time;
@@ -57,6 +56,7 @@ class PinnedBlock {
   void* p_ = nullptr;
 };
 
+// Mirrors the member arrays of BVHRT (MultiRenderer/BVH2Common.h:262-365).
 struct Scene {
   std::string build_name, layout_name;
   int prims_in_leaf = 2;
@@ -114,9 +114,12 @@ struct Scene {
   std::vector<FrameLeaf> frameLeaves;
   std::vector<float4> frameTex;      // 4 float4 per textured frame-octree leaf
   uint32_t cacheGeom = 0xFFFFFFFFu, cachePairs = 0;
-  // Six-wide tree (wide_bvh.h): three blocks per instance for the instance level, then the
-  // geometries; empty where the wide walk does not apply.
-  std::vector<WideBlock> wideBlocks;
+  // Six-wide tree (wide_bvh.h): wideCount blocks on the device, none where the wide walk does not apply.
+  // Three per instance for the instance level, which stays here in wideTop for later instance trees, then the
+  // geometries. wideBuild holds all of them between build_wide and the upload.
+  size_t wideCount = 0;
+  std::vector<WideBlock> wideTop;
+  std::unique_ptr<WideBlock[]> wideBuild;
   std::vector<uint32_t> wideSources;   // six TLAS node indices per block of the instance level
   std::vector<uint32_t> wideRoots;     // per geometry
   uint32_t wideRoot = 0, wideBlasLevels = 0, wideLevels = 0;
@@ -217,6 +220,7 @@ struct Scene {
   void update_cache_geom();
   void build_device_layout();
   void build_wide();
+  bool build_wide_tree();
   bool build_wide_instances(uint32_t* levels);
   hipError_t commit(); // device upload of every array
   void set_preset(const MultiRenderPreset& p);

@@ -1,6 +1,10 @@
-// Host collapse of the binary trees into the six-wide layout of wide_bvh.h.
+// Host collapse of the binary trees into the six-wide layout of wide_bvh.h, at every commit of new geometry:
+// subtrees are collapsed in parallel and each is copied to its place once. Commits with and without the tree, on 16
+// cores: 327,680 triangles 13.6 and 7.3 ms (33.7 when subtrees were appended one by one, moved again and kept),
+// 20,480 triangles 1.0 and 0.47, 1,280 triangles 0.44 and 0.30.
 #include <algorithm>
 #include <cstring>
+#include <new>
 
 #include "scene.h"
 #include "wide_bvh.h"
@@ -33,6 +37,36 @@ float half_area(float3 mn, float3 mx) {
 bool contains(float3 mn, float3 mx, const BVHNode& c) {
   return c.boxMin.x >= mn.x && c.boxMin.y >= mn.y && c.boxMin.z >= mn.z && c.boxMax.x <= mx.x && c.boxMax.y <= mx.y &&
          c.boxMax.z <= mx.z;
+}
+
+// A collapsed tree: its top, and subtrees whose own blocks follow it one subtree after the other. Child indices
+// count from the top's first block in the top and from a subtree's own first block in the subtree.
+struct Subtree {
+  Blocks blocks;
+  std::vector<uint32_t> nodes;   // places of the nodes among the blocks (the first is the root, which has none)
+  WideNode root;
+  uint32_t at = 0;               // the root's place in the top
+};
+struct Collapsed {
+  Blocks top;
+  std::vector<uint32_t> top_nodes;
+  std::vector<Subtree> subs;
+  size_t size() const {
+    size_t n = top.size();
+    for (const Subtree& s : subs) n += s.blocks.size();
+    return n;
+  }
+};
+
+// Copies a part's blocks to their place and makes the child indices of its nodes count from block 0 of the tree.
+void place(const Blocks& from, const std::vector<uint32_t>& nodes, size_t skip, WideBlock* tree, uint32_t base) {
+  std::copy(from.begin(), from.end(), tree + base);
+  for (size_t k = skip; k < nodes.size(); ++k) {
+    WideNode n;
+    std::memcpy(&n, tree + base + nodes[k], sizeof(n));
+    n.children += base;
+    std::memcpy(tree + base + nodes[k], &n, sizeof(n));
+  }
 }
 
 // One tree's collapse. Tree opens an inner word into its two binary children; Leaf gives the blocks of a
@@ -121,77 +155,54 @@ struct Collapse {
     return true;
   }
 
-  // The tree of `root` (its node becomes block 0 of `out`): the top breadth first until there are
-  // enough subtrees for the cores, then each subtree depth first into blocks of its own, appended in
-  // order, so that a subtree's blocks stay together.
-  bool run(Blocks& out, uint32_t* max_level, std::vector<uint32_t>* sources) const {
+  // The tree: its root is block 0 of `out.top`. The top is built breadth first until there are enough subtrees
+  // for the cores, then each subtree depth first into blocks of its own, so that a subtree's blocks stay together.
+  bool run(Collapsed& out, uint32_t* max_level, std::vector<uint32_t>* sources) const {
     const float inf = 3e38f;
     std::vector<Item> todo{Item{0u, 0u, 1u, 0u, make3(-inf, -inf, -inf), make3(inf, inf, inf)}};
-    out.assign(1, WideBlock{});
+    out.top.assign(1, WideBlock{});
     if (sources) sources->assign(WIDE_CHILDREN, 0xFFFFFFFFu);
     *max_level = 1;
     size_t at = 0;
     while (at < todo.size() && (sources || todo.size() - at < 256)) {
       const Item it = todo[at++];
       WideNode node;
-      if (!expand(it, out, &node, todo, max_level, sources)) return false;
-      std::memcpy(&out[it.block], &node, sizeof(node));
+      if (!expand(it, out.top, &node, todo, max_level, sources)) return false;
+      std::memcpy(&out.top[it.block], &node, sizeof(node));
+      out.top_nodes.push_back(it.block);
     }
     const int n_sub = int(todo.size() - at);
-    struct Sub {
-      Blocks blocks;
-      WideNode root;
-      uint32_t levels = 0;
-      bool ok = true;
-    };
-    std::vector<Sub> subs(size_t(n_sub) > 0 ? size_t(n_sub) : 0);
+    out.subs.resize(size_t(n_sub));
+    std::vector<uint32_t> levels(size_t(n_sub), 0u);
+    bool ok = true;
 #pragma omp parallel for schedule(dynamic, 1)
     for (int k = 0; k < n_sub; ++k) {
-      Sub& s = subs[size_t(k)];
-      std::vector<Item> stack{todo[at + size_t(k)]};
-      bool first = true;
-      while (s.ok && !stack.empty()) {
-        const Item it = stack.back();
-        stack.pop_back();
-        WideNode node;
-        s.ok = expand(it, s.blocks, &node, stack, &s.levels, nullptr);
-        if (first) s.root = node;
-        else if (s.ok) std::memcpy(&s.blocks[it.block], &node, sizeof(node));
-        first = false;
-      }
-    }
-    for (int k = 0; k < n_sub; ++k) {
-      Sub& s = subs[size_t(k)];
-      if (!s.ok || out.size() + s.blocks.size() >= WIDE_MAX_BLOCKS) return false;
-      const uint32_t base = uint32_t(out.size());
-      s.root.children += base;
-      std::memcpy(&out[todo[at + size_t(k)].block], &s.root, sizeof(s.root));
-      *max_level = std::max(*max_level, s.levels);
-      shift(s.blocks, s.root, base);
-      out.insert(out.end(), s.blocks.begin(), s.blocks.end());
-      s.blocks = Blocks();
-    }
-    return true;
-  }
-
-  // Adds `base` to the child indices of every node below `root`, whose own index is already moved.
-  static void shift(Blocks& blocks, const WideNode& root, uint32_t base) {
-    std::vector<WideNode> stack{root};
-    while (!stack.empty()) {
-      const WideNode n = stack.back();
-      stack.pop_back();
-      uint32_t b = (n.children & (WIDE_MAX_BLOCKS - 1)) - base;
-      for (uint32_t k = 0; k < (n.sizes >> 12); ++k) {
-        if (!(n.children >> (26 + k) & 1u)) {
-          WideNode c;
-          std::memcpy(&c, &blocks[b], sizeof(c));
-          c.children += base;
-          std::memcpy(&blocks[b], &c, sizeof(c));
-          stack.push_back(c);
+      Subtree& s = out.subs[size_t(k)];
+      bool good = true;
+      try {   // (nothing may leave the loop's threads)
+        std::vector<Item> stack{todo[at + size_t(k)]};
+        s.at = stack[0].block;
+        while (good && !stack.empty()) {
+          const Item it = stack.back();
+          stack.pop_back();
+          WideNode node;
+          const bool first = s.nodes.empty();
+          good = expand(it, s.blocks, &node, stack, &levels[size_t(k)], nullptr);
+          if (!good) break;
+          if (first) s.root = node;
+          else std::memcpy(&s.blocks[it.block], &node, sizeof(node));
+          s.nodes.push_back(it.block);
         }
-        b += (n.sizes >> (2 * k) & 3u) + 1;
+      } catch (const std::bad_alloc&) {
+        good = false;
       }
+      if (!good)
+#pragma omp atomic write
+        ok = false;
     }
+    if (!ok) return false;
+    for (uint32_t l : levels) *max_level = std::max(*max_level, l);
+    return out.size() < WIDE_MAX_BLOCKS;
   }
 };
 
@@ -288,12 +299,39 @@ namespace {
 // counts triangles: the rank is the index of the leaf's first one), and left.escapeIndex 1 where no plane
 // separates the two sides. `order` takes a box leaf's rank and the topmost such pair above it. False where
 // a mesh's triangle indices do not grow from left to right.
-bool mark_order(BVHNodePair* pairs, uint32_t n, bool mesh, std::vector<LeafOrder>& order) {
+bool apart(const BVHNode& l, const BVHNode& r) {
+  return l.leftOffset == LEAF_NORMAL || r.leftOffset == LEAF_NORMAL || l.boxMax.x <= r.boxMin.x || r.boxMax.x <= l.boxMin.x ||
+         l.boxMax.y <= r.boxMin.y || r.boxMax.y <= l.boxMin.y || l.boxMax.z <= r.boxMin.z || r.boxMax.z <= l.boxMin.z;
+}
+
+bool mark_mesh_order(BVHNodePair* pairs, uint32_t n) {
+  // per pair the first triangle below it and the one after the last: an empty side has neither
+  std::vector<uint2> span(n);
+  auto of = [&](const BVHNode& c, uint32_t empty) {
+    if (c.leftOffset == LEAF_NORMAL) return uint2{empty, empty};
+    if (c.leftOffset & LEAF_BIT) return uint2{extract_start(c.leftOffset), extract_start(c.leftOffset) + extract_count(c.leftOffset)};
+    return span[c.leftOffset];
+  };
+  // children are stored after their parent
+  for (uint32_t p = n; p-- > 0;) {
+    BVHNode &l = pairs[p].left, &r = pairs[p].right;
+    for (const BVHNode* c : {&l, &r})
+      if (!(c->leftOffset & LEAF_BIT) && (c->leftOffset <= p || c->leftOffset >= n)) return false;
+    const uint2 right = of(r, l.leftOffset == LEAF_NORMAL ? 0u : of(l, 0u).y);
+    const uint2 left = of(l, right.x);
+    if (left.y != right.x) return false;
+    span[p] = uint2{left.x, right.y};
+    r.escapeIndex = right.x;
+    l.escapeIndex = apart(l, r) ? 0u : 1u;
+  }
+  return n == 0 || span[0].x == 0;
+}
+
+bool mark_leaf_order(BVHNodePair* pairs, uint32_t n, std::vector<LeafOrder>& order) {
   std::vector<uint32_t> count(n, 0u), first(n, 0u), above(n, WIDE_NO_OVERLAP);
   auto leaves = [&](const BVHNode& c) -> uint32_t {
     if (c.leftOffset == LEAF_NORMAL) return 0u;   // the empty sibling of a one-leaf tree
-    if (c.leftOffset & LEAF_BIT) return mesh ? extract_count(c.leftOffset) : 1u;
-    return count[c.leftOffset];
+    return c.leftOffset & LEAF_BIT ? 1u : count[c.leftOffset];
   };
   // children are stored after their parent
   for (uint32_t p = n; p-- > 0;) {
@@ -301,21 +339,17 @@ bool mark_order(BVHNodePair* pairs, uint32_t n, bool mesh, std::vector<LeafOrder
       if (!(c->leftOffset & LEAF_BIT) && (c->leftOffset <= p || c->leftOffset >= n)) return false;
     count[p] = leaves(pairs[p].left) + leaves(pairs[p].right);
   }
-  order.assign(mesh || n == 0 ? 0u : count[0], LeafOrder{});
+  order.assign(n == 0 ? 0u : count[0], LeafOrder{});
   for (uint32_t p = 0; p < n; ++p) {
     BVHNode &l = pairs[p].left, &r = pairs[p].right;
-    const bool apart = l.leftOffset == LEAF_NORMAL || r.leftOffset == LEAF_NORMAL || l.boxMax.x <= r.boxMin.x ||
-                       r.boxMax.x <= l.boxMin.x || l.boxMax.y <= r.boxMin.y || r.boxMax.y <= l.boxMin.y ||
-                       l.boxMax.z <= r.boxMin.z || r.boxMax.z <= l.boxMin.z;
-    const uint32_t overlap = above[p] != WIDE_NO_OVERLAP || apart ? above[p] : p;
+    const bool separate = apart(l, r);
+    const uint32_t overlap = above[p] != WIDE_NO_OVERLAP || separate ? above[p] : p;
     uint32_t at = first[p];
     for (BVHNode* c : {&l, &r}) {
       if (c->leftOffset == LEAF_NORMAL) continue;
       if (!(c->leftOffset & LEAF_BIT)) {
         first[c->leftOffset] = at;
         above[c->leftOffset] = overlap;
-      } else if (mesh) {
-        if (extract_start(c->leftOffset) != at) return false;
       } else {
         if (extract_start(c->leftOffset) >= order.size()) return false;
         order[extract_start(c->leftOffset)] = LeafOrder{at, overlap};
@@ -323,14 +357,14 @@ bool mark_order(BVHNodePair* pairs, uint32_t n, bool mesh, std::vector<LeafOrder
       at += leaves(*c);
     }
     r.escapeIndex = first[p] + leaves(l);
-    l.escapeIndex = apart ? 0u : 1u;
+    l.escapeIndex = separate ? 0u : 1u;
   }
   return true;
 }
 
 }  // namespace
 
-// The instance level: its nodes and instance blocks fill the first 3 blocks per instance of wideBlocks
+// The instance level: its nodes and instance blocks fill the first 3 blocks per instance, wideTop
 // (fewer nodes than instances, two blocks an instance), so that a new instance tree of the same
 // instances fits again. Returns false when it cannot be packed.
 bool Scene::build_wide_instances(uint32_t* levels) {
@@ -352,7 +386,8 @@ bool Scene::build_wide_instances(uint32_t* levels) {
     }
   }
   const InstanceLeaf leaf{instances.data(), wideRoots.data(), ranks.data()};
-  std::vector<WideBlock> top;
+  Collapsed tree;
+  std::vector<WideBlock>& top = tree.top;
   wideSources.clear();
   *levels = 0;
   if (instances.size() == 1) {
@@ -360,36 +395,50 @@ bool Scene::build_wide_instances(uint32_t* levels) {
     leaf.write(pack_offset_and_size(0, 1), float3{}, float3{}, top.data());
     wideRoot = wide_ref(0, 2, true);
   } else {
-    const TlasTree tree{tlas.data()};
-    if (!Collapse<TlasTree, InstanceLeaf>{tree, leaf}.run(top, levels, &wideSources)) return false;
+    const TlasTree binary{tlas.data()};
+    if (!Collapse<TlasTree, InstanceLeaf>{binary, leaf}.run(tree, levels, &wideSources)) return false;
     wideRoot = wide_ref(0, 1, false);
   }
   if (top.size() > room) return false;
-  std::copy(top.begin(), top.end(), wideBlocks.begin());
+  wideTop = std::move(top);
+  wideTop.resize(room);
   return true;
 }
 
-// Builds wideBlocks from the device layout (devNodes, triSoup, frameLeaves, sbsNodes) and the TLAS, or
-// leaves it empty where the wide walk does not apply: it takes scenes of triangle meshes only, and scenes
-// of one instance of a frame octree, sparse voxel set or sparse brick set.
+// Builds wideBuild from the device layout (devNodes, triSoup, frameLeaves, sbsNodes) and the TLAS, or leaves
+// no tree where the wide walk does not apply: it takes scenes of triangle meshes only, and scenes of one
+// instance of a frame octree, sparse voxel set or sparse brick set. Nor is there one where memory is short.
 void Scene::build_wide() {
-  wideBlocks.clear();
+  bool ok = false;
+  try {
+    ok = build_wide_tree();
+  } catch (const std::bad_alloc&) {
+  }
+  if (ok) return;
+  wideBuild.reset();
+  wideCount = 0;
+  wideTop.clear();
   wideSources.clear();
+}
+
+bool Scene::build_wide_tree() {
   wideRoots.assign(geomData.size(), 0u);
   const uint32_t kinds = leaf_kinds();
   const bool sdf = (kinds == LK_FRAME || kinds == LK_SBS) && instances.size() == 1;
-  if ((kinds != LK_TRI && !sdf) || instances.empty()) return;
+  if ((kinds != LK_TRI && !sdf) || instances.empty()) return false;
   std::vector<uint8_t> used(geomData.size(), 0);
   for (const InstanceData& i : instances) used[i.geomId] = 1;
-  std::vector<Blocks> geom(geomData.size());
+  std::vector<Collapsed> geom(geomData.size());
   wideBlasLevels = 0;
   size_t total = 3 * instances.size();
   for (size_t g = 0; g < geomData.size(); ++g) {
     if (!used[g]) continue;
     const size_t first = geomData[g].bvhOffset, end = g + 1 < geomData.size() ? geomData[g + 1].bvhOffset : devNodes.size();
-    if (first >= end) return;   // an empty mesh
+    if (first >= end) return false;   // an empty mesh
     std::vector<LeafOrder> order;
-    if (!mark_order(devNodes.data() + first, uint32_t(end - first), kinds == LK_TRI, order)) return;
+    if (kinds == LK_TRI ? !mark_mesh_order(devNodes.data() + first, uint32_t(end - first))
+                        : !mark_leaf_order(devNodes.data() + first, uint32_t(end - first), order))
+      return false;
     const PairTree tree{devNodes.data() + first};
     uint32_t levels = 0;
     bool ok;
@@ -405,30 +454,37 @@ void Scene::build_wide() {
       const TriLeaf leaf{triSoup.data() + geomData[g].offset.x};
       ok = Collapse<PairTree, TriLeaf>{tree, leaf}.run(geom[g], &levels, nullptr);
     }
+    if (!ok) return false;
     wideRoots[g] = wide_ref(uint32_t(total), 1, false);
     total += geom[g].size();
-    if (!ok || total >= WIDE_MAX_BLOCKS) return;
+    if (total >= WIDE_MAX_BLOCKS) return false;
     wideBlasLevels = std::max(wideBlasLevels, levels);
   }
-  wideBlocks.resize(total);
   uint32_t levels = 0;
-  if (!build_wide_instances(&levels) || levels + wideBlasLevels > WIDE_MAX_LEVELS) {
-    wideBlocks.clear();
-    return;
-  }
+  if (!build_wide_instances(&levels) || levels + wideBlasLevels > WIDE_MAX_LEVELS) return false;
   wideLevels = levels + wideBlasLevels;
+  wideBuild.reset(new WideBlock[total]);   // not cleared: every block is written below
+  wideCount = total;
+  WideBlock* tree = wideBuild.get();
+  std::copy(wideTop.begin(), wideTop.end(), tree);
+  for (size_t g = 0; g < geom.size(); ++g) {
+    const Collapsed& c = geom[g];
+    if (c.top.empty()) continue;
+    const uint32_t base = wideRoots[g] & (WIDE_MAX_BLOCKS - 1);
+    place(c.top, c.top_nodes, 0, tree, base);
+    const int n_sub = int(c.subs.size());
+    std::vector<uint32_t> at(c.subs.size() + 1, base + uint32_t(c.top.size()));
+    for (int k = 0; k < n_sub; ++k) at[size_t(k) + 1] = at[size_t(k)] + uint32_t(c.subs[size_t(k)].blocks.size());
 #pragma omp parallel for schedule(dynamic, 1)
-  for (int g = 0; g < int(geom.size()); ++g) {
-    Blocks& b = geom[size_t(g)];
-    if (b.empty()) continue;
-    const uint32_t base = wideRoots[size_t(g)];
-    WideNode root;
-    std::memcpy(&root, &b[0], sizeof(root));
-    root.children += base;
-    std::memcpy(&b[0], &root, sizeof(root));
-    Collapse<PairTree, TriLeaf>::shift(b, root, base);
-    std::copy(b.begin(), b.end(), wideBlocks.begin() + base);
+    for (int k = 0; k < n_sub; ++k) {
+      const Subtree& s = c.subs[size_t(k)];
+      place(s.blocks, s.nodes, 1, tree, at[size_t(k)]);
+      WideNode root = s.root;
+      root.children += at[size_t(k)];
+      std::memcpy(tree + base + s.at, &root, sizeof(root));
+    }
   }
+  return true;
 }
 
 }  // namespace lrt

@@ -126,10 +126,16 @@ LRT_HD bool wide_pack_planes(const WideBox* box, uint32_t n, WideNode& out) {
       base = k == 0 || mn[k] < base ? mn[k] : base;
       top = k == 0 || mx[k] > top ? mx[k] : top;
     }
-    // smallest power of two whose 255 steps span the boxes (at least 2^-100)
-    int e = 27;
-    double step = 7.888609052210118e-31;   // 2^-100
+    // smallest power of two whose 255 steps span the boxes (at least 2^-100); the search begins eight to nine
+    // powers below the span, where 255 steps are too few
     const double span = double(top) - double(base);
+    uint64_t bits;
+    __builtin_memcpy(&bits, &span, sizeof(bits));
+    const int below = int(bits >> 52 & 0x7FF) - 1023 - 9;
+    int e = below < -100 ? 27 : below + 127;
+    bits = uint64_t(e - 127 + 1023) << 52;
+    double step;   // 2^(e - 127)
+    __builtin_memcpy(&step, &bits, sizeof(step));
     while (255.0 * step < span) { step *= 2.0; ++e; }
     for (;;) {
       bool fits = true;

@@ -217,3 +217,36 @@ def test_scenes_outside_the_terms_have_no_tree():
     one = np.repeat(f[:1], 7, axis=0)   # seven copies of one triangle share a leaf
     s.AddInstance(s.AddGeom_Triangles3f(v, one))
     assert tree(commit(s))[0].size == 0
+
+
+def test_subtrees_are_placed():
+    """A tree large enough for the parallel subtrees (hundreds of nodes below the top) beside smaller ones, read
+    twice: every triangle once, every child index inside its own geometry's blocks, the levels of the path."""
+    sizes = (40, 3, 25)
+    s = g.SceneRT()
+    for n in sizes:
+        s.AddInstance(s.AddGeom_Triangles3f(*g.gen_geodesic(n, 0.05, 4.0, n)))
+    blocks, root = tree(commit(s))
+    again, root2 = tree(s)
+    assert np.array_equal(blocks, again) and root == root2
+    spans = []
+
+    def leaf(at, count):
+        w = blocks[at:at + 2].reshape(-1)
+        f = w.view(np.float32)
+        seen, used = [], []
+
+        def tri(a, c):
+            used.extend(range(a, a + c))
+            return tri_leaf(blocks, seen)(a, c)
+        _, levels = walk(blocks, int(w[15]), tri)
+        n = sizes[int(w[20])]
+        assert sorted(p for p, _ in seen) == list(range(20 * n * n)) and len(set(used)) == len(used)
+        assert 3 < levels <= 40 or n == 3
+        spans.append((min([int(w[15]) & MASK] + used), max(used)))
+        return f[12:15].astype(np.float64), f[16:19].astype(np.float64)
+
+    walk(blocks, root, leaf)
+    spans.sort()
+    assert len(spans) == 3 and spans[0][0] == 9 and spans[-1][1] < len(blocks)
+    assert all(a[1] < b[0] for a, b in zip(spans, spans[1:]))
