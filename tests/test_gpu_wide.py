@@ -1,10 +1,12 @@
 """The wide walk (trace_wide.hip, the default on triangle scenes, single frame octrees and brick sets)
 and the multi-octree kernel (trace_multi.hip) against the binary walk, record for record: tile and batch edges, instances, first-hit and any-hit rays,
-rays and scenes that fall back to the sequential walk, a tree deeper than the LDS stack, the refitted
-instance level, graph replay and the allocation-free entry point."""
+rays and scenes that fall back to the sequential walk, trees deeper than the LDS stack, the refitted
+instance level, graph replay, several streams and the allocation-free entry point. Both scenes of a comparison
+say which walk they take."""
 import numpy as np
 import pytest
 
+import test_wide_cpu as cpu
 from conftest import assert_sdf_parity, raw_equal, sdf_check
 
 pytestmark = pytest.mark.gpu
@@ -33,17 +35,30 @@ def flags(torch, s, pos, dirs):
     return out.cpu().numpy()
 
 
-class Both:
-    """The same scene twice: the default (wide) walk and the binary walk."""
+LDS_STACK = 12   # WIDE_LDS_STACK (wide_walk.h): deeper trees spill
 
-    def __init__(self, g, build, tree=True):
+
+class Both:
+    """The same scene twice: the wide form, also for batches that crowd into a small scene, and the binary walk.
+    tree: the wide walk's, or none (multi-octrees and scenes without a wide form)."""
+
+    def __init__(self, g, build, tree=True, wide=True):
         self.g = g
         self.wide, self.binary = build(), build()
+        self.wide.set_walk(g.WALK_WIDE)
         self.binary.set_launch_config(256, 16, True)
         self.binary.set_tail_config(0, 1024)
+        self.binary.set_leaf_postponement(0)   # the sequential walk, leaf by leaf
+        self.walk = g.WALK_WIDE if wide else g.WALK_BINARY
         assert bool(self.wide.get_array("wide_blocks").size) == tree
 
+    def levels(self):
+        root = int(self.wide.get_array("wide_root").view(np.uint32)[0])
+        return cpu.tree_levels(self.wide.get_array("wide_blocks").view(np.uint32).reshape(-1, 16), root)
+
     def check(self, torch, pos, dirs, fn="trace_closest", any_hit=True):
+        n = pos.shape[0]
+        assert self.wide.walk_of_call(n) == self.walk and self.binary.walk_of_call(n) == self.g.WALK_BINARY
         a, b = (trace(torch, self.g, s, pos, dirs, fn) for s in (self.wide, self.binary))
         assert raw_equal(a, b), int((a.view(np.uint8).reshape(-1, 32) != b.view(np.uint8).reshape(-1, 32)).any(1).sum())
         if any_hit:
@@ -156,27 +171,66 @@ def test_ties(lrt, torch_dev):
     b.check(torch_dev, p, dirs[:5000].contiguous())
 
 
-def test_deep_tree(lrt, torch_dev):
-    """Triangles whose sizes fall by half each: a chain of nodes, more levels than stack entries in LDS."""
-    n = 66
-    k = 0.5 ** np.arange(n)
-    v = np.stack([np.stack([k, k * 0, k], 1), np.stack([k, k, -k], 1), np.stack([k, -k, k * 0], 1)], 1)
-    v = v.reshape(-1, 3).astype(np.float32)
-    f = np.arange(3 * n, dtype=np.uint32).reshape(-1, 3)
+def aimed_rays(torch, n, seed, at, octaves=30, far=100.0):
+    """Rays from around `at` to places nearer and nearer to it."""
+    rng = np.random.default_rng(seed)
+    pos = np.concatenate([rng.uniform(-0.2, 0.2, (n, 3)) + at, np.full((n, 1), 1e-4)], 1).astype(np.float32)
+    d = at + rng.normal(size=(n, 3)) * 0.5 ** rng.uniform(0, octaves, (n, 1)) - pos[:, :3]
+    dirs = np.concatenate([d / np.linalg.norm(d, axis=1, keepdims=True), np.full((n, 1), far)], 1).astype(np.float32)
+    return torch.from_numpy(pos).cuda(), torch.from_numpy(dirs).cuda()
+
+
+@pytest.mark.parametrize("n,ratio,n_inst,levels", [(66, 0.5, 1, 11), (200, 0.7, 1, 28), (200, 0.7, 12, 30), (200, 0.7, 60, 39),
+                                                   (200, 0.7, 100, None)])
+def test_deep_tree(lrt, torch_dev, n, ratio, n_inst, levels):
+    """Triangles whose sizes fall by a ratio each, alone and as instances whose sizes fall: a chain of nodes, up to
+    three times as many levels as stack entries in LDS. Batches whose rays are handed over in parts and batches
+    that fill the device; 100 instances have no tree (more than 40 levels)."""
+    def make():
+        s = lrt.SceneRT()
+        gid = s.AddGeom_Triangles3f(*cpu.chain_mesh(n, ratio))
+        for m in cpu.shrinking(n_inst):
+            s.AddInstance(gid, m)
+        s.CommitScene()
+        return s
+
+    b = Both(lrt, make, tree=levels is not None, wide=levels is not None)
+    assert levels is None or b.levels() == levels
+    for n_rays in (1, 100, 20000, 300001):
+        pos, dirs = aimed_rays(torch_dev, n_rays, 9, np.zeros(3))
+        if levels is None:   # (the two-pass scheme's hits are within some ulp here: triangles in front of their boxes)
+            b.wide.set_tail_config(0, 1024)
+        hits = b.check(torch_dev, pos, dirs)
+        assert n_rays == 1 or (hits["primId"] != lrt.MISS).mean() > 0.05
+        if n_rays <= 20000:
+            assert raw_equal(trace(torch_dev, lrt, b.wide, pos, dirs, "trace_closest_noalloc"), hits)
+
+
+@pytest.mark.parametrize("kind", ["frame", 1, 2, "indexed"])
+def test_deep_sdf_trees(lrt, torch_dev, kind):
+    """A frame octree and brick sets refined towards one point: more levels than stack entries in LDS, for traces
+    and, with the indexed set, for the differentiable calls (whose small batches take whole waves of rays then)."""
+    torch = torch_dev
 
     def make():
         s = lrt.SceneRT()
-        s.AddInstance(s.AddGeom_Triangles3f(v, f))
+        s.AddInstance(s.AddGeom_SdfFrameOctree(cpu.corner_octree(15)) if kind == "frame" else
+                      s.AddGeom_SdfSBS(*cpu.corner_bricks(15, kind)))
         s.CommitScene()
         return s
 
     b = Both(lrt, make)
-    rng = np.random.default_rng(3)
-    pos, dirs = random_rays(torch_dev, 20000, 9, extent=0.2)
-    target = torch_dev.from_numpy((rng.normal(size=(20000, 3)) * 0.5 ** rng.uniform(0, 30, (20000, 1))).astype(np.float32))
-    d = target.cuda() - pos[:, :3]
-    dirs[:, :3] = d / d.norm(dim=1, keepdim=True)
-    b.check(torch_dev, pos, dirs)
+    assert b.levels() > LDS_STACK
+    point = np.full(3, 2 * 0.333 - 1.0)   # the bits of the path are 1 0 1 0 ...: a third or two thirds of the cube
+    for at in (point, -point):
+        for n in (1, 100, 20000, 150001):
+            pos, dirs = aimed_rays(torch, n, 5, at)
+            dirs[::7, 3] = 0.15
+            hits = b.check(torch, pos, dirs)
+            assert n < 100 or (hits["primId"] != lrt.MISS).any()
+        if kind == "indexed":   # (fewer rays into the smallest bricks: short sums)
+            for n in (1, 100, 4097):
+                adjoint_agrees(torch, b, *aimed_rays(torch, n, 6, at, octaves=12))
 
 
 @pytest.mark.parametrize("depth", [2, 5, 8])
@@ -222,6 +276,66 @@ def test_instance_updates(lrt, torch_dev):
         s.UpdateInstance(0, moved[0])
         s.CommitScene()
     one.check(torch_dev, pos, dirs)
+
+
+@pytest.mark.parametrize("x,steps", [(9e29, ((1.2e30, 1), (9e29, 1), (1e31, 1))), (1.0, ((1e31, 2), (1.0, 1)))])
+def test_boxes_that_cannot_be_packed(lrt, torch_dev, x, steps):
+    """An instance far away moved past what a node's planes can hold (1e30) and back, by refits: the nodes above it
+    let every ray through meanwhile, and the exact boxes of instances decide as before. Where the instance tree is
+    built again with such a box, the scene goes without the wide walk."""
+    start = mats(40, 1, 4.0)
+    start[7][0, 3] = x
+    b = Both(lrt, mesh(lrt, 10, start))
+    pos, dirs = random_rays(torch_dev, 30000, 11, extent=5.0)
+    b.check(torch_dev, pos, dirs)
+    for x, kind in steps:
+        m = start[7].copy()
+        m[0, 3] = x
+        for s in (b.wide, b.binary):
+            s.UpdateInstance(7, m)
+            s.CommitScene()
+            assert s.commit_info()["kind"] == kind
+        if kind == 2:
+            b.walk = lrt.WALK_BINARY
+        b.check(torch_dev, pos, dirs)
+
+
+def test_streams(lrt, torch_dev):
+    """One scene traced on several streams at once, with rays for the second pass: each stream has its own queue
+    and counters."""
+    torch = torch_dev
+    bricks = Both(lrt, brick_scene(lrt, 4, 8, "indexed"))
+    for b in (Both(lrt, mesh(lrt, 40, mats(9, 1, 2.0))), bricks):
+        batches = []
+        for k, n in enumerate((60000, 999, 200001, 64)):
+            pos, dirs = random_rays(torch, n, 20 + k, extent=2.0)
+            dirs[::17, 1] = 0.0
+            batches.append((pos, dirs, b.check(torch, pos, dirs)))
+        streams = [torch.cuda.Stream() for _ in batches]
+        out = [torch.zeros((p.shape[0], 8), dtype=torch.int32, device="cuda") for p, _, _ in batches]
+        torch.cuda.synchronize()
+        for _ in range(5):
+            for h in out:
+                h.fill_(-1)
+            torch.cuda.synchronize()
+            for _ in range(4):
+                for (pos, dirs, _), st, h in zip(batches, streams, out):
+                    b.wide.trace_closest(pos, dirs, h, stream=st.cuda_stream)
+            torch.cuda.synchronize()
+            for (_, _, want), h in zip(batches, out):
+                assert raw_equal(h.cpu().numpy().view(lrt.HIT_DTYPE).reshape(-1), want)
+    # the differentiable calls, too
+    params = torch.from_numpy(bricks.wide.get_array("sbs_data_f")).cuda()
+    want = [torch.zeros((p.shape[0], 4), device="cuda") for p, _, _ in batches]
+    got = [torch.full_like(c, -7.0) for c in want]
+    for (pos, dirs, _), c in zip(batches, want):
+        bricks.wide.sbs_forward(0, params, pos, dirs, c)
+    torch.cuda.synchronize()
+    for _ in range(4):
+        for (pos, dirs, _), st, c in zip(batches, streams, got):
+            bricks.wide.sbs_forward(0, params, pos, dirs, c, stream=st.cuda_stream)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(want, got))
 
 
 def test_graph_replay_and_noalloc(lrt, torch_dev):
@@ -281,14 +395,10 @@ def test_bricks(lrt, torch_dev, depth, bs, kind):
         assert (hits["primId"] != lrt.MISS).sum() > 0
 
 
-@pytest.mark.parametrize("depth,n", [(3, 1), (3, 63), (4, 4097), (5, 50000)])
-def test_adjoint(lrt, torch_dev, depth, n):
+def adjoint_agrees(torch, b, pos, dirs):
     """Colour bit for bit, gradient and loss up to the order of the atomics (fp32 sums of up to 50,000 terms
     in another order: 1e-5 of the norm)."""
-    torch = torch_dev
-    b = Both(lrt, brick_scene(lrt, depth, 8, "indexed"))
-    pos, dirs = random_rays(torch, n, depth, extent=2.0)
-    dirs[::13, 1] = 0.0
+    n = pos.shape[0]
     params = torch.from_numpy(b.wide.get_array("sbs_data_f")).cuda()
     params += 0.002 * torch.randn(params.shape, device="cuda", generator=torch.Generator("cuda").manual_seed(1))
     target = torch.rand((n, 4), device="cuda", generator=torch.Generator("cuda").manual_seed(2))
@@ -308,6 +418,14 @@ def test_adjoint(lrt, torch_dev, depth, n):
         assert torch.equal(x, y)
     for x, y in zip(got[0][1] + got[0][2], got[1][1] + got[1][2]):
         assert float((x - y).norm()) <= 1e-5 * float(y.norm()) + 1e-12
+
+
+@pytest.mark.parametrize("depth,n", [(3, 1), (3, 63), (4, 4097), (5, 50000)])
+def test_adjoint(lrt, torch_dev, depth, n):
+    b = Both(lrt, brick_scene(lrt, depth, 8, "indexed"))
+    pos, dirs = random_rays(torch_dev, n, depth, extent=2.0)
+    dirs[::13, 1] = 0.0
+    adjoint_agrees(torch_dev, b, pos, dirs)
 
 
 @pytest.mark.parametrize("other", [1, 2, "indexed"])
@@ -457,12 +575,11 @@ def test_crowded_batches(lrt, torch_dev, kind, size, line):
     """Both sides of the line where default calls leave the wide walk, and batches beyond it with the walk set."""
     b = Both(lrt, mesh(lrt, size) if kind == "mesh" else brick_scene(lrt, size, 1, 1))
     for n in (line - 1, line):
-        assert b.wide.walk_of_call(n) == (lrt.WALK_WIDE if n < line else lrt.WALK_BINARY)
         pos, dirs = random_rays(torch_dev, n, 1)
-        b.check(torch_dev, pos, dirs)
-    b.wide.set_walk(lrt.WALK_WIDE)
-    assert b.wide.walk_of_call(line) == lrt.WALK_WIDE
-    b.check(torch_dev, pos, dirs)
+        for b.walk, setting in ((lrt.WALK_WIDE if n < line else lrt.WALK_BINARY, lrt.WALK_AUTO),
+                                (lrt.WALK_WIDE, lrt.WALK_WIDE)):
+            b.wide.set_walk(setting)
+            b.check(torch_dev, pos, dirs)
 
 
 @pytest.mark.parametrize("kind", ["crowded mesh", "instances", "multi", "mixed"])
@@ -519,7 +636,7 @@ def test_multi_octree_of_one_node(lrt, orc, torch_dev, first, voxels):
                 s.AddInstance(s.AddGeom_Triangles3f(*lrt.gen_geodesic(3, 0.05, 4.0, 2)), mats(1, 5, 2.0)[0])
             s.CommitScene()
             return s
-        b = Both(lrt, make, tree=False)
+        b = Both(lrt, make, tree=False, wide=not beside)
         pos, dirs = random_rays(torch_dev, 20001, 3, extent=2.5)
         dirs[::11, 0] = 0.0
         got = b.check(torch_dev, pos, dirs)

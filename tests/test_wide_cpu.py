@@ -57,6 +57,97 @@ def walk(blocks, root, leaf):
     return (mn, mx), levels + 1
 
 
+def tree_levels(blocks, root):
+    """Most nodes on a path, the instance level's and a geometry's together."""
+    known = {}
+
+    def below(at):
+        if at not in known:
+            known[at] = 1 + max([0] + [below(c) for _, c, _, is_leaf in children(blocks[at]) if not is_leaf])
+        return known[at]
+
+    if root >> 31:
+        return below(int(blocks[root & MASK][15]))
+    todo, most = [(root & MASK, 1)], 0
+    while todo:
+        at, level = todo.pop()
+        for _, c, _, is_leaf in children(blocks[at]):
+            if is_leaf:
+                most = max(most, level + below(int(blocks[c][15])))
+            else:
+                todo.append((c, level + 1))
+    return most
+
+
+def chain_mesh(n, ratio):
+    """Triangles whose sizes fall by a ratio each, about the origin: a chain of nodes."""
+    k = ratio ** np.arange(n)
+    v = np.stack([np.stack([k, k * 0, k], 1), np.stack([k, k, -k], 1), np.stack([k, -k, k * 0], 1)], 1)
+    return v.reshape(-1, 3).astype(np.float32), np.arange(3 * n, dtype=np.uint32).reshape(-1, 3)
+
+
+def shrinking(n, ratio=0.5):
+    """n instance matrices whose scales fall by a ratio each."""
+    return [np.diag([ratio ** k] * 3 + [1]).astype(np.float32) for k in range(n)]
+
+
+def corner_cells(levels):
+    """(x, y, z, size) of the cells of an octree refined towards one point of the cube, the siblings on the way
+    refined once more: cells of sizes 1 / 4 to 1 / 2^levels."""
+    path, cells = np.zeros(3, np.int64), []
+    for k in range(1, levels):
+        path = 2 * path + (k % 2)
+        base = path - (k % 2)
+        for c in np.ndindex(2, 2, 2):
+            if (base + c != path).any():
+                cells += [(*(2 * (base + c) + e), 2 << k) for e in np.ndindex(2, 2, 2)]
+    return cells
+
+
+# corner values of a cell crossed by a plane, x slowest
+CROSSED = np.array([(i >> 2) + 0.7 * (i >> 1 & 1) + 0.4 * (i & 1) - 1.0 for i in range(8)], np.float32)
+
+
+def corner_octree(levels):
+    """corner_cells as a frame octree, whose leaves are all crossed."""
+    nodes, path = [[CROSSED, 0]], 0
+    for k in range(1, levels):
+        nodes[path][1] = len(nodes)
+        first, bit = len(nodes), 7 * (k % 2)
+        nodes += [[CROSSED, 0] for _ in range(8)]
+        for c in range(8):
+            if c != bit:
+                nodes[first + c][1] = len(nodes)
+                nodes += [[CROSSED, 0] for _ in range(8)]
+        path = first + bit
+    out = np.zeros(len(nodes), g.FRAME_NODE_DTYPE)
+    out["values"], out["offset"] = [n[0] for n in nodes], [n[1] for n in nodes]
+    return out
+
+
+def corner_bricks(levels, kind):
+    """AddGeom_SdfSBS's arguments of corner_cells as 2^3 bricks: codes of `kind` bytes, which all share, or
+    "indexed", with distances and albedos of their own."""
+    h = np.zeros((), g.SBS_HEADER_DTYPE)
+    h["brick_size"], h["bytes_per_value"] = 2, 4 if kind == "indexed" else kind
+    nodes = np.array([((x << 16) | y, (z << 16) | s, 0, 0) for x, y, z, s in corner_cells(levels)], g.SBS_NODE_DTYPE)
+    x = np.stack(np.meshgrid(*[np.arange(3) - 1.0] * 3, indexing="ij"), 3).reshape(-1, 3)
+    d = (x @ [0.5, 0.35, 0.2]).astype(np.float32)   # of the plane, in half bricks
+    if kind == "indexed":
+        h["aux_data"], n = g.SDF_SBS_NODE_LAYOUT_ID32F_IRGB32F, 27 * nodes.size
+        point = np.arange(n).reshape(-1, 27)
+        words = np.concatenate([point, n + 3 * point[:, [0, 2, 6, 8, 18, 20, 24, 26]]], 1).astype(np.uint32)
+        nodes["data_offset"] = 35 * np.arange(nodes.size)
+        albedo = np.random.default_rng(1).uniform(0, 1, 3 * n).astype(np.float32)
+        return h, nodes, words.reshape(-1), np.concatenate([np.tile(0.1 * d, nodes.size), albedo])
+    h["aux_data"] = g.SDF_SBS_NODE_LAYOUT_DX
+    top = (1 << 8 * kind) - 1
+    codes = np.round((0.5 + 0.4 * d / np.abs(d).max()) * top).astype(np.uint32)
+    per = 4 // kind
+    codes = np.concatenate([codes, np.zeros(-len(codes) % per, np.uint32)]).reshape(-1, per)
+    return h, nodes, (codes << (8 * kind * np.arange(per, dtype=np.uint32))).sum(1).astype(np.uint32)
+
+
 def tri_leaf(blocks, seen):
     def leaf(at, count):
         boxes = []
@@ -250,3 +341,26 @@ def test_subtrees_are_placed():
     spans.sort()
     assert len(spans) == 3 and spans[0][0] == 9 and spans[-1][1] < len(blocks)
     assert all(a[1] < b[0] for a, b in zip(spans, spans[1:]))
+
+
+def test_most_levels():
+    """Trees of up to 40 levels are kept, deeper ones leave the scene to the binary walk: a mesh of 28 levels below
+    more and more levels of instances. The deep scenes that the GPU tests trace have the levels they need."""
+    def levels(mesh, n):
+        s = g.SceneRT()
+        gid = s.AddGeom_Triangles3f(*mesh)
+        for m in shrinking(n):
+            s.AddInstance(gid, m)
+        blocks, root = tree(commit(s))
+        return tree_levels(blocks, root) if blocks.size else None
+
+    deep, flat = chain_mesh(200, 0.7), chain_mesh(1, 1.0)
+    assert levels(deep, 1) == 28 and levels(flat, 1) == 1
+    assert 28 < levels(deep, 12) < levels(deep, 60) <= 40
+    assert levels(flat, 100) + 27 > 40 and levels(deep, 100) is None
+    for add in (lambda s: s.AddGeom_SdfFrameOctree(corner_octree(15)),
+                lambda s: s.AddGeom_SdfSBS(*corner_bricks(15, 2)),
+                lambda s: s.AddGeom_SdfSBS(*corner_bricks(15, "indexed"))):
+        s = g.SceneRT()
+        s.AddInstance(add(s))
+        assert 13 < tree_levels(*tree(commit(s))) <= 40
