@@ -689,18 +689,24 @@ uint32_t Scene::leaf_kinds() const {
   return k;
 }
 
-// With hundreds of rays a triangle the lanes of a wave go the same way, and a binary step of one shared fetch
-// and two box tests is cheaper than a wide one of six. Camera rays, wide against binary: 500 triangles, 182
-// thousand rays 56 us against 48 and 30 thousand 38 against 48; 1,280 triangles, 990 thousand 150 against 103 and
-// 182 thousand 62 against 61; 5,120 triangles, 990 thousand 178 against 162 and 182 thousand 77 against 98;
-// 20,480 triangles, 990 thousand 217 against 288. So the line is at 128 rays a triangle, and at 65,536 rays,
-// below which the wide walk's shorter chains win for any mesh. Bricks hold some
-// hundred voxels each: 384 bricks, 630 thousand rays 331 against 316 and 30 thousand 87 against 245; 6,144
-// bricks, 480 thousand 580 against 3,000: 1,024 rays a brick.
+// With hundreds of rays a triangle the lanes of a wave of camera rays go the same way, and a binary step of one
+// shared fetch and two box tests is cheaper than a wide one of six. Camera rays, us, binary against wide: 180
+// triangles, 990 thousand rays 85 against 141; 500 triangles, 182 thousand 56 against 65 and 70 thousand 52 against
+// 51; 1,280 triangles, 990 thousand 122 against 165; 2,880 triangles, 368 thousand 101 against 125; 5,120 triangles,
+// 656 thousand 145 against 174 and 182 thousand 108 against 89; 6,480 triangles, 830 thousand 178 against 202 and
+// 1.2 million 240 against 229; 8,000 triangles, 1.02 million 243 against 215 and 3 million 474 against 364; 20,480
+// triangles, 3 million 772 against 383. So the binary walk keeps batches of 65,536 rays and 128 a triangle into
+// meshes of up to 7,168 triangles. A brick holds many voxels: 64 bricks of 4^3, 1 million rays 222 against 300 and 66
+// thousand 123 against 94; 64 of 8^3, 630 thousand 316 against 328 and 182 thousand 212 against 135; 512 bricks, 524
+// thousand 528 against 351. There the lines are 8,192 rays a brick and 256 bricks.
+// Incoherent rays profit less or not at all, and the rule cannot know them: rays leaving the surfaces, 500 triangles,
+// 182 thousand 49 against 39 and 990 thousand 124 against 130; 2,880 triangles, 369 thousand 118 against 78; rays from
+// and to anywhere, 500 triangles, 3 million 391 against 337; 64 bricks, 1 million 741 against 316. For those
+// lrt_set_walk and lrt_autotune choose the wide walk.
 bool Scene::rays_crowd(uint64_t n) const {
   if (n < 65536 || instances.size() != 1 || geomTags.size() != 1) return false;
-  if (geomTags[0] == TAG_TRIANGLE) return n >= 128ull * (indices.size() / 3);
-  return geomTags[0] == TAG_SDF_BRICK && n >= 1024ull * sbsNodes.size();
+  if (geomTags[0] == TAG_TRIANGLE) return indices.size() / 3 <= 7168 && n >= 128ull * (indices.size() / 3);
+  return geomTags[0] == TAG_SDF_BRICK && sbsNodes.size() <= 256 && n >= 8192ull * sbsNodes.size();
 }
 
 // Postponed triangle leaves help coherent rays into one mesh (fewer wave-wide waits) and hurt

@@ -290,8 +290,9 @@ lrt_status lrt_eye_rays_dev(const float* proj_inv16, const float* world_view_inv
 /* Scenes of triangle meshes, and scenes of one instance of a frame octree, sparse voxel set or sparse brick
  * set, are traced by a six-wide walk built at commit that has no launch shape to choose, scenes of
  * multi-octrees by a kernel that has none either: the wide form. Other scenes, counted calls and the
- * INTERSECTION_COUNT mode take the binary walk, and so, by default, do large batches (65,536 rays or more) into one small
- * mesh or brick set (128 rays a triangle, 1,024 a brick), which it is faster on. Each of the launch-shape
+ * INTERSECTION_COUNT mode take the binary walk, and so do, by default, large batches (65,536 rays or more) into
+ * one small mesh or brick set (up to 7,168 triangles and 128 rays a triangle, or 256 bricks and 8,192 a brick):
+ * camera rays are faster on it there, incoherent ones mostly are not. Each of the launch-shape
  * calls below (lrt_set_launch_config, lrt_set_tail_config, lrt_set_leaf_postponement with 0 or 1,
  * lrt_set_ray_interleave, lrt_set_persistent) moves the scene to the binary walk in that shape;
  * lrt_autotune tries both and keeps the faster for every batch; lrt_set_walk chooses. Same hit records

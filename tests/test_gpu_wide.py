@@ -569,14 +569,15 @@ def test_multi_octrees(lrt, torch_dev, depth, count, lod, n):
         assert raw_equal(out.cpu().numpy().view(g.HIT_DTYPE).reshape(-1), hits)
 
 
-# the lines of Scene::rays_crowd: 65,536 rays, 128 a triangle, 1,024 a brick
-@pytest.mark.parametrize("kind,size,line", [("mesh", 1, 65536), ("mesh", 6, 92160), ("bricks", 2, 65536)])
+# the lines of Scene::rays_crowd: 65,536 rays, 128 a triangle up to 7,168 triangles, 8,192 a brick up to 256 bricks
+@pytest.mark.parametrize("kind,size,line", [("mesh", 1, 65536), ("mesh", 6, 92160), ("mesh", 18, 829440), ("mesh", 19, None),
+                                            ("bricks", 2, 524288), ("bricks", 3, None)])
 def test_crowded_batches(lrt, torch_dev, kind, size, line):
     """Both sides of the line where default calls leave the wide walk, and batches beyond it with the walk set."""
     b = Both(lrt, mesh(lrt, size) if kind == "mesh" else brick_scene(lrt, size, 1, 1))
-    for n in (line - 1, line):
+    for n in (line - 1, line) if line else (1000003,):
         pos, dirs = random_rays(torch_dev, n, 1)
-        for b.walk, setting in ((lrt.WALK_WIDE if n < line else lrt.WALK_BINARY, lrt.WALK_AUTO),
+        for b.walk, setting in ((lrt.WALK_BINARY if n == line else lrt.WALK_WIDE, lrt.WALK_AUTO),
                                 (lrt.WALK_WIDE, lrt.WALK_WIDE)):
             b.wide.set_walk(setting)
             b.check(torch_dev, pos, dirs)
