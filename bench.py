@@ -6,8 +6,9 @@ closest-hit trace call (both passes), or one fused forward + adjoint of the diff
 set. The default run (--workload all) prints ONE JSON line whose headline is the closest-hit
 icosphere7_512 workload (512x512 primary rays on a 327,680-triangle mesh, the reference's
 closest-hit configuration) and which carries every other workload under "sub_results", each with
-its ms/step, Mrays/s, roofline (algorithmic bytes per step from traversal counters / step time,
-against 8 TB/s; measured HBM bytes per step from the committed counter summaries; the limiting
+its ms/step, Mrays/s, the walk timed (the six-wide walk and the multi-octree kernel, "wide", have no
+launch shape; "launch" is then the binary walk's), roofline (algorithmic bytes per step from traversal
+counters / step time, against 8 TB/s; measured HBM bytes per step from the committed counter summaries; the limiting
 stage named by the committed counter ratios) and the CPU oracle timed on the host cores.
 
 Workloads (synthetic, seeded):
@@ -259,6 +260,9 @@ def run_batch(args, torch, g, cpu_target_s):
         tune = {"lds_stack": lds, "record": rec, "grid": grid, "given": True}
     elif not args.no_autotune:
         tune = batch.autotune(sh)
+    if args.walk:
+        batch.set_walk(WALKS[args.walk])
+    wide = batch.get_walk() == g.WALK_WIDE
     if args.copy_calibration:
         copy_calibration(torch)
 
@@ -269,7 +273,7 @@ def run_batch(args, torch, g, cpu_target_s):
     alg_bytes, hit_n = 0.0, 0.0
     for it in items:
         trav, hn = sbs_traversal_bytes(torch, g, it["scene"], it["pos"], it["dir"], sh)
-        alg_bytes += it["pos"].shape[0] * B_DIFF_RAY + trav + hn * B_DIFF_HIT
+        alg_bytes += it["pos"].shape[0] * B_DIFF_RAY + (0 if wide else trav) + hn * B_DIFF_HIT
         alg_bytes += it["params"].numel() * 4 + it["bricks"] * 729 * 8
         hit_n += hn
 
@@ -310,7 +314,7 @@ def run_batch(args, torch, g, cpu_target_s):
             "ms_per_scene_fused_launches": round(ms_plain_fused, 4),
             "batched_vs_per_scene_fused": round(ms_plain_fused / ms, 2),
             "recompute_misses": int(sum(it["scene"].sbs_recompute_misses() for it in items)),
-            "launch": tune, "autotuned": tune is not None,
+            "launch": tune, "walk": walk_name(wide), "autotuned": tune is not None,
             "algorithmic_bytes_per_ray": round(alg_bytes / n, 1)}
     cpu = None
     if cpu_target_s > 0:
@@ -319,7 +323,7 @@ def run_batch(args, torch, g, cpu_target_s):
         pos_np, dir_np = items[0]["pos"].cpu().numpy(), items[0]["dir"].cpu().numpy()
         cpu = cpu_baseline([it["scene"] for it in items], pos_np, dir_np, threads, cpu_target_s,
                            what="forward closest hit of the same rays (the oracle has no adjoint)")
-    return result("sbs_batch_64x4x128", n, ms, args, desc, alg_bytes, cpu, unit="Mrays/s (fwd+bwd, batched)")
+    return result("sbs_batch_64x4x128", n, ms, args, desc, alg_bytes, cpu, unit="Mrays/s (fwd+bwd, batched)", wide=wide)
 
 
 def copy_calibration(torch):
@@ -363,7 +367,10 @@ def run_diff(args, torch, g, cpu_target_s):
     # one fused pass: ray I/O, one traversal (the hit voxel is recorded by the walk's own brick
     # march, not marched again), 32 parameters read and 32 atomics per hit
     trav, hit_n = sbs_traversal_bytes(torch, g, scene, pos, dirs, sh)
-    alg_bytes = n * B_DIFF_RAY + trav + hit_n * B_DIFF_HIT
+    if args.walk:
+        scene.set_walk(WALKS[args.walk])
+    wide = scene.get_walk() != g.WALK_BINARY
+    alg_bytes = n * B_DIFF_RAY + (0 if wide else trav) + hit_n * B_DIFF_HIT
 
     if args.copy_calibration:
         copy_calibration(torch)
@@ -379,12 +386,12 @@ def run_diff(args, torch, g, cpu_target_s):
             "distance_values": int(nd), "views": 8, "width": 256, "height": 256, "rays": int(n),
             "hit_fraction": round(hit_n / n, 4), "scene_build_s": round(build_s, 2),
             "recompute_misses": scene.sbs_recompute_misses(), "loss": float(loss.item()),
-            "algorithmic_bytes_per_ray": round(alg_bytes / n, 1)}
+            "walk": walk_name(wide), "algorithmic_bytes_per_ray": round(alg_bytes / n, 1)}
     cpu = None
     if cpu_target_s > 0:
         cpu = cpu_baseline([scene], pos.cpu().numpy(), dirs.cpu().numpy(), threads, cpu_target_s,
                            what="forward closest hit of the same rays (the oracle has no adjoint)")
-    return result("sbs_diff_256_8x256", n, ms, args, desc, alg_bytes, cpu, unit="Mrays/s (fwd+bwd)")
+    return result("sbs_diff_256_8x256", n, ms, args, desc, alg_bytes, cpu, unit="Mrays/s (fwd+bwd)", wide=wide)
 
 
 def algorithmic_bytes(cnt, hits, kind):
@@ -495,6 +502,9 @@ def limiter(workload, ms, traffic):
     ta = cnt.get("TA busy / active cycles (8 XCDs)")
     if hbm is not None and hbm > 0.6:
         name = "hbm bandwidth"
+    elif cnt.get("vector unit busy (1024 SIMDs)", 0.0) > 0.8:
+        name = (f"vector instructions (at {cnt.get('active lanes of 64 per vector instruction', 0.0):.0f} of 64 lanes on "
+                "average)")
     elif ta is not None and ta > 0.5:
         name = "texture addresser (address expansion of divergent gathers)"
     else:
@@ -509,9 +519,19 @@ def limiter(workload, ms, traffic):
     return out
 
 
-def result(workload, n, ms, args, desc, alg_bytes, cpu, unit="Mrays/s"):
+WALKS = {"binary": 0, "wide": 1}   # WALK_* of the package
+
+
+def walk_name(wide):
+    return "wide" if wide else "binary"
+
+
+def result(workload, n, ms, args, desc, alg_bytes, cpu, unit="Mrays/s", wide=False):
+    """Bytes of a step on the wide walk are those of rays, records and gradients only: the counters that the byte
+    model takes its visits from are the binary walk's. Its counter summaries are files of their own."""
     mrays = n / (ms * 1e-3) / 1e6
     achieved = alg_bytes / (ms * 1e-3) / 1e9
+    workload += "_wide" if wide else ""
     traffic = load_traffic(workload)
     roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic}
@@ -532,6 +552,8 @@ def run_trace(name, args, torch, g, cpu_target_s):
     scene.set_leaf_postponement(args.leaf_postpone)
     scene.set_ray_interleave(args.ray_interleave)
     scene.set_persistent(bool(args.persistent))
+    if args.walk:
+        scene.set_walk(WALKS[args.walk])
     stream = torch.cuda.current_stream()
     sh = stream.cuda_stream
     if isinstance(w, tuple):   # explicit ray buffers
@@ -558,6 +580,9 @@ def run_trace(name, args, torch, g, cpu_target_s):
     tune = None
     if not args.no_autotune:
         tune = scene.autotune(pos, dirs, hits, stream=sh)
+    wide = scene.walk_of_call(n) == g.WALK_WIDE
+    if wide and kind != "multi":   # (the multi-octree kernel's visits are the counted walk's)
+        alg_bytes = float(B_RAY_IO * n)
     if args.copy_calibration:
         copy_calibration(torch)
 
@@ -588,12 +613,13 @@ def run_trace(name, args, torch, g, cpu_target_s):
                "ray_interleave": args.ray_interleave, "budget": args.budget, "tail_waves": args.tail_waves,
                "leaf_postpone": args.leaf_postpone, "persistent": args.persistent})
     desc.update({"hit_fraction": round(float((hits_np["primId"] != g.MISS).mean()), 4),
-                 "scene_build_s": round(build_s, 2), "launch": launch, "autotuned": tune is not None,
+                 "scene_build_s": round(build_s, 2), "walk": walk_name(wide),
+                 "launch": launch, "autotuned": tune is not None,
                  "stack_overflow_rays": overflow, "ms_eager": round(ms_eager, 4), "timed": "hip graph replay",
                  "records_differing_from_single_pass": differ,
                  "mean_fat_nodes_per_ray": round(float(cnt[:, 0].mean()), 2),
                  "algorithmic_bytes_per_ray": round(alg_bytes / n, 1)})
-    return result(name, n, ms, args, desc, alg_bytes, cpu)
+    return result(name, n, ms, args, desc, alg_bytes, cpu, wide=wide)
 
 
 def run_build(args, torch, g):
@@ -700,6 +726,8 @@ def main():
                     help="triangle leaf postponement when not autotuning (-1: on for one instance)")
     ap.add_argument("--persistent", type=int, default=0, choices=[0, 1],
                     help="persistent single-pass kernel when not autotuning")
+    ap.add_argument("--walk", default="", choices=[""] + list(WALKS),
+                    help="the walk to time instead of the tuner's choice or, untuned, the given binary shape")
     ap.add_argument("--batch-config", default="",
                     help="lds_stack,record,grid of the batched adjoint kernel instead of its autotuner")
     ap.add_argument("--copy-calibration", action="store_true",

@@ -40,7 +40,7 @@ def _col(row, *names):
 
 def short_name(name):
     """Kernel name without return type, namespaces and parameter list (library kernels)."""
-    name = name.replace("(anonymous namespace)::", "")
+    name = name.replace("(anonymous namespace)::", "").replace("(lrt::WideLeafKind)", "")
     m = re.search(r"\blrt::(k_\w+)", name)
     if m:
         return name[m.start(1):].split("(")[0]
@@ -131,6 +131,13 @@ def cmd_counters(a):
     if "SQ_WAIT_INST_ANY" in vals and "SQ_WAVE_CYCLES" in vals:
         derived.append(("wave cycles waiting on an instruction",
                         vals["SQ_WAIT_INST_ANY"] / max(1.0, vals["SQ_WAVE_CYCLES"])))
+    if "SQ_THREAD_CYCLES_VALU" in vals and "SQ_ACTIVE_INST_VALU" in vals:
+        derived.append(("active lanes of 64 per vector instruction",
+                        vals["SQ_THREAD_CYCLES_VALU"] / max(1.0, vals["SQ_ACTIVE_INST_VALU"])))
+    if "SQ_ACTIVE_INST_VALU" in vals and "GRBM_GUI_ACTIVE" in vals:
+        # SQ counters count in quads of cycles, summed over 1024 SIMDs
+        derived.append(("vector unit busy (1024 SIMDs)",
+                        vals["SQ_ACTIVE_INST_VALU"] * 4.0 * XCDS / 1024.0 / max(1.0, vals["GRBM_GUI_ACTIVE"])))
     if derived:
         lines += ["", "derived:"] + [f"{k:44s} {v:8.3f}" for k, v in derived]
     print("\n".join(lines))
