@@ -166,8 +166,8 @@ __global__ __launch_bounds__(BLOCK) void k_sbs_diff(SceneView s, SbsDiffArgs a) 
 // words a lane) takes the walk's result of each ray. A ray the wide walk leaves to the sequential one
 // (zero or non-finite components) is queued as `code` for a second kernel (walked here, its code took the
 // kernel from 4 waves a SIMD to 3: the batch of 12 x 4 x 128 x 128 rays 0.88 ms instead of 0.66).
-// What bounds it: vector instructions of solves and node steps at a sixth and half of the lanes, and the
-// waves with the most grazing rays. Whole calls, masks included, against one ray a lane of the binary walk:
+// What bounds it: vector instructions of solves and node steps, at 17 of 64 lanes on average with the units busy
+// two fifths of the time, and the waves with the most grazing rays. Whole calls, masks included, against one ray a lane of the binary walk:
 // 8 x 256 x 256 rays into 256^3 voxels 0.79 ms against 0.86, 3 x 201 x 201 rays into 128^3, forward and
 // backward apart, 0.57 against 0.87, the batch above 0.68 against 0.90.
 template <int MODE>

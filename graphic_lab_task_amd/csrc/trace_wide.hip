@@ -11,7 +11,8 @@
 // step (327,680 triangles, 512 x 512: 177 us against 262; octree of depth 9, 1024 x 1024: 0.45 ms against
 // 0.99); 1,000 rays take 33 us against 88. A brick set of 256^3 voxels, 800 x 600: 0.53 ms against 2.76
 // (most rays graze bricks and were left to the second pass); there it is the surface solves, about a
-// thousand vector instructions each, that a sixth of the lanes are in at a time.
+// thousand vector instructions each (on average 17 of 64 lanes are active, the vector units busy a third of the
+// time; the instanced rays keep them busy all the time at 22 lanes).
 //
 // Results are the sequential walk's (traverse.h). The packed boxes and the widened slab test only let
 // more leaves through. What the sequential walk finds is then decided with its own arithmetic:
@@ -23,9 +24,12 @@
 //    queued and walked again by the sequential kernel. So are rays the monotonic test does not cover
 //    (zero or non-finite components, box_test_fast) and rays that stop at the sequential walk's first
 //    hit. Of two triangles at one distance the first in the sequential order counts (wide_before).
-//    What is left open: a triangle in front of its own boxes by more than wide_limit's slack that
-//    another hit within that distance hides from this walk and not from the sequential one (none seen in
-//    80 million rays between overlapping instances).
+//    What is left open: a triangle in front of its own boxes by more than wide_limit's slack that another
+//    hit hides from this walk and not from the sequential one. That takes a ray in the triangle's plane to
+//    within rounding, whose computed distance is noise. Of 400,000 rays made to lie in the planes of 300 to
+//    30,000 overlapping triangles 9 to 76 records differ, tilted by 1e-7 7 to 39, by 1e-5 none or one (the
+//    two-pass binary walk: 205 to 316, 117 to 182, 1 to 5); none of 80 million rays between overlapping
+//    instances, nor of 600,000 into chains of triangles down to 1e-31 across.
 //  * an SDF walk ends at the first leaf that hits. Where a plane separates the two children of a binary
 //    node, every ray passes the leaves of one side before the other's and the sequential walk visits them
 //    in that order, so the answer is the hitting leaf with the smallest box entry. Two leaves of one

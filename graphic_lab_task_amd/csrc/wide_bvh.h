@@ -1,6 +1,10 @@
 // Six-wide BVH with quantised boxes: the layout that trace_wide.hip walks, and the rule that packs
 // one node (used by the host builder and by the device refit of the instance level).
 //
+// Nodes of one base and three power-of-two steps with 8-bit planes, children consecutive, are those of H. Ylitie, T.
+// Karras and S. Laine, "Efficient Incoherent Ray Traversal on GPUs Through Compressed Wide BVHs", HPG 2017 (eight
+// wide there; six make one line segment here, and the leaves carry the exact boxes the sequential walk tests).
+//
 // The tree is collapsed from the binary one (device-layout pairs, TLAS nodes) at commit and lives in
 // one array of 64-byte blocks, so that a node, a triangle or half an instance is one aligned line
 // segment of four 16-byte loads. The children of a node are consecutive: inner children take one

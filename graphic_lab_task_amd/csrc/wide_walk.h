@@ -10,7 +10,7 @@ enum WideLeafKind { WIDE_TRI, WIDE_FRAME, WIDE_BRICK };
 
 constexpr int WIDE_BLOCK = 64;
 constexpr int WIDE_LDS_STACK = 12;   // entries in LDS; the deeper ones spill
-// Idle lanes from which on parts of rays are handed over (8: 193 us in that case, 16: 186, 32: 186)
+// Idle lanes from which on parts of rays are handed over (327,680 triangles, 512 x 512: 8 193 us, 16 186, 32 186)
 constexpr uint32_t WIDE_SHARE = 16;
 constexpr uint32_t WIDE_DONE = 0xFFFFFFFFu;
 constexpr uint32_t WIDE_LEAF = 0x80000000u;

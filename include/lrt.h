@@ -295,8 +295,14 @@ lrt_status lrt_eye_rays_dev(const float* proj_inv16, const float* world_view_inv
  * camera rays are faster on it there, incoherent ones mostly are not. Each of the launch-shape
  * calls below (lrt_set_launch_config, lrt_set_tail_config, lrt_set_leaf_postponement with 0 or 1,
  * lrt_set_ray_interleave, lrt_set_persistent) moves the scene to the binary walk in that shape;
- * lrt_autotune tries both and keeps the faster for every batch; lrt_set_walk chooses. Same hit records
- * either way.
+ * lrt_autotune tries both and keeps the faster for every batch; lrt_set_walk chooses.
+ *
+ * All of these give the same hit records, those of the reference's sequential walk, with one exception: a ray
+ * that lies in a triangle's plane to within rounding (about 1e-6 of its direction) may find that triangle at a
+ * distance that is noise and in front of the triangle's own box. Whether it does depends on what was hit
+ * before, so the walks can differ there (a few in 10,000 of rays made to lie in such planes; none of 80
+ * million others); the two-pass scheme and postponed leaves can also differ by some ulp where several
+ * triangles are hit within rounding of each other.
  *
  * lrt_set_walk: LRT_WALK_AUTO (the default, as above), LRT_WALK_BINARY (in the shape set last), or
  * LRT_WALK_WIDE (the wide form for batches of any size, where the scene has one). The differentiable calls
@@ -317,7 +323,7 @@ lrt_status lrt_set_launch_config(lrt_scene* s, int block, int lds_stack, int xcd
 /* Two-pass scheme of the trace calls: rays still unfinished after `budget` traversal steps
  * (fat-node fetches plus leaf visits) in the one-ray-per-lane pass are finished by a second
  * pass where `tail_waves` persistent waves each walk one ray cooperatively; both passes
- * return the hit of the reference's sequential walk. budget 0 = single pass. Default 64/1024.
+ * return the hit of the reference's sequential walk (with the exception above). budget 0 = single pass. Default 64/1024.
  * No counterpart in the reference (its CPU loop has no wave tail). */
 lrt_status lrt_set_tail_config(lrt_scene* s, uint32_t budget, uint32_t tail_waves);
 
