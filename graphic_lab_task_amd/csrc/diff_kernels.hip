@@ -402,16 +402,30 @@ __global__ __launch_bounds__(BLOCK) void k_sbs_batch(SbsBatchLaunch L) {
   }
 }
 
+// A copy of an item that the same lanes of a wave share, through scalar loads. (Left where it is, its pointers are
+// loaded into vector registers and again after every store.)
+__device__ __forceinline__ SbsBatchItem batch_item(const SbsBatchLaunch& L, uint32_t it) {
+  typedef __attribute__((address_space(4))) const SbsBatchItem constant_item;
+  const SbsBatchItem* from = (const SbsBatchItem*)(constant_item*)(uintptr_t)(L.items + it);
+  SbsBatchItem item;
+  __builtin_memcpy(&item, from, sizeof(item));
+  return item;
+}
+
 // The wide form: one-wave blocks again, every item with a wide tree. A wave's chunks are dealt out for
 // three quarters of the batch, the rest comes from the counter (an atomic on one address takes about 16
-// ns, and with one for each of the 12,288 chunks of 12 x 4 x 128 x 128 rays that was 0.2 ms).
+// ns, and with one for each of the 12,288 chunks of 12 x 4 x 128 x 128 rays that was 0.2 ms). The waves' places
+// move on from round to round, as the views of the items repeat: at the same place a wave got the same part of
+// each image, and the waves of its middle were the last to end. A chunk is groups of neighbours from distant
+// parts of its item, as in the other wide kernels. 48 scenes of 32^3 to 256^3 voxels, 3.1 million rays: 2.95 ms
+// (binary form 4.01); places that stay 4.23, whole chunks of neighbours as well and items read in place 4.86.
 __global__ __launch_bounds__(WIDE_BLOCK, 4) void k_sbs_batch_wide(SbsBatchLaunch L) {
   __shared__ uint32_t lds[2 * WIDE_LDS_STACK * WIDE_BLOCK];
   __shared__ uint32_t result[3 * WIDE_BLOCK];
   const uint32_t lane = threadIdx.x;
   const uint32_t turns = uint32_t(uint64_t(L.total_chunks) * 3u / 4u / gridDim.x);
   for (uint32_t turn = 0;; ++turn) {
-    uint32_t chunk = turn * gridDim.x + blockIdx.x;
+    uint32_t chunk = turn * gridDim.x + (blockIdx.x + turn * 1367u) % gridDim.x;
     if (turn >= turns) {
       uint32_t got = 0;
       if (lane == 0) got = atomicAdd(L.counter, 1u);
@@ -419,11 +433,12 @@ __global__ __launch_bounds__(WIDE_BLOCK, 4) void k_sbs_batch_wide(SbsBatchLaunch
     }
     if (chunk >= L.total_chunks) break;   // the same for the whole wave
     const uint32_t it = __builtin_amdgcn_readfirstlane(find_item(L.chunk_begin, L.n_items, chunk));
-    const SbsBatchItem& item = L.items[it];
-    const uint32_t i = (chunk - L.chunk_begin[it]) * SBS_BATCH_CHUNK + lane;
+    const SbsBatchItem item = batch_item(L, it);
+    const uint32_t first = L.chunk_begin[it], chunks = L.chunk_begin[it + 1] - first;
+    const uint32_t i = (lane / WAVE_GROUP * chunks + chunk - first) * WAVE_GROUP + lane % WAVE_GROUP;
     float loss = diff_wave<3>(item.view, item.args, i < item.args.n, i, (wide_lds*)(lds), (wide_lds*)(result),
                               L.spill + size_t(blockIdx.x * WIDE_BLOCK + lane) * (STACK_SIZE - 8), L.queue,
-                              chunk * SBS_BATCH_CHUNK + lane);
+                              first * SBS_BATCH_CHUNK + i);
     loss = wave_sum(loss);
     if (lane == 0 && item.args.loss) atomicAdd(item.args.loss, loss);
     __syncthreads();

@@ -479,12 +479,20 @@ def test_adjoint_of_another_set(lrt, torch_dev, other):
             assert float((x - y).norm()) <= 1e-5 * float(y.norm()) + 1e-12
 
 
-def test_batch_forms_agree(lrt, torch_dev):
-    """The batched run in the wide form (its default) against the binary one."""
+@pytest.mark.parametrize("sizes", [((3, 1000), (5, 6400), (2, 1), (4, 0), (4, 65)),
+                                   ((2, 300001), (15, 777), (3, 130000), (2, 64))])
+def test_batch_forms_agree(lrt, torch_dev, sizes):
+    """The batched run in the wide form (its default) against the binary one: ragged items, and a batch of several
+    rounds of the waves with a set whose tree is deeper than the LDS stack (depth 15)."""
     torch = torch_dev
     items = []
-    for k, (depth, n) in enumerate([(3, 1000), (5, 6400), (2, 1), (4, 0), (4, 65)]):
-        s = brick_scene(lrt, depth, 8, "indexed", seed=k)()
+    for k, (depth, n) in enumerate(sizes):
+        if depth == 15:
+            s = lrt.SceneRT()
+            s.AddInstance(s.AddGeom_SdfSBS(*cpu.corner_bricks(15, "indexed")))
+            s.CommitScene()
+        else:
+            s = brick_scene(lrt, depth, 8, "indexed", seed=k)()
         pos, dirs = random_rays(torch, max(n, 1), k, extent=2.0)
         pos, dirs = pos[:n].contiguous(), dirs[:n].contiguous()
         dirs[::9, 2] = 0.0
@@ -504,8 +512,8 @@ def test_batch_forms_agree(lrt, torch_dev):
         runs.append([[it[k].clone() for k in ("colour", "grad", "loss")] for it in items])
     for a, b in zip(*runs):
         assert torch.equal(a[0], b[0])
-        for x, y in zip(a[1:], b[1:]):
-            assert float((x - y).norm()) <= 1e-5 * float(y.norm()) + 1e-12
+        for x, y in zip(a[1:], b[1:]):   # fp32 sums in another order; the loss of 300,001 rays: as many steps of 2^-24
+            assert float((x - y).norm()) <= max(1e-5, a[0].shape[0] * 2.0 ** -24) * float(y.norm()) + 1e-12
     batch.set_walk(lrt.WALK_WIDE)
     assert batch.get_walk() == lrt.WALK_BINARY   # the plan of scenes on the binary walk has no other
     for it in items:
