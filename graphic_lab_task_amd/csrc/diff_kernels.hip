@@ -416,9 +416,11 @@ __device__ __forceinline__ SbsBatchItem batch_item(const SbsBatchLaunch& L, uint
 // three quarters of the batch, the rest comes from the counter (an atomic on one address takes about 16
 // ns, and with one for each of the 12,288 chunks of 12 x 4 x 128 x 128 rays that was 0.2 ms). The waves' places
 // move on from round to round, as the views of the items repeat: at the same place a wave got the same part of
-// each image, and the waves of its middle were the last to end. A chunk is groups of neighbours from distant
-// parts of its item, as in the other wide kernels. 48 scenes of 32^3 to 256^3 voxels, 3.1 million rays: 2.95 ms
-// (binary form 4.01); places that stay 4.23, whole chunks of neighbours as well and items read in place 4.86.
+// each image, and the waves of its middle were the last to end. 48 scenes of 32^3 to 256^3 voxels, 3.1 million
+// rays: 3.05 ms (binary form 4.01), with places that stay 4.5 and items read in place as well 4.86; 12 scenes of
+// 32^3 to 128^3, 786 thousand rays: 0.64 against 0.69. Chunks of groups of neighbours from distant parts of the
+// item, as in the other wide kernels, take 2.95 and 0.62, but then nearly every chunk adds to the loss, not only
+// those that see the object, and its rounding error against 64 bits grows by a third (2.4e-7 to 3.1e-7).
 __global__ __launch_bounds__(WIDE_BLOCK, 4) void k_sbs_batch_wide(SbsBatchLaunch L) {
   __shared__ uint32_t lds[2 * WIDE_LDS_STACK * WIDE_BLOCK];
   __shared__ uint32_t result[3 * WIDE_BLOCK];
@@ -434,11 +436,10 @@ __global__ __launch_bounds__(WIDE_BLOCK, 4) void k_sbs_batch_wide(SbsBatchLaunch
     if (chunk >= L.total_chunks) break;   // the same for the whole wave
     const uint32_t it = __builtin_amdgcn_readfirstlane(find_item(L.chunk_begin, L.n_items, chunk));
     const SbsBatchItem item = batch_item(L, it);
-    const uint32_t first = L.chunk_begin[it], chunks = L.chunk_begin[it + 1] - first;
-    const uint32_t i = (lane / WAVE_GROUP * chunks + chunk - first) * WAVE_GROUP + lane % WAVE_GROUP;
+    const uint32_t i = (chunk - L.chunk_begin[it]) * SBS_BATCH_CHUNK + lane;
     float loss = diff_wave<3>(item.view, item.args, i < item.args.n, i, (wide_lds*)(lds), (wide_lds*)(result),
                               L.spill + size_t(blockIdx.x * WIDE_BLOCK + lane) * (STACK_SIZE - 8), L.queue,
-                              first * SBS_BATCH_CHUNK + i);
+                              chunk * SBS_BATCH_CHUNK + lane);
     loss = wave_sum(loss);
     if (lane == 0 && item.args.loss) atomicAdd(item.args.loss, loss);
     __syncthreads();
