@@ -981,7 +981,7 @@ lrt_status lrt_sbs_batch_create(const lrt_sbs_batch_item* items, uint32_t n_item
       return hip_fail(e, "batch table");
     if ((e = b->d_spill.reserve(size_t(max_grid) * lrt::SBS_BATCH_BLOCK * (lrt::STACK_SIZE - 8) * 4)) != hipSuccess)
       return hip_fail(e, "batch spill");
-    if ((e = b->d_counter.reserve(256)) != hipSuccess) return hip_fail(e, "batch counter");
+    if ((e = b->d_counter.reserve(256 + size_t(n_items) * sizeof(double))) != hipSuccess) return hip_fail(e, "batch counter");
     lrt::SbsBatchLaunch& L = b->L;
     L.items = static_cast<const lrt::SbsBatchItem*>(b->d_items.ptr());
     L.n_items = n_items;
@@ -990,6 +990,7 @@ lrt_status lrt_sbs_batch_create(const lrt_sbs_batch_item* items, uint32_t n_item
     L.total_bricks = uint32_t(total_bricks);
     L.total_chunks = chunk_begin.back();
     L.counter = static_cast<uint32_t*>(b->d_counter.ptr());
+    L.loss_sums = reinterpret_cast<double*>(static_cast<char*>(b->d_counter.ptr()) + 256);
     L.spill = static_cast<uint32_t*>(b->d_spill.ptr());
     L.grid = grid;
     L.lds_stack = 16;

@@ -301,6 +301,7 @@ __global__ void k_batch_zero(SbsBatchLaunch L) {
   const SbsBatchItem& item = L.items[blockIdx.y];
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     if (blockIdx.y == 0) *L.counter = 0;
+    L.loss_sums[blockIdx.y] = 0.0;
     if (item.args.loss) *item.args.loss = 0.0f;
   }
   float* g = item.args.grad;
@@ -418,9 +419,9 @@ __device__ __forceinline__ SbsBatchItem batch_item(const SbsBatchLaunch& L, uint
 // move on from round to round, as the views of the items repeat: at the same place a wave got the same part of
 // each image, and the waves of its middle were the last to end. 48 scenes of 32^3 to 256^3 voxels, 3.1 million
 // rays: 3.05 ms (binary form 4.01), with places that stay 4.5 and items read in place as well 4.86; 12 scenes of
-// 32^3 to 128^3, 786 thousand rays: 0.64 against 0.69. Chunks of groups of neighbours from distant parts of the
-// item, as in the other wide kernels, take 2.95 and 0.62, but then nearly every chunk adds to the loss, not only
-// those that see the object, and its rounding error against 64 bits grows by a third (2.4e-7 to 3.1e-7).
+// 32^3 to 128^3, 786 thousand rays: 0.66 against 0.69. The chunks' losses are summed in 64 bits and added to the
+// item's loss by the kernel over the queue: as fp32 sums in the order in which chunks end they were off by 2.4e-7
+// on average and 1.2e-6 at most (2.5e-8 and 5.3e-8 now, in the same time).
 __global__ __launch_bounds__(WIDE_BLOCK, 4) void k_sbs_batch_wide(SbsBatchLaunch L) {
   __shared__ uint32_t lds[2 * WIDE_LDS_STACK * WIDE_BLOCK];
   __shared__ uint32_t result[3 * WIDE_BLOCK];
@@ -441,13 +442,17 @@ __global__ __launch_bounds__(WIDE_BLOCK, 4) void k_sbs_batch_wide(SbsBatchLaunch
                               L.spill + size_t(blockIdx.x * WIDE_BLOCK + lane) * (STACK_SIZE - 8), L.queue,
                               chunk * SBS_BATCH_CHUNK + lane);
     loss = wave_sum(loss);
-    if (lane == 0 && item.args.loss) atomicAdd(item.args.loss, loss);
+    if (lane == 0) unsafeAtomicAdd(L.loss_sums + it, double(loss));
     __syncthreads();
   }
 }
 
 __global__ __launch_bounds__(WIDE_BLOCK) void k_sbs_batch_queued(SbsBatchLaunch L) {
   __shared__ uint32_t lds[16 * WIDE_BLOCK];
+  for (uint32_t k = blockIdx.x * WIDE_BLOCK + threadIdx.x; k < L.n_items; k += gridDim.x * WIDE_BLOCK) {
+    float* loss = L.items[k].args.loss;
+    if (loss) atomicAdd(loss, float(L.loss_sums[k]));   // (queued rays add theirs, items may share it)
+  }
   for_queued(L.queue, [&](bool mine, uint32_t k) {
     if (!mine) return;
     const uint32_t code = L.queue->list[k];   // chunk and ray

@@ -110,6 +110,7 @@ struct SbsBatchLaunch {
   uint32_t zero_blocks, mask_blocks, summary_blocks, brick_blocks;   // x extents of the set-up grids
   uint32_t mask_flag_bytes;      // LDS of the one-wave-per-brick mask build (0: bricks too large)
   uint32_t* counter;             // work counter (reset by the zero kernel)
+  double* loss_sums;             // per item, of the wide form (reset by the zero kernel)
   uint32_t* spill;               // grid * BLOCK * (STACK_SIZE - 8) words
   uint32_t grid;                 // persistent blocks (at most the resident blocks of the variant)
   int lds_stack;                 // stack entries in LDS: 8, 16 or 32

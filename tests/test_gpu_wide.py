@@ -528,6 +528,30 @@ def test_batch_forms_agree(lrt, torch_dev, sizes):
     assert batch.get_walk() == r["walk"]
 
 
+@pytest.mark.parametrize("n", [1, 65, 300001])
+def test_batch_loss(lrt, torch_dev, n):
+    """The batch's losses against float64 sums over the rendered colours. A term rounds by at most 5 steps of 2^-24
+    (difference, square, two sums), a chunk's sum by 6, the result by one; the chunks are summed in 64 bits."""
+    torch = torch_dev
+    items = []
+    for k, m in enumerate((n, 4097)):
+        s = brick_scene(lrt, 3, 8, "indexed", seed=k)()
+        pos, dirs = random_rays(torch, m, k, extent=2.0)
+        params = torch.from_numpy(s.get_array("sbs_data_f")).cuda()
+        items.append({"scene": s, "geom_id": 0, "params": params, "grad": torch.zeros_like(params),
+                      "loss": torch.full((1,), 9.0, device="cuda"), "pos": pos, "dir": dirs,
+                      "target": torch.rand((m, 4), device="cuda", generator=torch.Generator("cuda").manual_seed(k)),
+                      "colour": torch.zeros((m, 4), device="cuda")})
+    batch = lrt.SbsBatch(items)
+    assert batch.get_walk() == lrt.WALK_WIDE
+    for _ in range(3):
+        batch.run()
+        torch.cuda.synchronize()
+        for it in items:
+            want = float(((it["colour"][:, :3].double() - it["target"][:, :3].double()) ** 2).sum())
+            assert abs(float(it["loss"]) - want) <= 12 * 2.0 ** -24 * want
+
+
 @pytest.mark.parametrize("depth,count,lod,n", [(2, 1, 0.0, 1), (3, 2, 0.0, 63), (6, 1, 3.0, 70000), (7, 3, 0.0, 100001),
                                                (8, 1, 0.0, 400000)])
 def test_multi_octrees(lrt, torch_dev, depth, count, lod, n):
